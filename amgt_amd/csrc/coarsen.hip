@@ -28,13 +28,10 @@ namespace amgt {
 namespace {
 
 constexpr int kThreads = 256;
-// levels with few rows (<= kWaveMaxRows) that hold at least kWaveMinRowLen
-// entries per row on average use the wave kernel of extended+i for their F
-// rows (one wave per row holds ~38 KB of LDS: worth it only when the thread
-// kernel would leave the chip idle behind a few long serial rows)
-constexpr int kWaveMinRowLen = 12;
-constexpr int kWaveMaxRows = 1 << 18;       // the kernel of rows up to 256 entries
-constexpr int kWaveMaxRowsSmall = 1 << 21;  // the kernel of rows up to 64 entries
+// extended+i rows of 65 to 512 entries take the wave kernels on levels of at
+// most kWaveMaxRows rows (16 to 70 KB of LDS per wave: worth it only when the
+// thread kernel would leave the chip idle behind a few long serial rows)
+constexpr int kWaveMaxRows = 1 << 18;
 
 inline unsigned grid_of(int64_t n) { return unsigned((n + kThreads - 1) / kThreads); }
 
@@ -296,23 +293,6 @@ __device__ __forceinline__ void h_put(int2 *__restrict__ kv, uint32_t mask, int 
     }
 }
 
-// table size of a row: 0 for C and isolated rows, else the power of two at or
-// above 2 * (upper bound of its entries + its strong dependencies)
-__global__ __launch_bounds__(kThreads) void k_extpi_hsize(int32_t n, const int32_t *__restrict__ SI,
-                                                         const int32_t *__restrict__ cf,
-                                                         const int64_t *__restrict__ ub,
-                                                         int64_t *__restrict__ hs) {
-    const int i = blockIdx.x * kThreads + threadIdx.x;
-    if (i >= n) return;
-    int64_t z = 0;
-    if (cf[i] < 0 && cf[i] != -3) {
-        const int64_t need = 2 * (ub[i] + (SI[i + 1] - SI[i]));
-        z = 1;
-        while (z < need) z <<= 1;
-    }
-    hs[i] = z;
-}
-
 // qsort.c:395-417 (descending |w|) with an explicit stack in place of the
 // recursion.  Each partition step is the host's; the two subranges it leaves
 // are disjoint and sorted independently, so the order in which they are
@@ -371,33 +351,36 @@ __device__ void qsort2_abs(int32_t *v, double *w, int left, int right) {
     }
 }
 
-// One thread per row: the row's columns (fine indices) and weights in the
-// host's discovery order into scratch at off[i]; truncated in place; cnt[i] =
-// the row's final length.
+// Where a row's finished entries go: a fixed slot of `stride` entries per row
+// when rows are truncated to at most that many, else at off[i].
+struct RowSlots {
+    const int64_t *off;
+    int32_t stride;
+    int32_t *sj;
+    double *sw;
+    int32_t *cnt;
+    __device__ __forceinline__ int64_t at(int i) const {
+        return stride > 0 ? int64_t(i) * stride : off[i];
+    }
+};
+
+// One thread per listed row: the row's columns (fine indices) and weights in
+// the host's discovery order into work arrays at woff[t], truncated there, then
+// copied to the row's slot.
 __global__ __launch_bounds__(kThreads) void k_extpi_row(
-    int32_t n, const int32_t *__restrict__ I, const int32_t *__restrict__ J,
-    const double *__restrict__ A, const int32_t *__restrict__ SI, const int32_t *__restrict__ SJ,
-    const int32_t *__restrict__ cf, const int64_t *__restrict__ off, int max_elmts,
-    const int64_t *__restrict__ hoff, int2 *__restrict__ hkv,
-    const int32_t *__restrict__ skip, int32_t *__restrict__ sj, double *__restrict__ sw,
-    int32_t *__restrict__ cnt) {
-    const int i = blockIdx.x * kThreads + threadIdx.x;
-    if (i >= n) return;
-    if (skip && skip[i]) return;  // a row of the wave kernel
-    int32_t *cols = sj + off[i];
-    double *w = sw + off[i];
-    int2 *kv = hkv + hoff[i];
-    const uint32_t mask = uint32_t(hoff[i + 1] - hoff[i]) - 1u;
-    if (cf[i] >= 0) {  // C point: identity (par_lr_interp.c:1488-1495)
-        cols[0] = i;
-        w[0] = 1.0;
-        cnt[i] = 1;
-        return;
-    }
-    if (cf[i] == -3) {
-        cnt[i] = 0;
-        return;
-    }
+    int32_t count, const int32_t *__restrict__ rows, const int32_t *__restrict__ I,
+    const int32_t *__restrict__ J, const double *__restrict__ A, const int32_t *__restrict__ SI,
+    const int32_t *__restrict__ SJ, const int32_t *__restrict__ cf, int max_elmts,
+    const int64_t *__restrict__ woff, int32_t *__restrict__ wcol, double *__restrict__ wval,
+    const int64_t *__restrict__ hoff, int2 *__restrict__ hkv, RowSlots out,
+    int32_t *__restrict__ use) {
+    const int t = blockIdx.x * kThreads + threadIdx.x;
+    if (t >= count) return;
+    const int i = rows[t];
+    int32_t *cols = wcol + woff[t];
+    double *w = wval + woff[t];
+    int2 *kv = hkv + hoff[t];
+    const uint32_t mask = uint32_t(hoff[t + 1] - hoff[t]) - 1u;
     // structure (:1501-1560)
     int c = 0;
     for (int p = SI[i]; p < SI[i + 1]; ++p) {
@@ -505,12 +488,17 @@ __global__ __launch_bounds__(kThreads) void k_extpi_row(
         }
         c = max_elmts;
     }
-    cnt[i] = c;
+    const int64_t o = out.at(i);
+    for (int q = 0; q < c; ++q) {
+        out.sj[o + q] = cols[q];
+        out.sw[o + q] = w[q];
+    }
+    out.cnt[i] = c;
+    use[i] = 0;
 }
 
 // ---- extended+i, one wave per row (long rows of coarse levels) ------------------
-// The same results as k_extpi_row for rows whose columns are ascending (every
-// level exported from an mBSR handle): the host's order of discovery and of
+// The same results as k_extpi_row: the host's order of discovery and of
 // accumulation is kept, the independent parts run across the lanes.
 //  * discovery: the candidate columns in the host's order (lane per strong
 //    dependency, offsets by a scan), first occurrences found with an LDS
@@ -585,14 +573,14 @@ __global__ __launch_bounds__(64) void k_extpi_wave(
     int32_t count, const int32_t *__restrict__ rows, const int32_t *__restrict__ I,
     const int32_t *__restrict__ J, const double *__restrict__ A, const int32_t *__restrict__ SI,
     const int32_t *__restrict__ SJ, const int32_t *__restrict__ cf,
-    const int64_t *__restrict__ off, int max_elmts, int32_t *__restrict__ sj,
-    double *__restrict__ sw, int32_t *__restrict__ cnt, int32_t *__restrict__ use,
-    int overflow_code) {
+    const int8_t *__restrict__ dneg, const int64_t *__restrict__ woff,
+    int32_t *__restrict__ wcol, int max_elmts, RowSlots out, int32_t *__restrict__ use,
+    int overflow_code, int32_t *__restrict__ ovf) {
     __shared__ WaveRow<WA, WT, WH> s;
     if (blockIdx.x >= unsigned(count)) return;
     const int lane = threadIdx.x;
     const int i = rows[blockIdx.x];
-    int32_t *cand = sj + off[i];  // the row's candidates, then (by the fallback) its entries
+    int32_t *cand = wcol + woff[blockIdx.x];  // the row's candidates
     const int a0 = I[i], la = I[i + 1] - a0;
     const int s0 = SI[i], ls = SI[i + 1] - s0;
     for (int t = lane; t < la; t += 64) {
@@ -671,8 +659,11 @@ __global__ __launch_bounds__(64) void k_extpi_wave(
         atomicMin(&s.hval[h], t);
     }
     __syncthreads();
-    if (s.sc[2] > WT) {  // to the next capacity (overflow_code), or the thread kernel (0)
-        if (lane == 0) use[i] = overflow_code;
+    if (s.sc[2] > WT) {  // to the next capacity or the thread kernel
+        if (lane == 0) {
+            use[i] = overflow_code;
+            atomicAdd(ovf, 1);
+        }
         return;
     }
     int c = 0;
@@ -710,8 +701,7 @@ __global__ __launch_bounds__(64) void k_extpi_wave(
                 const int64_t b1 = I[i1], e1 = I[i1 + 1];
                 s.jb1[jj] = int32_t(b1);
                 s.je1[jj] = int32_t(e1);
-                const int64_t d1 = diag_pos(I, J, i1);
-                sgn = (d1 >= 0 && A[d1] < 0) ? -1 : 1;
+                sgn = dneg[i1] ? -1 : 1;
                 // the host's sum in the host's order; the row's entries are
                 // loaded eight at a time so that their loads overlap, and the
                 // entry of column i is noted on the way (the row's columns are
@@ -728,8 +718,8 @@ __global__ __launch_bounds__(64) void k_extpi_wave(
                     }
 #pragma unroll
                     for (int u = 0; u < 8; ++u) {
-                        if (q + u == d1) continue;
                         const int i2 = jq[u];
+                        if (i2 == i1) continue;
                         if (i2 == i) {
                             qi = q + u;
                             aqi = aq[u];
@@ -740,8 +730,8 @@ __global__ __launch_bounds__(64) void k_extpi_wave(
                     }
                 }
                 for (; q < e1; ++q) {
-                    if (q == d1) continue;
                     const int i2 = J[q];
+                    if (i2 == i1) continue;
                     const double aq1 = A[q];
                     if (i2 == i) {
                         qi = q;
@@ -821,88 +811,557 @@ __global__ __launch_bounds__(64) void k_extpi_wave(
             cc = max_elmts;
         }
         s.sc[1] = cc;
-        cnt[i] = cc;
+        out.cnt[i] = cc;
+        use[i] = 0;
     }
     __syncthreads();
     const int cc = s.sc[1];
+    const int64_t o = out.at(i);
     for (int q = lane; q < cc; q += 64) {
-        sj[off[i] + q] = s.pcol[q];
-        sw[off[i] + q] = s.pw[q];
+        out.sj[o + q] = s.pcol[q];
+        out.sw[o + q] = s.pw[q];
+    }
+}
+
+// ---- extended+i, G lanes per row (G = 8, 16, 32: rows of up to G entries in A and S) ----
+// The same results as k_extpi_row.  64 / G rows share a wave, a row's state is
+// 4 G columns and a table of 8 G slots in LDS (0.9 KB for G = 8, 29 KB per
+// workgroup whatever G), a lane holds one entry of A and one of S.  The
+// thread kernel is bound by its per-row tables in global memory (scattered
+// probes, a few lanes of a cache line used); here only the neighbours' rows
+// are read from memory, all of a row's neighbours at once, and every probe
+// and accumulation is in LDS.
+//  * discovery: lane p inserts the columns strong neighbour p contributes with
+//    the key (p, place) of its discovery (atomicMin keeps the first); a column
+//    belongs to the lane that holds its first place, and a prefix count over
+//    the lanes gives its position in the host's order;
+//  * lane jj: kind of entry jj; for a strong F neighbour the sum over its row
+//    in row order, the entries' columns looked up on the way (a row of at most
+//    eight entries stays in registers);
+//  * the weights entry by entry in row order: the columns of one entry are
+//    distinct, so its (at most eight) additions are independent;
+//  * truncation: if the largest weights are distinct in magnitude the sorted
+//    order is the order of their ranks, which the lanes count; otherwise lane 0
+//    of the group runs the host's quicksort.
+// 7-pt 128^3 (1.5 M F rows, variable coefficients): see k_extpi_group's launch.
+template <int G>
+struct GroupRow {
+    double pw[4 * G + 1];  // weights; slot 4 G takes terms that belong to no column
+    int32_t hkey[8 * G];   // column; at the end the kept columns in rank order
+    int32_t hval[8 * G];   // discovery key, then position; at the end the kept weights
+    int32_t pcol[4 * G];
+    int32_t nd;            // distinct columns
+    int32_t pad;
+};
+
+// slot of a key that is in the table
+template <int WH>
+__device__ __forceinline__ uint32_t lds_where(const int32_t *hkey, int k) {
+    uint32_t h = h_slot(k, WH - 1);
+    while (hkey[h] != k) h = (h + 1) & (WH - 1);
+    return h;
+}
+
+// the host's quicksort (qsort2_abs) for at most 128 entries: the pending
+// subranges, at most one per halving, stay in two registers (8 bits per bound)
+__device__ void qsort2_abs_128(int32_t *v, double *w, int right) {
+    uint64_t lo = uint64_t(right), hi = 0;  // (left << 8 | right), newest lowest
+    int top = right > 0 ? 1 : 0;
+    while (top > 0) {
+        const int l = int((lo >> 8) & 0xffu), r = int(lo & 0xffu);
+        lo = (lo >> 16) | (hi << 48);
+        hi >>= 16;
+        --top;
+        const int mid = (l + r) / 2;
+        {
+            const int32_t tv = v[l];
+            v[l] = v[mid];
+            v[mid] = tv;
+            const double tw = w[l];
+            w[l] = w[mid];
+            w[mid] = tw;
+        }
+        const double piv = fabs(w[l]);
+        int last = l;
+        for (int i = l + 1; i <= r; ++i) {
+            if (fabs(w[i]) > piv) {
+                ++last;
+                const int32_t tv = v[last];
+                v[last] = v[i];
+                v[i] = tv;
+                const double tw = w[last];
+                w[last] = w[i];
+                w[i] = tw;
+            }
+        }
+        {
+            const int32_t tv = v[l];
+            v[l] = v[last];
+            v[last] = tv;
+            const double tw = w[l];
+            w[l] = w[last];
+            w[last] = tw;
+        }
+        const bool left_big = last - l > r - last;
+        for (int half = 0; half < 2; ++half) {  // the larger subrange first
+            const bool left = (half == 0) == left_big;
+            const int nl = left ? l : last + 1, nr = left ? last - 1 : r;
+            if (nl >= nr) continue;
+            hi = (hi << 16) | (lo >> 48);
+            lo = (lo << 16) | uint64_t(nl << 8 | nr);
+            ++top;
+        }
+    }
+}
+
+__device__ __forceinline__ void wave_lds_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
+template <int G>
+__global__ __launch_bounds__(kThreads) void k_extpi_group(
+    int32_t n, const int32_t *__restrict__ I, const int32_t *__restrict__ J,
+    const double *__restrict__ A, const int32_t *__restrict__ SI, const int32_t *__restrict__ SJ,
+    const int32_t *__restrict__ cf, const int8_t *__restrict__ dneg, int max_elmts, RowSlots out,
+    int32_t *__restrict__ use, int code, int overflow_code, int32_t *__restrict__ ovf) {
+    constexpr int NG = kThreads / G, WH = 8 * G, WT = 4 * G;
+    __shared__ GroupRow<G> s_row[NG];
+    __shared__ int32_t s_list[kThreads];
+    __shared__ int s_wc[kThreads / 64];
+    const int tid = threadIdx.x, lane = tid & 63;
+    // this kernel's rows among the workgroup's, packed
+    const int row = blockIdx.x * kThreads + tid;
+    const bool mine = row < n && use[row] == code;
+    const uint64_t bal = __ballot(mine);
+    if (lane == 0) s_wc[tid >> 6] = __popcll(bal);
+    __syncthreads();
+    int at = 0, total = 0;
+#pragma unroll
+    for (int q = 0; q < kThreads / 64; ++q) {
+        if (q < (tid >> 6)) at += s_wc[q];
+        total += s_wc[q];
+    }
+    if (mine) s_list[at + __popcll(bal & ((1ull << lane) - 1ull))] = row;
+    __syncthreads();
+    GroupRow<G> &s = s_row[tid / G];
+    double *const tw = reinterpret_cast<double *>(s.hval);  // 4 G weights
+    const int gl = tid % G;
+    const uint64_t gmask = (G == 64 ? ~0ull : ((1ull << G) - 1ull)) << (lane - gl);
+    for (int k0 = 0; k0 < total; k0 += NG) {  // uniform: every lane stays for the wave steps
+        const bool on = k0 + tid / G < total;
+        const int i = on ? s_list[k0 + tid / G] : 0;
+        int a0 = 0, la = 0, s0 = 0, ls = 0;
+        if (on) {
+            a0 = I[i];
+            la = I[i + 1] - a0;
+            s0 = SI[i];
+            ls = SI[i + 1] - s0;
+        }
+        int ac = -1, sc = -1;
+        double av = 0.0;
+        if (gl < la) {
+            ac = J[a0 + gl];
+            av = A[a0 + gl];
+        }
+        if (gl < ls) sc = SJ[s0 + gl];
+        for (int t = gl; t < WH; t += G) {
+            s.hkey[t] = -1;
+            s.hval[t] = INT_MAX;
+        }
+        if (gl == 0) s.nd = 0;
+        const int cfa = ac >= 0 ? cf[ac] : -3;
+        const int cfs = sc >= 0 ? cf[sc] : -3;
+        const bool strongF = cfs < 0 && cfs != -3;
+        int q0 = 0, q1 = 0;
+        if (strongF) {
+            q0 = SI[sc];
+            q1 = SI[sc + 1];
+        }
+        int c8[8], f8[8];  // the first eight strong neighbours of sc and their markers
+#pragma unroll
+        for (int u = 0; u < 8; ++u) c8[u] = q0 + u < q1 ? SJ[q0 + u] : -1;
+#pragma unroll
+        for (int u = 0; u < 8; ++u) f8[u] = c8[u] >= 0 ? cf[c8[u]] : -1;
+        // every column this lane contributes, in the host's order: fn(column, key)
+        const int key0 = (gl + 1) << 24;  // keys exceed every position
+        auto contributed = [&](auto fn) {
+            if (cfs >= 0) fn(sc, key0);
+#pragma unroll
+            for (int u = 0; u < 8; ++u)
+                if (f8[u] >= 0) fn(c8[u], key0 + u);
+            for (int q = q0 + 8; q < q1; ++q) {
+                const int col = SJ[q];
+                if (cf[col] >= 0) fn(col, key0 + (q - q0));
+            }
+        };
+        wave_lds_sync();
+        // at most 4 G columns before the last check of every lane, one more per
+        // lane after it, and a strong F neighbour per lane: 6 G of 8 G slots
+        contributed([&](int col, int key) {
+            if (__atomic_load_n(&s.nd, __ATOMIC_RELAXED) > WT) return;
+            uint32_t h = h_slot(col, WH - 1);
+            for (;; h = (h + 1) & (WH - 1)) {
+                const int32_t prev = atomicCAS(&s.hkey[h], -1, col);
+                if (prev == -1) {
+                    atomicAdd(&s.nd, 1);
+                    break;
+                }
+                if (prev == col) break;
+            }
+            atomicMin(&s.hval[h], key);
+        });
+        wave_lds_sync();
+        const bool wide = q1 - q0 >= (1 << 24);  // places would not fit the key
+        const bool over = s.nd > WT || (__ballot(wide) & gmask) != 0ull;
+        const bool go = on && !over;
+        const int c = go ? s.nd : 0;
+        if (on && over && gl == 0) {
+            use[i] = overflow_code;
+            atomicAdd(ovf, 1);
+        }
+        int nf = 0;
+        if (go)
+            contributed([&](int col, int key) {
+                nf += s.hval[lds_where<WH>(s.hkey, col)] == key ? 1 : 0;
+            });
+        int pos = nf;
+#pragma unroll
+        for (int d = 1; d < G; d <<= 1) {
+            const int t = __shfl_up(pos, d, G);
+            if (gl >= d) pos += t;
+        }
+        pos -= nf;
+        wave_lds_sync();
+        if (go)
+            contributed([&](int col, int key) {
+                const uint32_t h = lds_where<WH>(s.hkey, col);
+                if (s.hval[h] == key) {
+                    s.pcol[pos] = col;
+                    s.hval[h] = pos++;
+                }
+            });
+        wave_lds_sync();
+        if (go && strongF) s.hval[lds_slot<WH>(s.hkey, sc)] = kStrongF;
+        for (int q = gl; q < c; q += G) s.pw[q] = 0.0;
+        wave_lds_sync();
+        // this lane's entry of row i
+        int info = -1, b1 = 0, e1 = 0, neg = 0;
+        bool longrow = false;
+        double dist = 0.0, dterm = 0.0, a8[8];
+        int p8[8];
+        if (go && ac >= 0 && ac != i) {
+            const int v = lds_find<WH>(s.hkey, s.hval, ac);
+            if (v >= 0) {
+                info = v;
+            } else if (v == kStrongF) {
+                b1 = I[ac];
+                e1 = I[ac + 1];
+                neg = dneg[ac];
+                longrow = e1 - b1 > 8;
+                double sum = 0.0, aqi = 0.0;
+                bool back = false;  // row ac holds column i with the right sign
+                for (int q = b1; q < e1; q += 8) {
+                    int j8[8];
+#pragma unroll
+                    for (int u = 0; u < 8; ++u) {
+                        j8[u] = q + u < e1 ? J[q + u] : ac;
+                        a8[u] = q + u < e1 ? A[q + u] : 0.0;
+                    }
+#pragma unroll
+                    for (int u = 0; u < 8; ++u) {
+                        p8[u] = WT;
+                        if (j8[u] == ac || !(neg ? a8[u] > 0.0 : a8[u] < 0.0)) continue;
+                        if (j8[u] == i) {
+                            back = true;
+                            aqi = a8[u];
+                            sum += a8[u];
+                        } else {
+                            const int p = lds_find<WH>(s.hkey, s.hval, j8[u]);
+                            if (p >= 0) {
+                                sum += a8[u];
+                                p8[u] = p;
+                            }
+                        }
+                    }
+                }
+                if (sum != 0) {
+                    info = -2;
+                    dist = av / sum;
+                    if (back) dterm = dist * aqi;
+                } else {
+                    info = -3;
+                    dterm = av;
+                }
+            } else if (cfa != -3) {
+                info = -3;
+                dterm = av;
+            }
+        }
+        const int maxla = __builtin_amdgcn_readlane(wave_incl_max(la), 63);
+        const double aii = (go && ac == i) ? av : 0.0;
+        const uint64_t has_d = __ballot(go && ac == i) & gmask;
+        double diagonal = __shfl(aii, has_d ? __ffsll((unsigned long long)has_d) - 1 : lane);
+        for (int jj = 0; jj < maxla; ++jj) {
+            // 0.0 for the entries that add nothing (adding it changes no sum
+            // that is compared or divided by)
+            diagonal += __shfl(dterm, jj, G);
+            if (gl == jj) {
+                if (info >= 0) {
+                    s.pw[info] += av;
+                } else if (info == -2 && !longrow) {
+                    double t8[8];
+#pragma unroll
+                    for (int u = 0; u < 8; ++u) t8[u] = s.pw[p8[u]];
+#pragma unroll
+                    for (int u = 0; u < 8; ++u) s.pw[p8[u]] = t8[u] + dist * a8[u];
+                }
+            }
+            const int spread = (info == -2 && longrow) ? 1 : 0;
+            if (__ballot(gl == jj && spread)) {
+                // a neighbour's row of more than eight entries: a lane per entry
+                const double dj = __shfl(dist, jj, G);
+                const int ng = __shfl(neg, jj, G), bj = __shfl(b1, jj, G);
+                const int ej = __shfl(spread, jj, G) ? __shfl(e1, jj, G) : bj;
+                for (int q = bj + gl; q < ej; q += G) {
+                    const double aq = A[q];
+                    if (!(ng ? aq > 0.0 : aq < 0.0)) continue;
+                    const int p = lds_find<WH>(s.hkey, s.hval, J[q]);
+                    if (p >= 0) s.pw[p] += dj * aq;
+                }
+            }
+            wave_lds_sync();
+        }
+        if (diagonal != 0)
+            for (int q = gl; q < c; q += G) s.pw[q] /= -diagonal;
+        wave_lds_sync();
+        // truncation (par_csr_matrix.c:3130-3215: tol 0, rescale)
+        const bool trunc = max_elmts > 0 && c > max_elmts;
+        const int cc = trunc ? max_elmts : c;
+        double factor = 1.0;
+        if (__ballot(trunc)) {
+            double row_sum = 0.0;
+            int rk[4];
+            bool tie = false;
+            if (trunc) {
+                for (int q = 0; q < c; ++q) row_sum += s.pw[q];
+#pragma unroll
+                for (int m = 0; m < 4; ++m) {
+                    const int q = gl + m * G;
+                    rk[m] = INT_MAX;
+                    if (q >= c) continue;
+                    const double a = fabs(s.pw[q]);
+                    int above = 0, same = 0;
+                    for (int r = 0; r < c; ++r) {
+                        const double b = fabs(s.pw[r]);
+                        above += b > a ? 1 : 0;
+                        same += b == a ? 1 : 0;
+                    }
+                    rk[m] = above;
+                    // (a weight that is no number equals nothing, not even itself)
+                    if (above < max_elmts && same != 1) tie = true;
+                }
+            }
+            const bool sorted = (__ballot(tie) & gmask) != 0ull;
+            if (trunc && sorted && gl == 0) qsort2_abs_128(s.pcol, s.pw, c - 1);
+            wave_lds_sync();
+            if (trunc) {
+#pragma unroll
+                for (int m = 0; m < 4; ++m) {
+                    const int q = gl + m * G;
+                    const int to = sorted ? q : rk[m];
+                    if (q < c && to < max_elmts) {
+                        s.hkey[to] = s.pcol[q];
+                        tw[to] = s.pw[q];
+                    }
+                }
+            }
+            wave_lds_sync();
+            if (trunc) {
+                double scale = 0.0;
+                for (int q = 0; q < max_elmts; ++q) scale += tw[q];
+                if (scale != 0. && scale != row_sum) factor = row_sum / scale;
+            }
+        }
+        if (go) {
+            const int64_t o = out.at(i);
+            for (int q = gl; q < cc; q += G) {
+                out.sj[o + q] = trunc ? s.hkey[q] : s.pcol[q];
+                out.sw[o + q] = trunc ? tw[q] * factor : s.pw[q];
+            }
+            if (gl == 0) {
+                out.cnt[i] = cc;
+                use[i] = 0;
+            }
+        }
+        wave_lds_sync();  // the next row reuses the state
     }
 }
 #pragma clang fp contract(fast)
 
-// rows the wave kernels cannot search: a row must be ascending, or hold its
-// diagonal first and the rest ascending (HYPRE's layout); diag_pos relies on
-// exactly that
-__global__ __launch_bounds__(kThreads) void k_rows_unsorted(int32_t n, const int32_t *__restrict__ I,
-                                                           const int32_t *__restrict__ J,
-                                                           int32_t *__restrict__ flag) {
-    const int i = blockIdx.x * kThreads + threadIdx.x;
-    if (i >= n) return;
-    int64_t p = I[i];
-    const int64_t e = I[i + 1];
-    if (p < e && J[p] == i) ++p;
-    int prev = -1;
-    for (; p < e; ++p) {
-        const int c = J[p];
-        if (c <= prev) {
-            *flag = 1;
-            return;
-        }
-        prev = c;
-    }
-}
-
-// rows for the wave kernels (0 = the thread kernel): kTier64 = rows of up to 64
-// entries, kTier128 / kTier256 = up to 128 / 256 (when allowed).  Each tier
-// first runs with a small table of P columns; a row with more distinct columns
-// moves on (use[i] = the next code) to the tier's large table, and from there
-// to the thread kernel.
+// Which kernel a row of extended+i takes (0: none, C points, isolated rows and
+// finished ones).  Codes 1..8 are listed rows: the wave kernels by row length
+// (each with a small table of P columns, then, for a row with more distinct
+// columns, the large one), then the thread kernel.  Codes 9..11: the lane-group
+// kernels, which find their rows themselves; their overflow goes to kTier64.
 constexpr int kTier64 = 1, kTier64Big = 2, kTier128 = 3, kTier128Big = 4, kTier256 = 5,
-              kTier256Big = 6, kTier512 = 7;
-__global__ __launch_bounds__(kThreads) void k_wave_rows(int32_t n, const int32_t *__restrict__ I,
-                                                       const int32_t *__restrict__ SI,
-                                                       const int32_t *__restrict__ cf,
-                                                       int allow_big, int32_t *__restrict__ use) {
+              kTier256Big = 6, kTier512 = 7, kThreadRow = 8, kGroup8 = 9, kGroup16 = 10,
+              kGroup32 = 11;
+constexpr int kListed = 8, kCodes = 11;
+
+// per row: C flag, kernel code, sign of the diagonal; C rows (the identity,
+// par_lr_interp.c:1488-1495) and isolated rows are finished here
+__global__ __launch_bounds__(kThreads) void k_extpi_class(
+    int32_t n, const int32_t *__restrict__ I, const int32_t *__restrict__ J,
+    const double *__restrict__ A, const int32_t *__restrict__ SI, const int32_t *__restrict__ cf,
+    int allow_big, int32_t *__restrict__ flag, int32_t *__restrict__ use,
+    int8_t *__restrict__ dneg, RowSlots out) {
     const int i = blockIdx.x * kThreads + threadIdx.x;
     if (i >= n) return;
-    const int la = I[i + 1] - I[i], ls = SI[i + 1] - SI[i];
+    const int f = cf[i];
+    const int len = max(I[i + 1] - I[i], SI[i + 1] - SI[i]);
     int u = 0;
-    if (cf[i] < 0 && cf[i] != -3) {
-        if (la <= 64 && ls <= 64) u = kTier64;
-        else if (allow_big && la <= 128 && ls <= 128) u = kTier128;
-        else if (allow_big && la <= 256 && ls <= 256) u = kTier256;
-        else if (allow_big && la <= 512 && ls <= 512) u = kTier512;
+    if (f >= 0) {
+        const int64_t o = out.at(i);
+        out.sj[o] = i;
+        out.sw[o] = 1.0;
+        out.cnt[i] = 1;
+    } else if (f == -3) {
+        out.cnt[i] = 0;
+    } else {
+        u = len <= 8 ? kGroup8 : (len <= 16 ? kGroup16 : (len <= 32 ? kGroup32 : kThreadRow));
+        if (len > 32 && len <= 64) u = kTier64;
+        if (allow_big && len > 64 && len <= 512)
+            u = len <= 128 ? kTier128 : (len <= 256 ? kTier256 : kTier512);
     }
+    flag[i] = f >= 0 ? 1 : 0;
     use[i] = u;
+    const int64_t d = diag_pos(I, J, i);
+    dneg[i] = (d >= 0 && A[d] < 0) ? 1 : 0;
 }
 
-__global__ __launch_bounds__(kThreads) void k_flag_eq(int32_t n, const int32_t *__restrict__ use,
-                                                     int which, int32_t *__restrict__ flag) {
+// rows per code: one partial per workgroup, one workgroup scans the listed
+// codes' partials into list offsets (the lists follow each other in the order
+// of the codes), then the lists are written, rows ascending
+struct CodeTotals {
+    int32_t c[kCodes];
+};
+// parts[q * ng + workgroup]: rows of code q + 1
+__global__ __launch_bounds__(kThreads) void k_code_part(int32_t n, const int32_t *__restrict__ use,
+                                                       int32_t ng, int32_t *__restrict__ parts) {
+    __shared__ int s_c[kThreads / 64][kCodes];
     const int i = blockIdx.x * kThreads + threadIdx.x;
-    if (i < n) flag[i] = use[i] == which ? 1 : 0;
+    const int u = i < n ? use[i] : 0;
+#pragma unroll
+    for (int q = 0; q < kCodes; ++q) {
+        const uint64_t m = __ballot(u == q + 1);
+        if ((threadIdx.x & 63) == 0) s_c[threadIdx.x >> 6][q] = __popcll(m);
+    }
+    __syncthreads();
+    if (threadIdx.x < kCodes) {
+        int c = 0;
+#pragma unroll
+        for (int w = 0; w < kThreads / 64; ++w) c += s_c[w][threadIdx.x];
+        parts[int64_t(threadIdx.x) * ng + blockIdx.x] = c;
+    }
 }
-
-__global__ __launch_bounds__(kThreads) void k_list_rows(int32_t n, const int32_t *__restrict__ flag,
-                                                       const int32_t *__restrict__ pos,
+// one workgroup, a wave per code; eight loads in flight per lane
+__global__ __launch_bounds__(64 * kCodes) void k_code_finish(int32_t ng,
+                                                            int32_t *__restrict__ parts,
+                                                            CodeTotals *__restrict__ tot) {
+    const int lane = threadIdx.x & 63, q = threadIdx.x >> 6;
+    int32_t *p = parts + int64_t(q) * ng;
+    int run = 0;
+    for (int base = 0; base < ng; base += 512) {
+        int v[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+            const int k = base + 64 * u + lane;
+            v[u] = k < ng ? p[k] : 0;
+        }
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+            const int k = base + 64 * u + lane;
+            const int incl = wave_incl_sum(v[u]);
+            if (k < ng) p[k] = run + incl - v[u];
+            run += __builtin_amdgcn_readlane(incl, 63);
+        }
+    }
+    if (lane == 0) tot->c[q] = run;
+}
+__global__ __launch_bounds__(kThreads) void k_code_list(int32_t n, const int32_t *__restrict__ use,
+                                                       const int32_t *__restrict__ parts,
+                                                       const CodeTotals *__restrict__ tot,
                                                        int32_t *__restrict__ list) {
+    __shared__ int s_c[kThreads / 64][kListed];
     const int i = blockIdx.x * kThreads + threadIdx.x;
-    if (i < n && flag[i]) list[pos[i]] = i;
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int u = i < n ? use[i] : 0;
+    uint64_t m = 0ull;
+#pragma unroll
+    for (int q = 0; q < kListed; ++q) {
+        const uint64_t b = __ballot(u == q + 1);
+        if (u == q + 1) m = b;
+        if (lane == 0) s_c[w][q] = __popcll(b);
+    }
+    __syncthreads();
+    if (u < 1 || u > kListed) return;
+    int pos = parts[int64_t(u - 1) * gridDim.x + blockIdx.x] + __popcll(m & ((1ull << lane) - 1ull));
+    for (int q = 0; q < u - 1; ++q) pos += tot->c[q];
+    for (int q = 0; q < w; ++q) pos += s_c[q][u - 1];
+    list[pos] = i;
+}
+
+// upper bound of each listed row's candidates (k_extpi_ub) and, for the rows
+// of the thread kernel (from t_thread on), its table: the power of two at or
+// above twice its candidates and strong dependencies
+__global__ __launch_bounds__(kThreads) void k_listed_sizes(
+    int32_t count, const int32_t *__restrict__ list, int32_t t_thread,
+    const int32_t *__restrict__ SI, const int32_t *__restrict__ SJ, const int32_t *__restrict__ cf,
+    int64_t *__restrict__ ub, int64_t *__restrict__ hs) {
+    const int t = blockIdx.x * kThreads + threadIdx.x;
+    if (t >= count) return;
+    const int i = list[t];
+    int64_t u = 0;
+    for (int p = SI[i]; p < SI[i + 1]; ++p) {
+        const int i1 = SJ[p];
+        if (cf[i1] >= 0) u += 1;
+        else if (cf[i1] != -3) u += SI[i1 + 1] - SI[i1];
+    }
+    ub[t] = u;
+    int64_t z = 0;
+    if (t >= t_thread) {
+        const int64_t need = 2 * (u + (SI[i + 1] - SI[i]));
+        z = 1;
+        while (z < need) z <<= 1;
+    }
+    hs[t] = z;
 }
 
 __global__ __launch_bounds__(kThreads) void k_extpi_out(
-    int32_t n, const int64_t *__restrict__ off, const int32_t *__restrict__ PI,
-    const int32_t *__restrict__ sj, const double *__restrict__ sw, const int32_t *__restrict__ f2c,
+    int32_t n, const int32_t *__restrict__ PI, RowSlots rows, const int32_t *__restrict__ f2c,
     int32_t *__restrict__ PJ, double *__restrict__ PA) {
     const int i = blockIdx.x * kThreads + threadIdx.x;
     if (i >= n) return;
-    const int64_t s = off[i];
+    const int64_t s = rows.at(i);
     const int len = PI[i + 1] - PI[i];
     for (int q = 0; q < len; ++q) {
-        PJ[PI[i] + q] = f2c[sj[s + q]];
-        PA[PI[i] + q] = sw[s + q];
+        PJ[PI[i] + q] = f2c[rows.sj[s + q]];
+        PA[PI[i] + q] = rows.sw[s + q];
     }
+}
+
+// the same with a thread per slot (a power of two of slots per row)
+__global__ __launch_bounds__(kThreads) void k_extpi_out_slots(
+    int64_t slots, int shift, const int32_t *__restrict__ PI, RowSlots rows,
+    const int32_t *__restrict__ f2c, int32_t *__restrict__ PJ, double *__restrict__ PA) {
+    const int64_t t = int64_t(blockIdx.x) * kThreads + threadIdx.x;
+    if (t >= slots) return;
+    const int i = int(t >> shift), q = int(t) & ((1 << shift) - 1);
+    const int p = PI[i];
+    if (q >= PI[i + 1] - p) return;
+    PJ[p + q] = f2c[rows.sj[t]];
+    PA[p + q] = rows.sw[t];
 }
 
 struct Tmp {
@@ -1052,158 +1511,192 @@ int amgt_amg_extpi_interp(int32_t n, const int32_t *A_i, const int32_t *A_j,
     *P_j = nullptr;
     *P_data = nullptr;
     Tmp tmp(s);
-    int64_t *ub = nullptr, *off = nullptr;
-    int32_t *flag = nullptr, *f2c = nullptr, *cnt = nullptr, *sj = nullptr;
-    double *sw = nullptr;
     const dim3 g(grid_of(n)), b(kThreads);
-    AMGT_TRY(tmp.get(&ub, size_t(n) + 1));
-    AMGT_TRY(tmp.get(&off, size_t(n) + 1));
+    // Rows truncated to a few entries get a fixed slot each (a power of two,
+    // so that the output kernel takes a thread per slot); otherwise the slots
+    // are sized by the rows' upper bounds.
+    constexpr int kMaxSlot = 16;
+    int shift = 0;
+    while ((1 << shift) < max_elmts) ++shift;
+    RowSlots slots{};
+    int32_t *flag = nullptr, *f2c = nullptr, *cnt = nullptr, *use = nullptr, *ovf = nullptr;
+    int8_t *dneg = nullptr;
+    int32_t *parts = nullptr;
+    CodeTotals *tot = nullptr;
     AMGT_TRY(tmp.get(&flag, size_t(n) + 1));
     AMGT_TRY(tmp.get(&f2c, size_t(n) + 1));
     AMGT_TRY(tmp.get(&cnt, size_t(n) + 1));
+    AMGT_TRY(tmp.get(&use, size_t(n) + 1));
+    AMGT_TRY(tmp.get(&dneg, size_t(n) + 1));
+    AMGT_TRY(tmp.get(&ovf, 1));
+    AMGT_TRY(tmp.get(&parts, size_t(g.x) * kCodes + 1));
+    AMGT_TRY(tmp.get(&tot, 1));
+    int64_t total_slots = 0;
+    if (max_elmts > 0 && max_elmts <= kMaxSlot) {
+        slots.stride = 1 << shift;
+        total_slots = int64_t(n) << shift;
+    } else {
+        int64_t *ub = nullptr, *off = nullptr;
+        AMGT_TRY(tmp.get(&ub, size_t(n) + 1));
+        AMGT_TRY(tmp.get(&off, size_t(n) + 1));
+        if (n > 0)
+            hipLaunchKernelGGL(k_extpi_ub, g, b, 0, s, n, S_i, S_j, cf_marker, ub);
+        AMGT_HIP(hipGetLastError());
+        AMGT_TRY(exclusive_scan_i64(ub, off, n, s));
+        const Readback rb[1] = {{&total_slots, off + n, sizeof(int64_t)}};
+        AMGT_TRY(readback(rb, 1, s));
+        slots.off = off;
+    }
+    AMGT_TRY(tmp.get(&slots.sj, size_t(total_slots)));
+    AMGT_TRY(tmp.get(&slots.sw, size_t(total_slots)));
+    slots.cnt = cnt;
+
+    // rows per kernel
+    CodeTotals h{};
+    int32_t nc = 0, nnz = 0, h_ovf = 0;
+    auto count_codes = [&]() -> int {
+        hipLaunchKernelGGL(k_code_part, g, b, 0, s, n, use, int32_t(g.x), parts);
+        hipLaunchKernelGGL(k_code_finish, dim3(1), dim3(64 * kCodes), 0, s, int32_t(g.x), parts,
+                           tot);
+        AMGT_HIP(hipGetLastError());
+        return AMGT_OK;
+    };
+    if (n > 0) {
+        hipLaunchKernelGGL(k_extpi_class, g, b, 0, s, n, A_i, A_j, A_data, S_i, cf_marker,
+                           n <= kWaveMaxRows ? 1 : 0, flag, use, dneg, slots);
+        AMGT_TRY(count_codes());
+    }
+    AMGT_TRY(exclusive_scan_i32(flag, f2c, n, s));
+    if (n > 0) {
+        const Readback rb[2] = {{&nc, f2c + n, sizeof(int32_t)}, {&h, tot, sizeof(CodeTotals)}};
+        AMGT_TRY(readback(rb, 2, s));
+    }
+    AMGT_HIP(hipMemsetAsync(ovf, 0, sizeof(int32_t), s));
     int32_t *pi = static_cast<int32_t *>(dev_alloc(sizeof(int32_t) * (size_t(n) + 1), s));
     if (!pi) {
         set_error("allocation of P row pointer failed");
         return AMGT_ERR_ALLOC;
     }
-    int st = AMGT_OK;
-    int64_t total_ub = 0;
-    int32_t nc = 0, nnz = 0;
-    if (n > 0) {
-        hipLaunchKernelGGL(k_is_coarse, g, b, 0, s, n, cf_marker, flag);
-        hipLaunchKernelGGL(k_extpi_ub, g, b, 0, s, n, S_i, S_j, cf_marker, ub);
-        if (hipGetLastError() != hipSuccess) st = AMGT_ERR_HIP;
-    }
-    if (st == AMGT_OK) st = exclusive_scan_i32(flag, f2c, n, s);
-    if (st == AMGT_OK) st = exclusive_scan_i64(ub, off, n, s);
-    if (st == AMGT_OK) {
-        const Readback rb[2] = {{&total_ub, off + n, sizeof(int64_t)},
-                                {&nc, f2c + n, sizeof(int32_t)}};
-        st = readback(rb, 2, s);
-    }
-    if (st == AMGT_OK) st = tmp.get(&sj, size_t(total_ub));
-    if (st == AMGT_OK) st = tmp.get(&sw, size_t(total_ub));
-    // per-row tables
-    int64_t *hs = nullptr, *hoff = nullptr;
-    int2 *hkv = nullptr;
-    int64_t total_h = 0;
-    if (st == AMGT_OK) st = tmp.get(&hs, size_t(n) + 1);
-    if (st == AMGT_OK) st = tmp.get(&hoff, size_t(n) + 1);
-    if (st == AMGT_OK && n > 0) {
-        hipLaunchKernelGGL(k_extpi_hsize, g, b, 0, s, n, S_i, cf_marker, ub, hs);
-        if (hipGetLastError() != hipSuccess) st = AMGT_ERR_HIP;
-    }
-    if (st == AMGT_OK) st = exclusive_scan_i64(hs, hoff, n, s);
-    if (st == AMGT_OK) {
-        const Readback rb[1] = {{&total_h, hoff + n, sizeof(int64_t)}};
-        st = readback(rb, 1, s);
-    }
-    if (st == AMGT_OK) st = tmp.get(&hkv, size_t(total_h));
-    if (st == AMGT_OK && total_h > 0 &&
-        hipMemsetAsync(hkv, 0xff, sizeof(int2) * size_t(total_h), s) != hipSuccess)
-        st = AMGT_ERR_HIP;
-    // long rows with ascending columns (coarse levels): a wave per row
-    int32_t *use = nullptr, *upos = nullptr;
-    int32_t nwave = 0;
-    if (st == AMGT_OK && n > 0) {
-        int64_t nnzA = 0;
-        int32_t h_unsorted = 0;
-        int32_t *unsorted = nullptr;
-        int32_t lastI = 0;
-        {
-            const Readback rb[1] = {{&lastI, A_i + n, sizeof(int32_t)}};
+    auto fail = [&](int st) {
+        dev_free(pi, s);
+        return st;
+    };
+    // the listed rows, then those that overflowed a table (at most kTier64,
+    // its large table, the thread kernel: each round moves a row on)
+    auto listed_rows = [&]() -> int {
+        int32_t np = 0;
+        for (int q = 0; q < kListed; ++q) np += h.c[q];
+        if (np == 0) return AMGT_OK;
+        int32_t *list = nullptr, *wcol = nullptr;
+        int64_t *ub = nullptr, *woff = nullptr, *hs = nullptr, *hoff = nullptr;
+        double *wval = nullptr;
+        int2 *hkv = nullptr;
+        const int32_t nthread = h.c[kThreadRow - 1];
+        AMGT_TRY(tmp.get(&list, size_t(np)));
+        AMGT_TRY(tmp.get(&ub, size_t(np) + 1));
+        AMGT_TRY(tmp.get(&woff, size_t(np) + 1));
+        AMGT_TRY(tmp.get(&hs, size_t(np) + 1));
+        hipLaunchKernelGGL(k_code_list, g, b, 0, s, n, use, parts, tot, list);
+        hipLaunchKernelGGL(k_listed_sizes, dim3(grid_of(np)), b, 0, s, np, list, np - nthread, S_i,
+                           S_j, cf_marker, ub, hs);
+        AMGT_HIP(hipGetLastError());
+        AMGT_TRY(exclusive_scan_i64(ub, woff, np, s));
+        int64_t total_w = 0, total_h = 0;
+        if (nthread > 0) {
+            AMGT_TRY(tmp.get(&hoff, size_t(np) + 1));
+            AMGT_TRY(exclusive_scan_i64(hs, hoff, np, s));
+            const Readback rb[2] = {{&total_w, woff + np, sizeof(int64_t)},
+                                    {&total_h, hoff + np, sizeof(int64_t)}};
+            AMGT_TRY(readback(rb, 2, s));
+            AMGT_TRY(tmp.get(&wval, size_t(total_w)));
+            AMGT_TRY(tmp.get(&hkv, size_t(total_h)));
+            AMGT_HIP(hipMemsetAsync(hkv, 0xff, sizeof(int2) * size_t(total_h), s));
+        } else {
+            const Readback rb[1] = {{&total_w, woff + np, sizeof(int64_t)}};
+            AMGT_TRY(readback(rb, 1, s));
+        }
+        AMGT_TRY(tmp.get(&wcol, size_t(total_w)));
+        int32_t t0 = 0;
+        for (int code = 1; code <= kListed; ++code) {
+            const int32_t cw = h.c[code - 1];
+            if (cw == 0) continue;
+            const int32_t *rows = list + t0;
+            const int64_t *wo = woff + t0;
+#define AMGT_EXTPI_WAVE(WA_, WT_, WH_, NEXT_)                                                  \
+    hipLaunchKernelGGL((k_extpi_wave<WA_, WT_, WH_>), dim3(unsigned(cw)), dim3(64), 0, s, cw,  \
+                       rows, A_i, A_j, A_data, S_i, S_j, cf_marker, dneg, wo, wcol, max_elmts, \
+                       slots, use, NEXT_, ovf)
+            switch (code) {
+                case kTier64: AMGT_EXTPI_WAVE(64, 128, 512, kTier64Big); break;      // ~8.4 KB
+                case kTier64Big: AMGT_EXTPI_WAVE(64, 384, 1024, kThreadRow); break;  // ~15.6 KB
+                case kTier128: AMGT_EXTPI_WAVE(128, 256, 1024, kTier128Big); break;  // ~16 KB
+                case kTier256: AMGT_EXTPI_WAVE(256, 768, 2048, kTier256Big); break;  // ~35 KB
+                case kTier128Big: AMGT_EXTPI_WAVE(256, 768, 2048, kThreadRow); break;
+                case kTier256Big: AMGT_EXTPI_WAVE(256, 1536, 4096, kThreadRow); break;  // ~60 KB
+                case kTier512: AMGT_EXTPI_WAVE(512, 1536, 4096, kThreadRow); break;  // ~70 KB
+                default:
+                    hipLaunchKernelGGL(k_extpi_row, dim3(grid_of(cw)), b, 0, s, cw, rows, A_i, A_j,
+                                       A_data, S_i, S_j, cf_marker, max_elmts, wo, wcol, wval,
+                                       hoff + t0, hkv, slots, use);
+            }
+#undef AMGT_EXTPI_WAVE
+            t0 += cw;
+        }
+        AMGT_HIP(hipGetLastError());
+        return AMGT_OK;
+    };
+    // (after the lists of round 0 are written: an overflow changes the row's code)
+    auto group_rows = [&]() -> int {
+#define AMGT_EXTPI_GROUP(G_, CODE_)                                                            \
+    if (h.c[CODE_ - 1] > 0)                                                                    \
+    hipLaunchKernelGGL((k_extpi_group<G_>), g, b, 0, s, n, A_i, A_j, A_data, S_i, S_j,         \
+                       cf_marker, dneg, max_elmts, slots, use, CODE_, kTier64, ovf)
+        AMGT_EXTPI_GROUP(8, kGroup8);
+        AMGT_EXTPI_GROUP(16, kGroup16);
+        AMGT_EXTPI_GROUP(32, kGroup32);
+#undef AMGT_EXTPI_GROUP
+        AMGT_HIP(hipGetLastError());
+        return AMGT_OK;
+    };
+    for (int round = 0; n > 0 && round < 4; ++round) {
+        int st = listed_rows();
+        if (st == AMGT_OK && round == 0) st = group_rows();
+        if (st == AMGT_OK) st = exclusive_scan_i32(cnt, pi, n, s);
+        if (st == AMGT_OK) {
+            const Readback rb[2] = {{&nnz, pi + n, sizeof(int32_t)}, {&h_ovf, ovf, sizeof(int32_t)}};
+            st = readback(rb, 2, s);
+        }
+        if (st == AMGT_OK && h_ovf == 0) break;
+        if (st == AMGT_OK) st = count_codes();
+        if (st == AMGT_OK) {
+            const Readback rb[1] = {{&h, tot, sizeof(CodeTotals)}};
             st = readback(rb, 1, s);
         }
-        nnzA = lastI;
-        if (st == AMGT_OK && n <= kWaveMaxRowsSmall && nnzA >= int64_t(kWaveMinRowLen) * n) {
-            st = tmp.get(&unsorted, 1);
-            if (st == AMGT_OK &&
-                (hipMemsetAsync(unsorted, 0, sizeof(int32_t), s) != hipSuccess))
-                st = AMGT_ERR_HIP;
-            if (st == AMGT_OK) {
-                hipLaunchKernelGGL(k_rows_unsorted, g, b, 0, s, n, A_i, A_j, unsorted);
-                const Readback rb[1] = {{&h_unsorted, unsorted, sizeof(int32_t)}};
-                st = hipGetLastError() != hipSuccess ? AMGT_ERR_HIP : readback(rb, 1, s);
-            }
-            if (st == AMGT_OK && !h_unsorted) {
-                int32_t *flag2 = nullptr;
-                st = tmp.get(&use, size_t(n) + 1);
-                if (st == AMGT_OK) st = tmp.get(&upos, size_t(n) + 1);
-                if (st == AMGT_OK) st = tmp.get(&flag2, size_t(n) + 1);
-                if (st == AMGT_OK) {
-                    hipLaunchKernelGGL(k_wave_rows, g, b, 0, s, n, A_i, S_i, cf_marker,
-                                       n <= kWaveMaxRows ? 1 : 0, use);
-                    if (hipGetLastError() != hipSuccess) st = AMGT_ERR_HIP;
-                }
-                // (rows with this code, kernel, code for the rows that overflow it)
-                const int stages[7][2] = {{kTier64, kTier64Big}, {kTier64Big, 0},
-                                          {kTier128, kTier128Big}, {kTier128Big, 0},
-                                          {kTier256, kTier256Big}, {kTier256Big, 0},
-                                          {kTier512, 0}};
-                for (int sg = 0; sg < 7 && st == AMGT_OK; ++sg) {
-                    const int which = stages[sg][0], next = stages[sg][1];
-                    int32_t cntw = 0;
-                    hipLaunchKernelGGL(k_flag_eq, g, b, 0, s, n, use, which, flag2);
-                    if (hipGetLastError() != hipSuccess) st = AMGT_ERR_HIP;
-                    if (st == AMGT_OK) st = exclusive_scan_i32(flag2, upos, n, s);
-                    if (st == AMGT_OK) {
-                        const Readback rb[1] = {{&cntw, upos + n, sizeof(int32_t)}};
-                        st = readback(rb, 1, s);
-                    }
-                    if (st != AMGT_OK || cntw == 0) continue;
-                    int32_t *wl = nullptr;
-                    st = tmp.get(&wl, size_t(cntw));
-                    if (st != AMGT_OK) break;
-                    hipLaunchKernelGGL(k_list_rows, g, b, 0, s, n, flag2, upos, wl);
-#define AMGT_EXTPI_WAVE(WA_, WT_, WH_)                                                     \
-    hipLaunchKernelGGL((k_extpi_wave<WA_, WT_, WH_>), dim3(unsigned(cntw)), dim3(64), 0, s, cntw, \
-                       wl, A_i, A_j, A_data, S_i, S_j, cf_marker, off, max_elmts, sj, sw, cnt, \
-                       use, next)
-                    switch (which) {
-                        case kTier64: AMGT_EXTPI_WAVE(64, 128, 512); break;      // ~8.4 KB
-                        case kTier64Big: AMGT_EXTPI_WAVE(64, 384, 1024); break;  // ~15.6 KB
-                        case kTier128: AMGT_EXTPI_WAVE(128, 256, 1024); break;   // ~16 KB
-                        case kTier256Big: AMGT_EXTPI_WAVE(256, 1536, 4096); break;  // ~60 KB
-                        case kTier512: AMGT_EXTPI_WAVE(512, 1536, 4096); break;   // ~70 KB
-                        default: AMGT_EXTPI_WAVE(256, 768, 2048); break;         // ~35 KB
-                    }
-#undef AMGT_EXTPI_WAVE
-                    if (hipGetLastError() != hipSuccess) st = AMGT_ERR_HIP;
-                    nwave += cntw;
-                }
-            }
-        }
+        if (st == AMGT_OK && hipMemsetAsync(ovf, 0, sizeof(int32_t), s) != hipSuccess)
+            st = AMGT_ERR_HIP;
+        if (st != AMGT_OK) return fail(st);
     }
-    if (st == AMGT_OK && n > 0) {
-        hipLaunchKernelGGL(k_extpi_row, g, b, 0, s, n, A_i, A_j, A_data, S_i, S_j, cf_marker, off,
-                           max_elmts, hoff, hkv, nwave > 0 ? use : nullptr, sj, sw, cnt);
-        if (hipGetLastError() != hipSuccess) st = AMGT_ERR_HIP;
-    }
-    if (st == AMGT_OK) st = exclusive_scan_i32(cnt, pi, n, s);
-    if (st == AMGT_OK) {
-        const Readback rb[1] = {{&nnz, pi + n, sizeof(int32_t)}};
-        st = readback(rb, 1, s);
-    }
-    int32_t *pj = nullptr;
-    double *pa = nullptr;
-    if (st == AMGT_OK) {
-        pj = static_cast<int32_t *>(dev_alloc(sizeof(int32_t) * (size_t(nnz) + 1), s));
-        pa = static_cast<double *>(dev_alloc(sizeof(double) * (size_t(nnz) + 1), s));
-        if (!pj || !pa) {
-            set_error("allocation of P failed");
-            st = AMGT_ERR_ALLOC;
-        }
-    }
-    if (st == AMGT_OK && n > 0) {
-        hipLaunchKernelGGL(k_extpi_out, g, b, 0, s, n, off, pi, sj, sw, f2c, pj, pa);
-        if (hipGetLastError() != hipSuccess) st = AMGT_ERR_HIP;
-    }
-    if (st != AMGT_OK) {
-        if (st == AMGT_ERR_HIP) set_error("extended+i interpolation: kernel launch or copy failed");
-        dev_free(pi, s);
+    if (n == 0) AMGT_TRY(exclusive_scan_i32(cnt, pi, 0, s));
+    int32_t *pj = static_cast<int32_t *>(dev_alloc(sizeof(int32_t) * (size_t(nnz) + 1), s));
+    double *pa = static_cast<double *>(dev_alloc(sizeof(double) * (size_t(nnz) + 1), s));
+    if (!pj || !pa) {
+        set_error("allocation of P failed");
         if (pj) dev_free(pj, s);
         if (pa) dev_free(pa, s);
-        return st;
+        return fail(AMGT_ERR_ALLOC);
+    }
+    if (n > 0) {
+        if (slots.stride > 0)
+            hipLaunchKernelGGL(k_extpi_out_slots, dim3(grid_of(total_slots)), b, 0, s, total_slots,
+                               shift, pi, slots, f2c, pj, pa);
+        else
+            hipLaunchKernelGGL(k_extpi_out, g, b, 0, s, n, pi, slots, f2c, pj, pa);
+        if (hipGetLastError() != hipSuccess) {
+            set_error("extended+i interpolation: kernel launch failed");
+            dev_free(pj, s);
+            dev_free(pa, s);
+            return fail(AMGT_ERR_HIP);
+        }
     }
     *n_coarse = nc;
     *nnzP = nnz;
