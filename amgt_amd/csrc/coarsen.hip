@@ -831,35 +831,38 @@ __global__ __launch_bounds__(64) void k_extpi_wave(
 // probes, a few lanes of a cache line used); here only the neighbours' rows
 // are read from memory, all of a row's neighbours at once, and every probe
 // and accumulation is in LDS.
-//  * discovery: lane p inserts the columns strong neighbour p contributes with
-//    the key (p, place) of its discovery (atomicMin keeps the first); a column
-//    belongs to the lane that holds its first place, and a prefix count over
-//    the lanes gives its position in the host's order;
+//  * discovery: each lane counts the columns its strong neighbour contributes,
+//    a prefix over the lanes places them in one list in the host's order, the
+//    lanes insert the list's columns into the table with their place
+//    (atomicMin keeps the first) and a ballot counts the firsts before each;
 //  * lane jj: kind of entry jj; for a strong F neighbour the sum over its row
-//    in row order, the entries' columns looked up on the way (a row of at most
-//    eight entries stays in registers);
-//  * the weights entry by entry in row order: the columns of one entry are
-//    distinct, so its (at most eight) additions are independent;
+//    in row order, the entries' columns looked up on the way and the terms of
+//    P columns (few of a row's entries) kept in LDS;
+//  * the weights entry by entry in row order, a lane per term (the columns of
+//    one entry are distinct);
 //  * truncation: if the largest weights are distinct in magnitude the sorted
 //    order is the order of their ranks, which the lanes count; otherwise lane 0
 //    of the group runs the host's quicksort.
-// 7-pt 128^3 (1.5 M F rows, variable coefficients): see k_extpi_group's launch.
+// Issue-bound by the probe loops, which diverge: the first form, which walked
+// each lane's own columns three times (37 loops), took 1140 us on 7-pt 128^3
+// (1.5 M F rows), the thread kernel 4845 us.
+constexpr int kTerms = 4;  // terms of one neighbour kept in LDS
 template <int G>
 struct GroupRow {
-    double pw[4 * G + 1];  // weights; slot 4 G takes terms that belong to no column
-    int32_t hkey[8 * G];   // column; at the end the kept columns in rank order
-    int32_t hval[8 * G];   // discovery key, then position; at the end the kept weights
+    double pw[4 * G];          // first the list of candidate columns (8 G), then weights
+    double ta[kTerms * G];     // terms of entry jj at kTerms * jj; kept columns at the end
+    int2 kv[8 * G];            // (column, place then position); kept weights at the end
+    uint64_t tp[G];            // positions of the terms, 16 bits each (0xffff: none)
     int32_t pcol[4 * G];
-    int32_t nd;            // distinct columns
-    int32_t pad;
 };
 
-// slot of a key that is in the table
 template <int WH>
-__device__ __forceinline__ uint32_t lds_where(const int32_t *hkey, int k) {
-    uint32_t h = h_slot(k, WH - 1);
-    while (hkey[h] != k) h = (h + 1) & (WH - 1);
-    return h;
+__device__ __forceinline__ int kv_find(const int2 *kv, int k) {
+    for (uint32_t h = h_slot(k, WH - 1);; h = (h + 1) & (WH - 1)) {
+        const int2 e = kv[h];
+        if (e.x == k) return e.y;
+        if (e.x == -1) return -1;
+    }
 }
 
 // the host's quicksort (qsort2_abs) for at most 128 entries: the pending
@@ -945,9 +948,13 @@ __global__ __launch_bounds__(kThreads) void k_extpi_group(
     if (mine) s_list[at + __popcll(bal & ((1ull << lane) - 1ull))] = row;
     __syncthreads();
     GroupRow<G> &s = s_row[tid / G];
-    double *const tw = reinterpret_cast<double *>(s.hval);  // 4 G weights
+    int32_t *const cand = reinterpret_cast<int32_t *>(s.pw);  // 8 G candidates
+    double *const tw = reinterpret_cast<double *>(s.kv);      // 4 G kept weights
+    int32_t *const keep = reinterpret_cast<int32_t *>(s.ta);  // and their columns
     const int gl = tid % G;
-    const uint64_t gmask = (G == 64 ? ~0ull : ((1ull << G) - 1ull)) << (lane - gl);
+    const int sh = lane - gl;  // first lane of the group
+    const uint64_t gones = (1ull << G) - 1ull, gmask = gones << sh;
+    constexpr int TL = 6 * G;  // candidates: with G strong F neighbours 7 G of 8 G slots
     for (int k0 = 0; k0 < total; k0 += NG) {  // uniform: every lane stays for the wave steps
         const bool on = k0 + tid / G < total;
         const int i = on ? s_list[k0 + tid / G] : 0;
@@ -965,11 +972,7 @@ __global__ __launch_bounds__(kThreads) void k_extpi_group(
             av = A[a0 + gl];
         }
         if (gl < ls) sc = SJ[s0 + gl];
-        for (int t = gl; t < WH; t += G) {
-            s.hkey[t] = -1;
-            s.hval[t] = INT_MAX;
-        }
-        if (gl == 0) s.nd = 0;
+        for (int t = gl; t < WH; t += G) s.kv[t] = make_int2(-1, INT_MAX);
         const int cfa = ac >= 0 ? cf[ac] : -3;
         const int cfs = sc >= 0 ? cf[sc] : -3;
         const bool strongF = cfs < 0 && cfs != -3;
@@ -983,86 +986,105 @@ __global__ __launch_bounds__(kThreads) void k_extpi_group(
         for (int u = 0; u < 8; ++u) c8[u] = q0 + u < q1 ? SJ[q0 + u] : -1;
 #pragma unroll
         for (int u = 0; u < 8; ++u) f8[u] = c8[u] >= 0 ? cf[c8[u]] : -1;
-        // every column this lane contributes, in the host's order: fn(column, key)
-        const int key0 = (gl + 1) << 24;  // keys exceed every position
-        auto contributed = [&](auto fn) {
-            if (cfs >= 0) fn(sc, key0);
+        int nk = cfs >= 0 ? 1 : 0;
+#pragma unroll
+        for (int u = 0; u < 8; ++u) nk += f8[u] >= 0 ? 1 : 0;
+        for (int q = q0 + 8; q < q1; ++q) nk += cf[SJ[q]] >= 0 ? 1 : 0;
+        int o = nk;
+#pragma unroll
+        for (int d = 1; d < G; d <<= 1) {
+            const int t = __shfl_up(o, d, G);
+            if (gl >= d) o += t;
+        }
+        const int T = __shfl(o, G - 1, G);
+        o -= nk;
+        const bool fits = T <= TL;
+        if (fits && nk > 0) {
+            if (cfs >= 0) cand[o++] = sc;
 #pragma unroll
             for (int u = 0; u < 8; ++u)
-                if (f8[u] >= 0) fn(c8[u], key0 + u);
+                if (f8[u] >= 0) cand[o++] = c8[u];
             for (int q = q0 + 8; q < q1; ++q) {
                 const int col = SJ[q];
-                if (cf[col] >= 0) fn(col, key0 + (q - q0));
+                if (cf[col] >= 0) cand[o++] = col;
             }
-        };
+        }
         wave_lds_sync();
-        // at most 4 G columns before the last check of every lane, one more per
-        // lane after it, and a strong F neighbour per lane: 6 G of 8 G slots
-        contributed([&](int col, int key) {
-            if (__atomic_load_n(&s.nd, __ATOMIC_RELAXED) > WT) return;
-            uint32_t h = h_slot(col, WH - 1);
-            for (;; h = (h + 1) & (WH - 1)) {
-                const int32_t prev = atomicCAS(&s.hkey[h], -1, col);
-                if (prev == -1) {
-                    atomicAdd(&s.nd, 1);
-                    break;
+        // candidate t: its slot; the smallest place of a column stays with it
+        int ct[6], slot[6];
+#pragma unroll
+        for (int m = 0; m < 6; ++m) {
+            const int t = gl + m * G;
+            const bool in = fits && t < T;
+            ct[m] = 0;
+            slot[m] = 0;
+            if (!__ballot(in)) continue;
+            if (in) {
+                ct[m] = cand[t];
+                uint32_t h = h_slot(ct[m], WH - 1);
+                for (;; h = (h + 1) & (WH - 1)) {
+                    const int32_t prev = atomicCAS(&s.kv[h].x, -1, ct[m]);
+                    if (prev == -1 || prev == ct[m]) break;
                 }
-                if (prev == col) break;
+                atomicMin(&s.kv[h].y, t);
+                slot[m] = int(h);
             }
-            atomicMin(&s.hval[h], key);
-        });
+        }
         wave_lds_sync();
-        const bool wide = q1 - q0 >= (1 << 24);  // places would not fit the key
-        const bool over = s.nd > WT || (__ballot(wide) & gmask) != 0ull;
+        int c = 0;
+#pragma unroll
+        for (int m = 0; m < 6; ++m) {
+            const int t = gl + m * G;
+            const bool in = fits && t < T;
+            if (!__ballot(in)) continue;
+            const bool first = in && s.kv[slot[m]].y == t;
+            const uint64_t f = (__ballot(first) >> sh) & gones;
+            const int pos = c + __popcll(f & ((1ull << gl) - 1ull));
+            if (first && pos < WT) {
+                s.pcol[pos] = ct[m];
+                s.kv[slot[m]].y = pos;  // at most the column's place: equals no later one
+            }
+            c += __popcll(f);
+        }
+        const bool over = !fits || c > WT;
         const bool go = on && !over;
-        const int c = go ? s.nd : 0;
+        if (!go) c = 0;
         if (on && over && gl == 0) {
             use[i] = overflow_code;
             atomicAdd(ovf, 1);
         }
-        int nf = 0;
-        if (go)
-            contributed([&](int col, int key) {
-                nf += s.hval[lds_where<WH>(s.hkey, col)] == key ? 1 : 0;
-            });
-        int pos = nf;
-#pragma unroll
-        for (int d = 1; d < G; d <<= 1) {
-            const int t = __shfl_up(pos, d, G);
-            if (gl >= d) pos += t;
+        if (go && strongF) {
+            uint32_t h = h_slot(sc, WH - 1);
+            for (;; h = (h + 1) & (WH - 1)) {
+                const int32_t prev = atomicCAS(&s.kv[h].x, -1, sc);
+                if (prev == -1 || prev == sc) break;
+            }
+            s.kv[h].y = kStrongF;
         }
-        pos -= nf;
         wave_lds_sync();
-        if (go)
-            contributed([&](int col, int key) {
-                const uint32_t h = lds_where<WH>(s.hkey, col);
-                if (s.hval[h] == key) {
-                    s.pcol[pos] = col;
-                    s.hval[h] = pos++;
-                }
-            });
-        wave_lds_sync();
-        if (go && strongF) s.hval[lds_slot<WH>(s.hkey, sc)] = kStrongF;
-        for (int q = gl; q < c; q += G) s.pw[q] = 0.0;
-        wave_lds_sync();
+        for (int q = gl; q < c; q += G) s.pw[q] = 0.0;  // (the candidates are done)
         // this lane's entry of row i
-        int info = -1, b1 = 0, e1 = 0, neg = 0;
-        bool longrow = false;
-        double dist = 0.0, dterm = 0.0, a8[8];
-        int p8[8];
+        int b1 = 0, e1 = 0, neg = 0, nt = 0;
+        bool spread = false;
+        uint64_t tp = ~0ull;
+        double dist = 0.0, dterm = 0.0;
+        double *const ta = s.ta + kTerms * gl;
         if (go && ac >= 0 && ac != i) {
-            const int v = lds_find<WH>(s.hkey, s.hval, ac);
+            const int v = kv_find<WH>(s.kv, ac);
             if (v >= 0) {
-                info = v;
+                ta[0] = av;
+                tp = ~0xffffull | uint64_t(v);
             } else if (v == kStrongF) {
                 b1 = I[ac];
                 e1 = I[ac + 1];
                 neg = dneg[ac];
-                longrow = e1 - b1 > 8;
                 double sum = 0.0, aqi = 0.0;
                 bool back = false;  // row ac holds column i with the right sign
                 for (int q = b1; q < e1; q += 8) {
                     int j8[8];
+                    double a8[8];
+                    int2 e8[8];
+                    uint32_t h8[8];
 #pragma unroll
                     for (int u = 0; u < 8; ++u) {
                         j8[u] = q + u < e1 ? J[q + u] : ac;
@@ -1070,34 +1092,48 @@ __global__ __launch_bounds__(kThreads) void k_extpi_group(
                     }
 #pragma unroll
                     for (int u = 0; u < 8; ++u) {
-                        p8[u] = WT;
+                        h8[u] = h_slot(j8[u], WH - 1);
+                        e8[u] = s.kv[h8[u]];
+                    }
+#pragma unroll
+                    for (int u = 0; u < 8; ++u) {
                         if (j8[u] == ac || !(neg ? a8[u] > 0.0 : a8[u] < 0.0)) continue;
                         if (j8[u] == i) {
                             back = true;
                             aqi = a8[u];
                             sum += a8[u];
-                        } else {
-                            const int p = lds_find<WH>(s.hkey, s.hval, j8[u]);
-                            if (p >= 0) {
-                                sum += a8[u];
-                                p8[u] = p;
-                            }
+                            continue;
                         }
+                        while (e8[u].x != j8[u] && e8[u].x != -1) {
+                            h8[u] = (h8[u] + 1) & (WH - 1);
+                            e8[u] = s.kv[h8[u]];
+                        }
+                        if (e8[u].x == -1 || e8[u].y < 0) continue;
+                        sum += a8[u];
+                        if (nt < kTerms) {
+                            ta[nt] = a8[u];
+                            tp ^= uint64_t(0xffffu ^ e8[u].y) << (16 * nt);
+                        }
+                        ++nt;
                     }
                 }
                 if (sum != 0) {
-                    info = -2;
                     dist = av / sum;
                     if (back) dterm = dist * aqi;
+                    spread = nt > kTerms;
+                    if (spread) tp = ~0ull;
+                    else
+                        for (int t = 0; t < nt; ++t) ta[t] = dist * ta[t];
                 } else {
-                    info = -3;
+                    tp = ~0ull;
                     dterm = av;
                 }
             } else if (cfa != -3) {
-                info = -3;
                 dterm = av;
             }
         }
+        s.tp[gl] = tp;
+        wave_lds_sync();
         const int maxla = __builtin_amdgcn_readlane(wave_incl_max(la), 63);
         const double aii = (go && ac == i) ? av : 0.0;
         const uint64_t has_d = __ballot(go && ac == i) & gmask;
@@ -1106,27 +1142,19 @@ __global__ __launch_bounds__(kThreads) void k_extpi_group(
             // 0.0 for the entries that add nothing (adding it changes no sum
             // that is compared or divided by)
             diagonal += __shfl(dterm, jj, G);
-            if (gl == jj) {
-                if (info >= 0) {
-                    s.pw[info] += av;
-                } else if (info == -2 && !longrow) {
-                    double t8[8];
-#pragma unroll
-                    for (int u = 0; u < 8; ++u) t8[u] = s.pw[p8[u]];
-#pragma unroll
-                    for (int u = 0; u < 8; ++u) s.pw[p8[u]] = t8[u] + dist * a8[u];
-                }
+            if (gl < kTerms) {
+                const int p = reinterpret_cast<const uint16_t *>(&s.tp[jj])[gl];
+                if (p < WT) s.pw[p] += s.ta[kTerms * jj + gl];
             }
-            const int spread = (info == -2 && longrow) ? 1 : 0;
             if (__ballot(gl == jj && spread)) {
-                // a neighbour's row of more than eight entries: a lane per entry
+                // a neighbour with more terms: its row again, a lane per entry
                 const double dj = __shfl(dist, jj, G);
                 const int ng = __shfl(neg, jj, G), bj = __shfl(b1, jj, G);
-                const int ej = __shfl(spread, jj, G) ? __shfl(e1, jj, G) : bj;
+                const int ej = __shfl(int(spread), jj, G) ? __shfl(e1, jj, G) : bj;
                 for (int q = bj + gl; q < ej; q += G) {
                     const double aq = A[q];
                     if (!(ng ? aq > 0.0 : aq < 0.0)) continue;
-                    const int p = lds_find<WH>(s.hkey, s.hval, J[q]);
+                    const int p = kv_find<WH>(s.kv, J[q]);
                     if (p >= 0) s.pw[p] += dj * aq;
                 }
             }
@@ -1171,7 +1199,7 @@ __global__ __launch_bounds__(kThreads) void k_extpi_group(
                     const int q = gl + m * G;
                     const int to = sorted ? q : rk[m];
                     if (q < c && to < max_elmts) {
-                        s.hkey[to] = s.pcol[q];
+                        keep[to] = s.pcol[q];
                         tw[to] = s.pw[q];
                     }
                 }
@@ -1186,7 +1214,7 @@ __global__ __launch_bounds__(kThreads) void k_extpi_group(
         if (go) {
             const int64_t o = out.at(i);
             for (int q = gl; q < cc; q += G) {
-                out.sj[o + q] = trunc ? s.hkey[q] : s.pcol[q];
+                out.sj[o + q] = trunc ? keep[q] : s.pcol[q];
                 out.sw[o + q] = trunc ? tw[q] * factor : s.pw[q];
             }
             if (gl == 0) {
