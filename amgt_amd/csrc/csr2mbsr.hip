@@ -9,10 +9,14 @@
 // with the diagonal), unlike the reference's windowed bitmask that assumes
 // sorted columns once ncols > 32768 (csr_matvec_device.c:701-722).
 //
-// Bins by entries per block row: <= 64 (one wave, rank sort over an LDS copy
-// of the keys), <= 1024 (256-thread workgroup, LDS bitonic), <= 8192
-// (1024-thread workgroup, LDS bitonic).  Larger block rows return
-// AMGT_ERR_UNSUPPORTED.
+// A workgroup converts a tile of consecutive block rows (cut by a pass over the
+// row pointers so that a tile starts about every 768 entries and holds at most
+// kTileCap): rank sort of each row's keys in LDS, coalesced loads and stores,
+// the tile's blocks packed.  Then one workgroup scans the tiles' block counts
+// and the packed blocks are copied to their places.  Tiles over the capacity (a
+// block row of more than 256 entries) are left to a second pass, a workgroup per
+// block row (rank sort up to kTileCap entries, LDS bitonic up to 8192).
+// Larger block rows return AMGT_ERR_UNSUPPORTED.
 #include "internal.hpp"
 #include "rowpass.hpp"
 
@@ -27,42 +31,20 @@ namespace {
 
 constexpr uint32_t kPadKey = 0xFFFFFFFFu;
 
-enum : int { kErrDup = 1, kErrCol = 2 };
+enum : int { kErrDup = 1, kErrCol = 2, kErrBig = 4, kErrPtr = 8 };
 
-// Per-conversion device scratch counters.
-struct ConvCounters {
-    int32_t bin_count[4];  // host side only: rows per bin, [3] = 1 if a row is too large
-    int32_t err;
-    int32_t pad;
-};
+constexpr int kTileThreads = 256;
+constexpr int kTileCap = 1024;   // entries of a tile
+constexpr int kTileRows = 128;   // block rows of a tile, at most
+// entries between the starts of two tiles: the tile's last block row must fit
+// behind them (257 or 513 entries); 768 for block rows of at most 128 on average
+constexpr int kTileStart = 768, kTileStartLong = 512, kTileLongRow = 128;
 
-__global__ void k_fill_i32(int32_t *p, int32_t v, int64_t n) {
-    int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (i < n) p[i] = v;
-}
-
-__global__ void k_zero_counters(ConvCounters *c) {
-    if (threadIdx.x == 0) {
-        for (int i = 0; i < 4; ++i) c->bin_count[i] = 0;
-        c->err = 0;
-        c->pad = 0;
-    }
-}
-
-__device__ __forceinline__ int bin_of(int n) {
-    return n <= 64 ? 0 : (n <= 1024 ? 1 : (n <= 8192 ? 2 : 3));
-}
-
-// Entries of block row i (CSR rows 4i .. 4i+3), for the row passes.
-struct RowEntries {
-    const int32_t *I;
-    int32_t nrows;
-    __device__ int64_t operator()(int i) const { return I[min(4 * i + 4, nrows)] - I[4 * i]; }
-};
-
-__device__ __forceinline__ void wave_sync_conv() {
-    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-    __builtin_amdgcn_wave_barrier();
+// row pointer i, kept inside [0, nnz]: the pointers are verified only with the
+// readback after the sorts, so no load may follow a wrong one out of the arrays
+__device__ __forceinline__ int entry_at(const int32_t *__restrict__ I, int i, int nnz) {
+    const int v = I[i];
+    return v < 0 ? 0 : (v > nnz ? nnz : v);
 }
 
 // Key of CSR entry p in block row starting at row r0.
@@ -79,114 +61,299 @@ __device__ __forceinline__ uint32_t entry_key(int p, int r0, int nrows, int ncol
     return (uint32_t(c >> 2) << 4) | uint32_t(r << 2) | uint32_t(c & 3);
 }
 
-// ---- bin 0: one wave per block row, <= 64 entries, rank sort in LDS.
-// tmp_col/tmp_map receive the row's blocks at offset I[4br] (upper-bound slot).
-__global__ __launch_bounds__(256) void k_sort_wave(
-    int32_t nrows, int32_t ncols, const int32_t *__restrict__ I, const int32_t *__restrict__ J,
-    const double *__restrict__ A, int32_t brow, double *__restrict__ val,
-    int32_t *__restrict__ tmp_col, uint32_t *__restrict__ tmp_map,
-    int32_t *__restrict__ blk_cnt, ConvCounters *cnt, int values_only, int packed) {
-    __shared__ __align__(16) uint32_t s_key[4][64];
-    __shared__ uint32_t s_sorted[4][64];
-    const int lane = threadIdx.x & 63;
-    const int br = blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (br >= brow) return;  // whole wave exits together
-    const int r0 = 4 * br;
-    const int s = I[r0];
-    const int e = I[min(r0 + 4, nrows)];
-    const int n = e - s;
-    if (n > 64) return;  // listed for the workgroup sorts
-    int err = 0;
-    uint32_t key = kPadKey;
-    int src = 0;
-    if (lane < n) {
-        src = s + lane;
-        key = entry_key(src, r0, nrows, ncols, I, J, &err);
+// First block row of every tile: block row br belongs to tile I[4 br] / start +
+// br / rows (start entries, rows block rows: a new tile begins where either
+// count passes a multiple).  A tile thus holds at most `rows` block rows and
+// start - 1 entries before its last one, whatever the row lengths: with a fixed
+// number of block rows per tile the regular runs of long rows of an
+// interpolation operator (24 entries per block row where the average is 13.5)
+// passed the capacity.  Every tile gets a value even for row pointers that do
+// not ascend, which are reported.
+__global__ __launch_bounds__(kTileThreads) void k_conv_cut(int32_t nrows, int32_t brow,
+                                                           int32_t nnz, int32_t start,
+                                                           int32_t rows, int32_t ntiles,
+                                                           const int32_t *__restrict__ I,
+                                                           int32_t *__restrict__ tile_lo,
+                                                           int32_t *__restrict__ err) {
+    const int br = blockIdx.x * kTileThreads + threadIdx.x;
+    if (br > brow) return;
+    if (br < brow) {
+        bool bad = false;
+        for (int r = 4 * br; r < min(4 * br + 4, nrows); ++r) bad |= I[r + 1] < I[r];
+        if (bad) atomicOr(err, kErrPtr);
     }
-    // Rank sort: every lane counts the keys below its own over an LDS copy of
-    // the row's keys (four per read; ties, i.e. duplicate entries, by lane), so
-    // the work is a few VALU operations per key instead of a 21-stage shuffle
-    // network (this kernel is bound by VALU issue).  With fewer than 2^24 - 4
-    // columns the key and the lane fit one 32-bit integer, all distinct, and
-    // the rank is one comparison per key.
-    const int w = threadIdx.x >> 6;
-    const bool valid = lane < n;
-    int rank = 0;
-    if (packed) {
-        const uint32_t pk = valid ? (key << 6) | uint32_t(lane) : kPadKey;
-        s_key[w][lane] = pk;
-        wave_sync_conv();
-        for (int j = 0; j < n; j += 4) {
-            const uint4 kk = *reinterpret_cast<const uint4 *>(&s_key[w][j]);
-            rank += kk.x < pk ? 1 : 0;
-            rank += kk.y < pk ? 1 : 0;
-            rank += kk.z < pk ? 1 : 0;
-            rank += kk.w < pk ? 1 : 0;
-        }
-    } else {
-        s_key[w][lane] = key;
-        wave_sync_conv();
-        for (int j = 0; j < n; j += 4) {
-            const uint4 kk = *reinterpret_cast<const uint4 *>(&s_key[w][j]);
-            rank += (kk.x < key || (kk.x == key && j < lane)) ? 1 : 0;
-            rank += (kk.y < key || (kk.y == key && j + 1 < lane)) ? 1 : 0;
-            rank += (kk.z < key || (kk.z == key && j + 2 < lane)) ? 1 : 0;
-            rank += (kk.w < key || (kk.w == key && j + 3 < lane)) ? 1 : 0;
-        }
-    }
-    if (valid) {
-        s_sorted[w][rank] = key;
-        if (A) val[s + rank] = A[src];
-    }
-    wave_sync_conv();
-    // lane p now holds the p-th smallest key
-    key = valid ? s_sorted[w][lane] : kPadKey;
-    const uint32_t prev = __shfl_up(key, 1);
-    if (valid && lane > 0 && prev == key) err |= kErrDup;
-    if (!values_only) {
-        const bool head = valid && (lane == 0 || (prev >> 4) != (key >> 4));
-        const uint64_t heads = __ballot(head);
-        // OR of the bits of each block: segmented inclusive scan over equal
-        // block columns; the block's last entry holds the whole bitmap
-        uint32_t map = valid ? (1u << (key & 15u)) : 0u;
-#pragma unroll
-        for (int d = 1; d < 16; d <<= 1) {
-            const uint32_t k2 = __shfl_up(key, d);
-            const uint32_t m2 = __shfl_up(map, d);
-            if (lane >= d && (k2 >> 4) == (key >> 4)) map |= m2;
-        }
-        const uint32_t nxt = __shfl_down(key, 1);
-        const bool tail = valid && (lane == n - 1 || (nxt >> 4) != (key >> 4));
-        if (tail) {
-            const uint64_t le = (lane == 63) ? ~0ull : ((2ull << lane) - 1ull);
-            const int brank = __popcll(heads & le) - 1;
-            tmp_col[s + brank] = int32_t(key >> 4);
-            tmp_map[s + brank] = map;
-        }
-        if (lane == 0) blk_cnt[br] = __popcll(heads);
-    }
-    if (err) atomicOr(&cnt->err, err);
+    const int before = br > 0 ? entry_at(I, 4 * (br - 1), nnz) / start + (br - 1) / rows : -1;
+    const int key = br < brow ? entry_at(I, 4 * br, nnz) / start + br / rows : ntiles;
+    for (int t = before + 1; t <= key; ++t) tile_lo[t] = br;
 }
 
-// ---- bins 1/2: one workgroup per block row, LDS bitonic sort of CAP keys.
+// What a tile leaves behind: its block count, the largest block count of its
+// rows and their squares' sum, error bits, whether it exceeds the capacity.
+struct TilePart {
+    int32_t blocks;
+    uint32_t mx_flags;  // largest block count << 8 | over << 4 | error bits
+    unsigned long long sumsq;
+    static constexpr uint32_t kOver = 16u;
+};
+struct ConvTotals {
+    int32_t nblk, max_blocks, err, over;
+    unsigned long long sumsq;
+};
+
+// A tile (kList: the single block rows of listed tiles, row w % kTileRows of tile
+// tiles[w / kTileRows], written to the row's own slot with its block count in
+// cnt).  Every entry's place in its block row is the number of smaller
+// keys there, counted over an LDS copy of the row's keys (four per read; rows
+// padded to a multiple of four with keys above all others).  The blocks of the
+// tile go to tmp_col / tmp_map from the tile's first entry on, packed; rel = a
+// block row's first block within the tile.
+// The entries of a tile are contiguous in the CSR and in the output, so loads
+// and stores are coalesced and all lanes work; a wave per block row (28 entries
+// of 64 lanes on 7-pt 128^3, a pass over per-row slots to pack the blocks) took
+// 241 + 126 us there against the copy rate's 67.
+template <bool kList>
+__global__ __launch_bounds__(kTileThreads) void k_conv_tile(
+    int32_t nrows, int32_t ncols, int32_t nnz, const int32_t *__restrict__ I,
+    const int32_t *__restrict__ J, const double *__restrict__ A,
+    const int32_t *__restrict__ tile_lo, const int32_t *__restrict__ tiles,
+    double *__restrict__ val, int32_t *__restrict__ tmp_col,
+    uint16_t *__restrict__ tmp_map, int32_t *__restrict__ rel_or_cnt,
+    TilePart *__restrict__ parts, int values_only) {
+    constexpr int NW = kTileThreads / 64, EPT = kTileCap / kTileThreads;
+    constexpr int kPad = kTileCap + 3 * kTileRows;
+    __shared__ __align__(16) uint32_t s_key[kPad];     // padded rows; then the block bitmaps
+    __shared__ __align__(16) uint32_t s_sorted[kTileCap];
+    __shared__ uint16_t s_rid[kTileCap];               // CSR row within the tile
+    __shared__ int s_I[4 * kTileRows + 1];             // row starts within the tile
+    __shared__ int s_ps[kTileRows + 1];                // padded block row starts
+    __shared__ int s_first[kTileRows + 1];
+    __shared__ int s_wt[NW], s_err;
+    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+    int t0, rows, part;  // first block row, block rows, index in parts
+    if constexpr (kList) {
+        part = tiles[blockIdx.x / kTileRows];
+        t0 = tile_lo[part] + int(blockIdx.x % kTileRows);
+        if (t0 >= tile_lo[part + 1]) return;
+        rows = 1;
+    } else {
+        part = blockIdx.x;
+        t0 = tile_lo[part];
+        rows = tile_lo[part + 1] - t0;
+        if (rows <= 0 || rows > kTileRows) {  // (over kTileRows: bad row pointers)
+            if (tid == 0) parts[part] = TilePart{0, 0u, 0ull};
+            return;
+        }
+    }
+    const int nr = min(4 * rows, nrows - 4 * t0);  // CSR rows
+    const int base = entry_at(I, 4 * t0, nnz);
+    const int n = entry_at(I, 4 * t0 + nr, nnz) - base;
+    if (n < 0 || n > kTileCap) {  // uniform
+        if (!kList && tid == 0) parts[part] = TilePart{0, TilePart::kOver, 0ull};
+        return;  // (kList: k_sort_block's row)
+    }
+    int cj[EPT];
+    double ca[EPT];
+#pragma unroll
+    for (int k = 0; k < EPT; ++k) {
+        const int e = tid + k * kTileThreads;
+        cj[k] = e < n ? J[base + e] : 0;
+        ca[k] = (A && e < n) ? A[base + e] : 0.0;
+    }
+    for (int t = tid; t <= nr; t += kTileThreads) {
+        const int v = entry_at(I, 4 * t0 + t, nnz) - base;
+        s_I[t] = v < 0 ? 0 : (v > n ? n : v);
+    }
+    for (int t = tid; t < kPad; t += kTileThreads) s_key[t] = kPadKey;
+    for (int t = tid; t < kTileCap; t += kTileThreads) {
+        s_sorted[t] = kPadKey;
+        s_rid[t] = 0;
+    }
+    if (tid == 0) s_err = 0;
+    __syncthreads();
+    if (w == 0) {  // padded starts of the block rows, two per lane
+        int len[2];
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            const int r = 2 * lane + u;
+            len[u] = 0;
+            if (r < rows) len[u] = (max(s_I[min(4 * r + 4, nr)] - s_I[4 * r], 0) + 3) & ~3;
+        }
+        const int incl = wave_incl_sum(len[0] + len[1]);
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            const int at = incl - len[1] - (u == 0 ? len[0] : 0);
+            if (2 * lane + u <= rows) s_ps[2 * lane + u] = at;
+        }
+        if (lane == 63 && rows == kTileRows) s_ps[rows] = incl;
+    }
+    {  // the entries' rows: a power of two of lanes per row
+        int lpr = kTileThreads;
+        while (lpr > 1 && nr * lpr > kTileThreads) lpr >>= 1;
+        for (int row = tid / lpr; row < nr; row += kTileThreads / lpr)
+            for (int e = s_I[row] + tid % lpr; e < s_I[row + 1]; e += lpr) s_rid[e] = uint16_t(row);
+    }
+    __syncthreads();
+    uint32_t key[EPT];
+    int rid[EPT];
+    int err = 0;
+#pragma unroll
+    for (int k = 0; k < EPT; ++k) {
+        const int e = tid + k * kTileThreads;
+        key[k] = kPadKey;
+        rid[k] = 0;
+        if (e < n) {
+            int c = cj[k];
+            if (c < 0 || c >= ncols) {
+                err |= kErrCol;
+                c = 0;
+            }
+            rid[k] = s_rid[e];
+            const int br = rid[k] >> 2;
+            key[k] = (uint32_t(c >> 2) << 4) | uint32_t((rid[k] & 3) << 2) | uint32_t(c & 3);
+            const int at = s_ps[br] + (e - s_I[4 * br]);
+            if (at >= 0 && at < kPad) s_key[at] = key[k];  // (always, for ascending pointers)
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < EPT; ++k) {
+        const int e = tid + k * kTileThreads;
+        if (e >= n) continue;
+        const int br = rid[k] >> 2;
+        int rank = 0;
+        const int j1 = min(s_ps[br + 1], kPad);
+        for (int j = s_ps[br]; j < j1; j += 4) {
+            const uint4 kk = *reinterpret_cast<const uint4 *>(&s_key[j]);
+            rank += kk.x < key[k] ? 1 : 0;
+            rank += kk.y < key[k] ? 1 : 0;
+            rank += kk.z < key[k] ? 1 : 0;
+            rank += kk.w < key[k] ? 1 : 0;
+        }
+        const int to = min(s_I[4 * br] + rank, n - 1);
+        s_sorted[to] = key[k];
+        // places within the entry's own block row: a wave's stores stay within a
+        // few cache lines
+        if (A) val[base + to] = ca[k];
+    }
+    __syncthreads();
+    // four consecutive sorted entries per thread; equal keys (duplicate
+    // entries) share a place and leave a hole
+    const int p0 = EPT * tid;
+    uint32_t sk[EPT];
+    int sb[EPT], head[EPT], nh = 0;
+    uint32_t pk = (p0 > 0 && p0 < n) ? s_sorted[p0 - 1] : kPadKey;
+    int pb = (p0 > 0 && p0 < n) ? s_rid[p0 - 1] >> 2 : -1;
+#pragma unroll
+    for (int k = 0; k < EPT; ++k) {
+        const bool in = p0 + k < n;
+        sk[k] = in ? s_sorted[p0 + k] : kPadKey;
+        sb[k] = in ? s_rid[p0 + k] >> 2 : -1;
+        if (in && sk[k] == kPadKey) err |= kErrDup;
+        head[k] = in && (sb[k] != pb || (sk[k] >> 4) != (pk >> 4)) ? 1 : 0;
+        nh += head[k];
+        pk = sk[k];
+        pb = sb[k];
+    }
+    if (err) atomicOr(&s_err, err);
+    if (values_only) {
+        __syncthreads();
+        if (tid == 0) {
+            if constexpr (kList) {
+                if (s_err) atomicOr(&parts[part].mx_flags, uint32_t(s_err));
+            } else {
+                parts[part] = TilePart{0, uint32_t(s_err), 0ull};
+            }
+        }
+        return;
+    }
+    const int incl = wave_incl_sum(nh);
+    if (lane == 63) s_wt[w] = incl;
+    for (int t = tid; t < kTileCap; t += kTileThreads) s_key[t] = 0u;  // the bitmaps
+    __syncthreads();
+    int slot = incl - nh - 1, total = 0;  // the block of the entry before this thread's
+#pragma unroll
+    for (int q = 0; q < NW; ++q) {
+        if (q < w) slot += s_wt[q];
+        total += s_wt[q];
+    }
+    uint32_t map = 0;
+    int prevb = (p0 > 0 && p0 < n) ? s_rid[p0 - 1] >> 2 : -1;
+#pragma unroll
+    for (int k = 0; k < EPT; ++k) {
+        if (p0 + k >= n) break;
+        if (head[k]) {
+            if (map) atomicOr(&s_key[slot], map);
+            map = 0;
+            ++slot;
+            tmp_col[base + slot] = int32_t(sk[k] >> 4);
+            if (sb[k] != prevb) s_first[sb[k]] = slot;
+        }
+        map |= 1u << (sk[k] & 15u);
+        prevb = sb[k];
+    }
+    if (map) atomicOr(&s_key[slot], map);
+    __syncthreads();
+    for (int t = tid; t < total; t += kTileThreads) tmp_map[base + t] = uint16_t(s_key[t]);
+    if (w == 0) {
+        // a row's first block; an empty row's is the next entry's
+        auto first_of = [&](int br) {
+            if (br >= rows) return total;
+            const int lo = s_I[4 * br];
+            return lo < n ? s_first[s_rid[lo] >> 2] : total;
+        };
+        if constexpr (kList) {
+            if (lane == 0) {
+                rel_or_cnt[t0] = total;
+                if (s_err) atomicOr(&parts[part].mx_flags, uint32_t(s_err));
+            }
+        } else {
+            unsigned long long sq = 0ull;
+            int mx = 0;
+            const int f0 = first_of(2 * lane), f1 = first_of(2 * lane + 1),
+                      f2 = first_of(2 * lane + 2);
+#pragma unroll
+            for (int u = 0; u < 2; ++u) {
+                const int c = max(u == 0 ? f1 - f0 : f2 - f1, 0);
+                if (2 * lane + u >= rows) continue;
+                rel_or_cnt[t0 + 2 * lane + u] = u == 0 ? f0 : f1;
+                sq += static_cast<unsigned long long>(c) * unsigned(c);
+                mx = max(mx, c);
+            }
+            for (int d = 32; d > 0; d >>= 1) sq += __shfl_xor(sq, d);
+            mx = wave_incl_max(mx);
+            if (lane == 63)
+                parts[part] = TilePart{total, uint32_t(mx) << 8 | uint32_t(s_err), sq};
+        }
+    }
+}
+
+// ---- block rows of kTileCap + 1 to CAP entries in listed tiles: a workgroup per
+// row (workgroup w: row w % kTileRows of tile tiles[w / kTileRows]), LDS bitonic
+// sort of CAP keys.
 template <int THREADS, int CAP>
 __global__ __launch_bounds__(THREADS) void k_sort_block(
-    int32_t nrows, int32_t ncols, const int32_t *__restrict__ I, const int32_t *__restrict__ J,
-    const double *__restrict__ A, const int32_t *__restrict__ list, int32_t count,
-    double *__restrict__ val, int32_t *__restrict__ tmp_col, uint32_t *__restrict__ tmp_map,
-    int32_t *__restrict__ blk_cnt, ConvCounters *cnt, int values_only) {
+    int32_t nrows, int32_t ncols, int32_t nnz, const int32_t *__restrict__ I,
+    const int32_t *__restrict__ J, const double *__restrict__ A,
+    const int32_t *__restrict__ tile_lo, const int32_t *__restrict__ tiles,
+    double *__restrict__ val, int32_t *__restrict__ tmp_col,
+    uint16_t *__restrict__ tmp_map, int32_t *__restrict__ blk_cnt, int32_t *__restrict__ err_out,
+    int values_only) {
     __shared__ uint32_t s_key[CAP];
     __shared__ int32_t s_aux[CAP];  // source index, then block rank
     __shared__ int32_t s_wave_tot[THREADS / 64];
     __shared__ int s_err;
     const int t = threadIdx.x;
-    const int w = blockIdx.x;
-    if (w >= count) return;
-    const int br = list[w];
+    const int tile = tiles[blockIdx.x / kTileRows];
+    const int br = tile_lo[tile] + int(blockIdx.x % kTileRows);
+    if (br >= tile_lo[tile + 1]) return;
     const int r0 = 4 * br;
-    const int s = I[r0];
-    const int e = I[min(r0 + 4, nrows)];
-    const int n = e - s;
+    const int s = entry_at(I, r0, nnz);
+    const int n = entry_at(I, min(r0 + 4, nrows), nnz) - s;
+    if (n <= kTileCap) return;  // k_conv_tile's row
+    if (n > CAP) {
+        if (t == 0) atomicOr(err_out, kErrBig);
+        return;
+    }
     int np = 64;
     while (np < n) np <<= 1;
     if (t == 0) s_err = 0;
@@ -263,38 +430,160 @@ __global__ __launch_bounds__(THREADS) void k_sort_block(
                 }
                 int rank = s_aux[i];
                 tmp_col[s + rank] = int32_t(key >> 4);
-                tmp_map[s + rank] = map;
+                tmp_map[s + rank] = uint16_t(map);
             }
         }
         if (t == 0) blk_cnt[br] = carry;
     }
-    if (t == 0 && s_err) atomicOr(&cnt->err, s_err);
+    if (t == 0 && s_err) atomicOr(err_out, s_err);
 }
 
-// Copies each block row's blocks from the upper-bound slot to the compact
-// arrays; one wave per block row.
-__global__ __launch_bounds__(256) void k_compact(int32_t nrows, int32_t brow,
-                                                 const int32_t *__restrict__ I,
-                                                 const int32_t *__restrict__ blk_ptr,
-                                                 const int32_t *__restrict__ tmp_col,
-                                                 const uint32_t *__restrict__ tmp_map,
-                                                 int32_t *__restrict__ blk_col,
-                                                 uint16_t *__restrict__ blk_map,
-                                                 int32_t *__restrict__ val_ptr) {
-    const int lane = threadIdx.x & 63;
-    const int br = blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (br > brow) return;
-    if (br == brow) {
-        if (lane == 0) val_ptr[brow] = I[nrows];
+// Block counts of the rows of listed tiles (cnt) -> the tile's part and the
+// rows' first blocks within the tile, in place; a workgroup per tile.
+__global__ __launch_bounds__(64) void k_conv_list_sum(const int32_t *__restrict__ tile_lo,
+                                                      const int32_t *__restrict__ tiles,
+                                                      int32_t *__restrict__ cnt,
+                                                      TilePart *__restrict__ parts) {
+    const int t = tiles[blockIdx.x], lane = threadIdx.x;
+    int run = 0, mx = 0;
+    unsigned long long sq = 0ull;
+    for (int b0 = tile_lo[t]; b0 < tile_lo[t + 1]; b0 += 64) {
+        const int br = b0 + lane;
+        const bool in = br < tile_lo[t + 1];
+        const int c = in ? cnt[br] : 0;
+        const int incl = wave_incl_sum(c);
+        if (in) cnt[br] = run + incl - c;
+        run += __builtin_amdgcn_readlane(incl, 63);
+        mx = max(mx, c);
+        sq += static_cast<unsigned long long>(c) * unsigned(c);
+    }
+    for (int d = 32; d > 0; d >>= 1) {
+        sq += __shfl_xor(sq, d);
+        mx = max(mx, __shfl_xor(mx, d));
+    }
+    if (lane == 0) {
+        TilePart &p = parts[t];
+        p.blocks = run;
+        p.mx_flags = (p.mx_flags & 0xffu) | uint32_t(mx) << 8;
+        p.sumsq = sq;
+    }
+}
+
+// One workgroup: the tiles' first blocks, the totals and the list of the tiles
+// over the capacity (in no order); four consecutive tiles per thread and step.
+constexpr int kFinThreads = 1024;
+__global__ __launch_bounds__(kFinThreads) void k_conv_finish(int32_t ntiles,
+                                                             const TilePart *__restrict__ parts,
+                                                             const int32_t *__restrict__ err_in,
+                                                             int32_t *__restrict__ first,
+                                                             int32_t *__restrict__ tiles,
+                                                             ConvTotals *__restrict__ tot) {
+    constexpr int NW = kFinThreads / 64;
+    __shared__ int s_w[NW], s_mx[NW], s_err[NW], s_over;
+    __shared__ unsigned long long s_sq[NW];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    int run = 0, mx = 0, err = 0;
+    unsigned long long sq = 0ull;
+    if (threadIdx.x == 0) s_over = 0;
+    __syncthreads();
+    for (int g = 0; g < ntiles; g += 4 * kFinThreads) {
+        const int t = g + 4 * int(threadIdx.x);
+        TilePart p[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) p[u] = t + u < ntiles ? parts[t + u] : TilePart{};
+        int sum = 0;
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            sum += p[u].blocks;
+            mx = max(mx, int(p[u].mx_flags >> 8));
+            err |= int(p[u].mx_flags & 15u);
+            if (p[u].mx_flags & TilePart::kOver) tiles[atomicAdd(&s_over, 1)] = t + u;
+            sq += p[u].sumsq;
+        }
+        const int incl = wave_incl_sum(sum);
+        __syncthreads();  // the previous step's totals are read
+        if (lane == 63) s_w[w] = incl;
+        __syncthreads();
+        int at = run + incl - sum, all = 0;
+#pragma unroll
+        for (int q = 0; q < NW; ++q) {
+            if (q < w) at += s_w[q];
+            all += s_w[q];
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            if (t + u < ntiles) first[t + u] = at;
+            at += p[u].blocks;
+        }
+        run += all;
+    }
+    for (int d = 32; d > 0; d >>= 1) {
+        mx = max(mx, __shfl_xor(mx, d));
+        err |= __shfl_xor(err, d);
+        sq += __shfl_xor(sq, d);
+    }
+    if (lane == 0) {
+        s_mx[w] = mx;
+        s_err[w] = err;
+        s_sq[w] = sq;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        ConvTotals r{run, 0, *err_in, s_over, 0ull};
+        for (int q = 0; q < NW; ++q) {
+            r.max_blocks = max(r.max_blocks, s_mx[q]);
+            r.err |= s_err[q];
+            r.sumsq += s_sq[q];
+        }
+        *tot = r;
+    }
+}
+
+__global__ void k_conv_zero(int32_t *p) {
+    if (threadIdx.x == 0) *p = 0;
+}
+
+// row pointers of a matrix without rows
+__global__ void k_empty_ptrs(int32_t *blk_ptr, int32_t *val_ptr) {
+    if (threadIdx.x == 0) blk_ptr[0] = val_ptr[0] = 0;
+}
+
+// The tiles' blocks to their places, block and value row pointers.
+__global__ __launch_bounds__(kTileThreads) void k_conv_pack(
+    int32_t nrows, int32_t brow, int32_t nblk, const int32_t *__restrict__ I,
+    const int32_t *__restrict__ tile_lo, const TilePart *__restrict__ parts, const int32_t *__restrict__ first,
+    const int32_t *__restrict__ rel, const int32_t *__restrict__ tmp_col,
+    const uint16_t *__restrict__ tmp_map, int32_t *__restrict__ blk_ptr,
+    int32_t *__restrict__ blk_col, uint16_t *__restrict__ blk_map,
+    int32_t *__restrict__ val_ptr) {
+    const int t = blockIdx.x, t0 = tile_lo[t], rows = tile_lo[t + 1] - t0;
+    if (rows <= 0) return;
+    const int to = first[t];
+    if (threadIdx.x < unsigned(rows)) {  // rows <= kTileRows < kTileThreads
+        blk_ptr[t0 + threadIdx.x] = to + rel[t0 + threadIdx.x];
+        val_ptr[t0 + threadIdx.x] = I[4 * (t0 + threadIdx.x)];
+    }
+    if (t0 + rows == brow && threadIdx.x == 0) {
+        blk_ptr[brow] = nblk;
+        val_ptr[brow] = I[nrows];
+    }
+    const int blocks = parts[t].blocks;
+    if (!(parts[t].mx_flags & TilePart::kOver)) {
+        const int from = I[4 * t0];
+        for (int k = threadIdx.x; k < blocks; k += kTileThreads) {
+            blk_col[to + k] = tmp_col[from + k];
+            blk_map[to + k] = tmp_map[from + k];
+        }
         return;
     }
-    const int s = I[4 * br];
-    const int p0 = blk_ptr[br], p1 = blk_ptr[br + 1];
-    for (int t = lane; t < p1 - p0; t += 64) {
-        blk_col[p0 + t] = tmp_col[s + t];
-        blk_map[p0 + t] = uint16_t(tmp_map[s + t]);
+    for (int r = 0; r < rows; ++r) {  // each row in its own slot
+        const int from = I[4 * (t0 + r)], f = rel[t0 + r];
+        const int c = (r + 1 < rows ? rel[t0 + r + 1] : blocks) - f;
+        for (int k = threadIdx.x; k < c; k += kTileThreads) {
+            blk_col[to + f + k] = tmp_col[from + k];
+            blk_map[to + f + k] = tmp_map[from + k];
+        }
     }
-    if (lane == 0) val_ptr[br] = s;
 }
 
 }  // namespace
@@ -320,78 +609,104 @@ double stand_from(const RowStats &h, int64_t nblk, int32_t brow) {
 
 namespace {
 
-int launch_sorts(int32_t nrows, int32_t ncols, const int32_t *I, const int32_t *J, const double *A,
-                 const int32_t *list, int32_t brow, const int32_t bin_count[4], double *val,
-                 int32_t *tmp_col, uint32_t *tmp_map, int32_t *blk_cnt, ConvCounters *cnt,
-                 int values_only, hipStream_t s) {
-    if (bin_count[3] > 0) {
-        set_error("CSR->mBSR: a block row has more than 8192 entries (4 rows with > 2048 "
-                  "nonzeros on average); this build does not convert such rows");
-        return AMGT_ERR_UNSUPPORTED;
+// Device scratch of one conversion.
+struct ConvWork {
+    int32_t ntiles = 0;
+    TilePart *parts = nullptr;
+    ConvTotals *tot = nullptr;
+    int32_t *first = nullptr, *rel = nullptr, *tmp_col = nullptr, *tiles = nullptr;
+    int32_t *tile_lo = nullptr, *err = nullptr;
+    uint16_t *tmp_map = nullptr;
+    hipStream_t s = nullptr;
+    ~ConvWork() {
+        tmp_free(parts, s);
+        tmp_free(tot, s);
+        tmp_free(first, s);
+        tmp_free(rel, s);
+        tmp_free(tmp_col, s);
+        tmp_free(tmp_map, s);
+        tmp_free(tiles, s);
+        tmp_free(tile_lo, s);
+        tmp_free(err, s);
     }
-    if (brow > 0) {
-        int grid = (brow + 3) / 4;
-        // columns <= 2^24 - 5: keys below 2^26 - 16, packed keys below kPadKey
-        const int packed = ncols < (1 << 24) - 4 ? 1 : 0;
-        hipLaunchKernelGGL(k_sort_wave, dim3(grid), dim3(256), 0, s, nrows, ncols, I, J, A, brow,
-                           val, tmp_col, tmp_map, blk_cnt, cnt, values_only, packed);
-        AMGT_HIP(hipGetLastError());
+};
+
+// Sorts every tile (values, and unless values_only the packed blocks) and reads
+// the totals back with rowptr[0] and rowptr[nrows], which are verified: one
+// synchronisation unless a tile exceeds the capacity.
+int sort_tiles(int32_t nrows, int32_t ncols, int64_t nnz, const int32_t *I, const int32_t *J,
+               const double *A, int32_t brow, double *val, int values_only, ConvWork &w,
+               ConvTotals *ht, hipStream_t s) {
+    w.s = s;
+    // smaller tiles where there would be too few to fill the chip
+    const int32_t nz = int32_t(nnz);
+    const int32_t full = nnz <= int64_t(kTileLongRow) * brow ? kTileStart : kTileStartLong;
+    const int32_t start = std::max(64, std::min(full, nz / 2048));
+    const int32_t rows = std::max(4, std::min(kTileRows, brow / 1024));
+    w.ntiles = brow > 0 ? nz / start + brow / rows + 1 : 0;
+    AMGT_TRY(tmp_alloc_t(&w.tile_lo, size_t(w.ntiles) + 1, s));
+    AMGT_TRY(tmp_alloc_t(&w.err, 1, s));
+    AMGT_TRY(tmp_alloc_t(&w.parts, size_t(w.ntiles), s));
+    AMGT_TRY(tmp_alloc_t(&w.tot, 1, s));
+    AMGT_TRY(tmp_alloc_t(&w.first, size_t(w.ntiles), s));
+    AMGT_TRY(tmp_alloc_t(&w.tiles, size_t(w.ntiles), s));
+    if (!values_only) {
+        AMGT_TRY(tmp_alloc_t(&w.rel, size_t(brow), s));
+        AMGT_TRY(tmp_alloc_t(&w.tmp_col, size_t(nnz), s));
+        AMGT_TRY(tmp_alloc_t(&w.tmp_map, size_t(nnz), s));
     }
-    if (bin_count[1] > 0) {
-        hipLaunchKernelGGL((k_sort_block<256, 1024>), dim3(bin_count[1]), dim3(256), 0, s, nrows,
-                           ncols, I, J, A, list + brow, bin_count[1], val, tmp_col, tmp_map,
-                           blk_cnt, cnt, values_only);
-        AMGT_HIP(hipGetLastError());
+    hipLaunchKernelGGL(k_conv_zero, dim3(1), dim3(64), 0, s, w.err);
+    if (w.ntiles > 0) {
+        hipLaunchKernelGGL(k_conv_cut, dim3(unsigned(brow / kTileThreads + 1)), dim3(kTileThreads),
+                           0, s, nrows, brow, nz, start, rows, w.ntiles, I, w.tile_lo, w.err);
+        hipLaunchKernelGGL((k_conv_tile<false>), dim3(unsigned(w.ntiles)), dim3(kTileThreads), 0,
+                           s, nrows, ncols, nz, I, J, A, w.tile_lo,
+                           static_cast<const int32_t *>(nullptr), val, w.tmp_col, w.tmp_map, w.rel,
+                           w.parts, values_only);
     }
-    if (bin_count[2] > 0) {
-        hipLaunchKernelGGL((k_sort_block<1024, 8192>), dim3(bin_count[2]), dim3(1024), 0, s,
-                           nrows, ncols, I, J, A, list + 2 * int64_t(brow), bin_count[2], val,
-                           tmp_col, tmp_map, blk_cnt, cnt, values_only);
+    auto totals = [&](int32_t *ends) -> int {
+        hipLaunchKernelGGL(k_conv_finish, dim3(1), dim3(kFinThreads), 0, s, w.ntiles, w.parts,
+                           w.err, w.first, w.tiles, w.tot);
         AMGT_HIP(hipGetLastError());
+        const Readback rb[3] = {{ht, w.tot, sizeof(ConvTotals)},
+                                {&ends[0], I, sizeof(int32_t)},
+                                {&ends[1], I + nrows, sizeof(int32_t)}};
+        return readback(rb, 3, s);
+    };
+    int32_t ends[2] = {0, 0};
+    AMGT_TRY(totals(ends));
+    if (ends[0] != 0 || int64_t(ends[1]) != nnz) {
+        set_error("CSR->mBSR: rowptr[0] must be 0 and rowptr[nrows] must equal nnz");
+        return AMGT_ERR_INPUT;
+    }
+    if (ht->err & kErrPtr) {
+        set_error("CSR->mBSR: row pointers must ascend");
+        return AMGT_ERR_INPUT;
+    }
+    if (ht->over > 0) {  // the rows of the tiles over the capacity, one by one
+        const int32_t nt = ht->over;
+        const dim3 grid(unsigned(nt) * unsigned(kTileRows));
+        hipLaunchKernelGGL((k_conv_tile<true>), grid, dim3(kTileThreads), 0, s, nrows, ncols, nz, I,
+                           J, A, w.tile_lo, w.tiles, val, w.tmp_col, w.tmp_map, w.rel, w.parts,
+                           values_only);
+        hipLaunchKernelGGL((k_sort_block<1024, 8192>), grid, dim3(1024), 0, s, nrows, ncols, nz, I,
+                           J, A, w.tile_lo, w.tiles, val, w.tmp_col, w.tmp_map, w.rel,
+                           w.err, values_only);
+        if (!values_only)
+            hipLaunchKernelGGL(k_conv_list_sum, dim3(unsigned(nt)), dim3(64), 0, s,
+                               w.tile_lo, w.tiles, w.rel, w.parts);
+        AMGT_HIP(hipGetLastError());
+        AMGT_TRY(totals(ends));
+        if (ht->err & kErrBig) {
+            set_error("CSR->mBSR: a block row has more than 8192 entries (4 rows with > 2048 "
+                      "nonzeros on average); this build does not convert such rows");
+            return AMGT_ERR_UNSUPPORTED;
+        }
     }
     return AMGT_OK;
 }
 
-struct HostHeader {
-    int32_t i0, in;
-};
-
 }  // namespace
-
-// Bins block rows by entries: <= 64 (wave sort, not listed: it walks every
-// block row), <= 1024 and larger (listed at list + brow and list + 2*brow for
-// the workgroup sorts).  bin_count[3] flags a block row over 8192 entries.
-// hh (optional): I[0] and I[nrows], read back with the bins.
-static int bin_block_rows(int32_t nrows, int32_t brow, const int32_t *I, int32_t **list,
-                          ConvCounters *cnt, ConvCounters *h_cnt, HostHeader *hh,
-                          hipStream_t s) {
-    AMGT_TRY(tmp_alloc_t(list, size_t(brow) * 3 + 1, s));
-    rowpass::Part *parts = nullptr;
-    RowStats *tot = nullptr;
-    AMGT_TRY(tmp_alloc_t(&parts, size_t(rowpass::groups(brow)) + 1, s));
-    AMGT_TRY(tmp_alloc_t(&tot, 1, s));
-    hipLaunchKernelGGL(k_zero_counters, dim3(1), dim3(64), 0, s, cnt);
-    AMGT_HIP(hipGetLastError());
-    const RowEntries f{I, nrows};
-    int st = rowpass::count(brow, f, 64, 1024, parts, tot, s);
-    RowStats ht{};
-    if (st == AMGT_OK) {
-        const Readback rb[3] = {{&ht, tot, sizeof(RowStats)},
-                                {hh ? &hh->i0 : nullptr, I, sizeof(int32_t)},
-                                {hh ? &hh->in : nullptr, I + nrows, sizeof(int32_t)}};
-        st = readback(rb, hh ? 3 : 1, s);
-    }
-    *h_cnt = ConvCounters{};
-    h_cnt->bin_count[0] = ht.cnt[0];
-    h_cnt->bin_count[1] = ht.cnt[1];
-    h_cnt->bin_count[2] = ht.cnt[2];
-    h_cnt->bin_count[3] = ht.max_blocks > 8192 ? 1 : 0;
-    if (st == AMGT_OK && h_cnt->bin_count[3] == 0 && ht.cnt[1] + ht.cnt[2] > 0)
-        st = rowpass::scatter(brow, f, 64, 1024, parts, *list, int64_t(brow), 6u, s);
-    tmp_free(parts, s);
-    tmp_free(tot, s);
-    return st;
-}
 
 int csr_to_mbsr(int32_t nrows, int32_t ncols, int64_t nnz, const int32_t *rowptr,
                 const int32_t *colidx, const double *A, hipStream_t s, Mbsr *out) {
@@ -413,9 +728,6 @@ int csr_to_mbsr(int32_t nrows, int32_t ncols, int64_t nnz, const int32_t *rowptr
         set_error("CSR->mBSR: ncols > 2^30 - 8 does not fit the 32-bit sort key");
         return AMGT_ERR_UNSUPPORTED;
     }
-    // I[0] == 0 and I[nrows] == nnz are verified with the bins' readback below
-    HostHeader hh{0, 0};
-
     m.blk_ptr = static_cast<int32_t *>(dev_alloc(sizeof(int32_t) * (size_t(m.brow) + 1), s));
     m.val_ptr = static_cast<int32_t *>(dev_alloc(sizeof(int32_t) * (size_t(m.brow) + 1), s));
     if (!m.blk_ptr || !m.val_ptr) {
@@ -429,85 +741,37 @@ int csr_to_mbsr(int32_t nrows, int32_t ncols, int64_t nnz, const int32_t *rowptr
             return AMGT_ERR_ALLOC;
         }
     }
-    ConvCounters *cnt = nullptr;
-    AMGT_TRY(tmp_alloc_t(&cnt, 1, s));
-    ConvCounters hc;
-    int32_t *list = nullptr;
-    int st = bin_block_rows(nrows, m.brow, rowptr, &list, cnt, &hc, &hh, s);
-    if (st != AMGT_OK) {
-        tmp_free(cnt, s);
-        return st;
-    }
-    if (hh.i0 != 0 || int64_t(hh.in) != nnz) {
-        tmp_free(list, s);
-        tmp_free(cnt, s);
-        set_error("CSR->mBSR: rowptr[0] must be 0 and rowptr[nrows] must equal nnz");
+    ConvWork w;
+    ConvTotals ht{};
+    AMGT_TRY(sort_tiles(nrows, ncols, nnz, rowptr, colidx, A, m.brow, m.val, 0, w, &ht, s));
+    if (ht.err & kErrCol) {
+        set_error("CSR->mBSR: column index out of range");
         return AMGT_ERR_INPUT;
     }
-    int32_t *tmp_col = nullptr, *blk_cnt = nullptr;
-    uint32_t *tmp_map = nullptr;
-    RowStats *rstats = nullptr;
-    RowStats hrs{};
-    st = tmp_alloc_t(&rstats, 1, s);
-    if (st == AMGT_OK) st = tmp_alloc_t(&tmp_col, size_t(nnz), s);
-    if (st == AMGT_OK) st = tmp_alloc_t(&tmp_map, size_t(nnz), s);
-    if (st == AMGT_OK) st = tmp_alloc_t(&blk_cnt, size_t(m.brow) + 1, s);
-    if (st == AMGT_OK && m.brow > 0) {
-        hipLaunchKernelGGL(k_fill_i32, dim3((m.brow + 255) / 256), dim3(256), 0, s, blk_cnt, 0,
-                           int64_t(m.brow));
-        st = launch_sorts(nrows, ncols, rowptr, colidx, A, list, m.brow, hc.bin_count, m.val,
-                          tmp_col, tmp_map, blk_cnt, cnt, 0, s);
+    if (ht.err & kErrDup) {
+        set_error("CSR->mBSR: duplicate (row, col) entry");
+        return AMGT_ERR_INPUT;
     }
-    if (st == AMGT_OK) st = exclusive_scan_i32(blk_cnt, m.blk_ptr, m.brow, s);
-    int32_t nblk = 0;
-    if (st == AMGT_OK) {
-        const Readback rb[1] = {{&nblk, m.blk_ptr + m.brow, sizeof(int32_t)}};
-        st = readback(rb, 1, s);
+    const int32_t nblk = ht.nblk;
+    m.nblk = nblk;
+    m.blk_col = static_cast<int32_t *>(dev_alloc(sizeof(int32_t) * size_t(nblk ? nblk : 1), s));
+    m.blk_map = static_cast<uint16_t *>(dev_alloc(sizeof(uint16_t) * size_t(nblk ? nblk : 1), s));
+    if (!m.blk_col || !m.blk_map) {
+        set_error("CSR->mBSR: block allocation failed");
+        return AMGT_ERR_ALLOC;
     }
-    if (st == AMGT_OK) {
-        m.nblk = nblk;
-        m.blk_col = static_cast<int32_t *>(dev_alloc(sizeof(int32_t) * size_t(nblk ? nblk : 1), s));
-        m.blk_map = static_cast<uint16_t *>(dev_alloc(sizeof(uint16_t) * size_t(nblk ? nblk : 1), s));
-        if (!m.blk_col || !m.blk_map) {
-            set_error("CSR->mBSR: block allocation failed");
-            st = AMGT_ERR_ALLOC;
-        }
-    }
-    if (st == AMGT_OK) {
-        hipLaunchKernelGGL(k_compact, dim3((m.brow + 1 + 3) / 4), dim3(256), 0, s, nrows, m.brow,
-                           rowptr, m.blk_ptr, tmp_col, tmp_map, m.blk_col, m.blk_map, m.val_ptr);
-        st = row_stats_launch(m.blk_ptr, m.brow, rstats, s);
-        hipError_t e = hipGetLastError();
-        if (st == AMGT_OK && e != hipSuccess) {
-            set_error(std::string("CSR->mBSR: ") + hipGetErrorString(e));
-            st = AMGT_ERR_HIP;
-        }
-        if (st == AMGT_OK) {
-            const Readback rb[2] = {{&hc, cnt, sizeof(ConvCounters)},
-                                    {&hrs, rstats, sizeof(RowStats)}};
-            st = readback(rb, 2, s);
-        }
-        if (st == AMGT_OK) {
-            m.stand = stand_from(hrs, nblk, m.brow);
-            m.avg_nnz = nblk ? double(nnz) / double(nblk) : 0.0;
-            m.max_row_blocks = hrs.max_blocks;
-            m.spmv_kernel = default_spmv_kernel(m);
-            if (hc.err & kErrCol) {
-                set_error("CSR->mBSR: column index out of range");
-                st = AMGT_ERR_INPUT;
-            } else if (hc.err & kErrDup) {
-                set_error("CSR->mBSR: duplicate (row, col) entry");
-                st = AMGT_ERR_INPUT;
-            }
-        }
-    }
-    tmp_free(tmp_col, s);
-    tmp_free(tmp_map, s);
-    tmp_free(blk_cnt, s);
-    tmp_free(rstats, s);
-    tmp_free(list, s);
-    tmp_free(cnt, s);
-    return st;
+    if (w.ntiles > 0)
+        hipLaunchKernelGGL(k_conv_pack, dim3(unsigned(w.ntiles)), dim3(kTileThreads), 0, s, nrows,
+                           m.brow, nblk, rowptr, w.tile_lo, w.parts, w.first, w.rel, w.tmp_col,
+                           w.tmp_map, m.blk_ptr, m.blk_col, m.blk_map, m.val_ptr);
+    else
+        hipLaunchKernelGGL(k_empty_ptrs, dim3(1), dim3(64), 0, s, m.blk_ptr, m.val_ptr);
+    AMGT_HIP(hipGetLastError());
+    m.stand = stand_from(RowStats{{0, 0, 0}, ht.max_blocks, ht.sumsq}, nblk, m.brow);
+    m.avg_nnz = nblk ? double(nnz) / double(nblk) : 0.0;
+    m.max_row_blocks = ht.max_blocks;
+    m.spmv_kernel = default_spmv_kernel(m);
+    return AMGT_OK;
 }
 
 int mbsr_refresh_values(Mbsr *Ap, const int32_t *rowptr, const int32_t *colidx,
@@ -521,16 +785,9 @@ int mbsr_refresh_values(Mbsr *Ap, const int32_t *rowptr, const int32_t *colidx,
         }
         m.pattern_only = false;
     }
-    ConvCounters *cnt = nullptr;
-    AMGT_TRY(tmp_alloc_t(&cnt, 1, s));
-    ConvCounters hc;
-    int32_t *list = nullptr;
-    int st = bin_block_rows(m.nrows, m.brow, rowptr, &list, cnt, &hc, nullptr, s);
-    if (st == AMGT_OK && m.brow > 0)
-        st = launch_sorts(m.nrows, m.ncols, rowptr, colidx, A, list, m.brow, hc.bin_count, m.val,
-                          nullptr, nullptr, nullptr, cnt, 1, s);
-    tmp_free(list, s);
-    tmp_free(cnt, s);
+    ConvWork w;
+    ConvTotals ht{};
+    const int st = sort_tiles(m.nrows, m.ncols, m.nnz, rowptr, colidx, A, m.brow, m.val, 1, w, &ht, s);
     // low-precision copies and the transpose are stale now
     dev_free(m.val32, s);
     m.val32 = nullptr;

@@ -82,6 +82,33 @@ def test_conversion_bit_exact(dev, name):
     check_structure(M, ref)
 
 
+# (rows, columns, entries per CSR row): tiles of the conversion filled to their
+# capacity of 1024 entries and one past it, in one block row or over many; a
+# last block row of 1 to 3 CSR rows; one tall block row among empty ones
+@pytest.mark.parametrize("m,n,lens", [
+    (4, 2000, [256] * 4), (4, 2000, [256, 257, 256, 256]), (8, 2000, [0, 0, 1024, 0, 1, 0, 0, 1024]),
+    (4 * 40, 900, [7] * 160), (4 * 4100 + 1, 300, [5] * 16401), (4 * 300 + 3, 4000, [1, 0, 2] * 401),
+    (4 * 64 + 2, 5000, [3] * 128 + [1200] + [3] * 129), (4096, 64, [0] * 4095 + [64]),
+    (16, 16, [16] * 16),
+])
+def test_conversion_tile_edges(dev, m, n, lens):
+    print(f"[conversion tiles] {m} x {n}", flush=True)
+    rng = np.random.default_rng(m + n)
+    I = np.zeros(m + 1, np.int32)
+    I[1:] = np.cumsum(lens)
+    J = np.concatenate([rng.permutation(n)[:k] for k in lens]).astype(np.int32)
+    A = rng.standard_normal(len(J))
+    ref = O.csr2mbsr(m, n, I, J, A)
+    M = make(dev, m, n, I, J, A)
+    inf = M.info()
+    assert inf["nblk"] == ref["nblk"]
+    assert inf["max_row_blocks"] == int(np.diff(ref["blk_ptr"]).max())
+    assert inf["stand"] == pytest.approx(O.mbsr_stats(ref)[0], rel=1e-12, abs=1e-12)
+    check_structure(M, ref)
+    M.update_values(T(I, dev), T(J, dev), T(2.0 * A, dev))
+    assert np.array_equal(M.arrays()["val"].cpu().numpy(), 2.0 * ref["val"])
+
+
 def test_conversion_pattern_only_and_empty(dev):
     (m, n), I, J, A = CASES["rand_rect"]()
     M = make(dev, m, n, I, J, None)
