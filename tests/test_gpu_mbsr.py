@@ -105,6 +105,12 @@ def test_conversion_tile_edges(dev, m, n, lens):
     assert inf["max_row_blocks"] == int(np.diff(ref["blk_ptr"]).max())
     assert inf["stand"] == pytest.approx(O.mbsr_stats(ref)[0], rel=1e-12, abs=1e-12)
     check_structure(M, ref)
+    # the export: ascending columns, values moved exactly
+    S = sp.csr_matrix((A, J, I), shape=(m, n))
+    S.sort_indices()
+    EI, EJ, EV = (t.cpu().numpy() for t in M.to_csr())
+    assert np.array_equal(EI, S.indptr) and np.array_equal(EJ, S.indices)
+    assert np.array_equal(EV, S.data)
     M.update_values(T(I, dev), T(J, dev), T(2.0 * A, dev))
     assert np.array_equal(M.arrays()["val"].cpu().numpy(), 2.0 * ref["val"])
 
