@@ -325,17 +325,30 @@ __device__ __forceinline__ double round_out<double>(double x) {
 // wave takes RPW rows and issues each stage's loads for all of them before
 // it waits.
 //
-// rows / ub_off NULL: the bounded form, every block row 0 .. count-1 with its
-// slot of the temporaries at row * stride, where the host's bound (largest A
-// row times largest B row, at most 64) holds every row's products.  A row
+// rows / ub_off NULL: the bounded form, every block row 0 .. count-1, where the
+// host's bound (stride = largest A row times largest B row, at most 64) holds
+// every row's products.  The workgroup's rows share its part of the temporaries
+// and pack their blocks there, row i from loc[i] on (CSlots): with a slot of
+// `stride` entries per row the ten blocks of an average row cost several cache
+// lines each way.  A row
 // that breaks the bound writes no structure and a block count of -1, which
 // the size pass reports as an error.
 constexpr int kSymRegRows = 2;  // rows per wave of k_symbolic_reg
+constexpr int kSymWgRows = 4 * kSymRegRows;  // rows per workgroup
+
+// Where the symbolic pass left a block row's C blocks: at ub_off[i], or in the
+// bounded form at loc[i] in the part of the row's workgroup.
+struct CSlots {
+    const int64_t *ub_off;
+    uint16_t *loc;
+    int32_t stride;
+    __device__ __forceinline__ int64_t at(int i) const {
+        return ub_off ? ub_off[i] : int64_t(i / kSymRegRows) * kSymRegRows * stride + loc[i];
+    }
+};
 template <int RPW>
 __global__ __launch_bounds__(256) void k_symbolic_reg(int count, const int32_t *__restrict__ rows,
-                                                      SpgemmArgs g,
-                                                      const int64_t *__restrict__ ub_off,
-                                                      int32_t stride, int packed,
+                                                      SpgemmArgs g, CSlots slots, int packed,
                                                       int32_t *__restrict__ tcol,
                                                       uint32_t *__restrict__ tmap,
                                                       int32_t *__restrict__ cnt_out,
@@ -346,6 +359,8 @@ __global__ __launch_bounds__(256) void k_symbolic_reg(int count, const int32_t *
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     const int r0 = (blockIdx.x * 4 + w) * RPW;
     if (r0 >= count) return;  // whole wave; the waves share no LDS
+    const int64_t *const ub_off = slots.ub_off;
+    const int32_t stride = slots.stride;
     int i[RPW], na[RPW], a_beg[RPW];
     bool on[RPW];
 #pragma unroll
@@ -485,11 +500,19 @@ __global__ __launch_bounds__(256) void k_symbolic_reg(int count, const int32_t *
         if (in[u]) atomicOr(&s_cm[w][u][cslot], s_sm[w][u][lane]);
     }
     wave_sync();
+    int at = 0;  // the rows' places in the wave's part
 #pragma unroll
     for (int u = 0; u < RPW; ++u) {
         if (!ok[u]) continue;  // wave-uniform
         const int ncb = __popcll(heads[u]);
-        const int64_t slot = ub_off ? ub_off[i[u]] : int64_t(i[u]) * stride;
+        int64_t slot;
+        if (ub_off) {
+            slot = ub_off[i[u]];
+        } else {
+            if (lane == 0) slots.loc[i[u]] = uint16_t(at);
+            slot = int64_t(r0) * stride + at;
+            at += ncb;
+        }
         const bool head = ((heads[u] >> lane) & 1ull) != 0ull;
         const int cslot = __popcll(heads[u] & ((2ull << lane) - 1ull)) - 1;
         if (head) tcol[slot + cslot] = sk[u];
@@ -625,11 +648,9 @@ __global__ __launch_bounds__(256) void k_upper_bound(int32_t brow, const int32_t
     rowpass::write_part(i < brow, vb, v, 0, kBin1Ub, parts);
 }
 
-// (rows: the block rows to copy, or every row 0 .. count-1 when NULL; ub_off
-// NULL: the row's slot is at row * stride)
+// (rows: the block rows to copy, or every row 0 .. count-1 when NULL)
 __global__ __launch_bounds__(256) void k_compact_c(int32_t count, const int32_t *__restrict__ rows,
-                                                   const int64_t *__restrict__ ub_off,
-                                                   int32_t stride,
+                                                   CSlots slots,
                                                    const int32_t *__restrict__ cptr,
                                                    const int32_t *__restrict__ tcol,
                                                    const uint32_t *__restrict__ tmap,
@@ -639,7 +660,7 @@ __global__ __launch_bounds__(256) void k_compact_c(int32_t count, const int32_t 
     const int r = blockIdx.x * 4 + (threadIdx.x >> 6);
     if (r >= count) return;
     const int i = rows ? rows[r] : r;
-    const int64_t s = ub_off ? ub_off[i] : int64_t(i) * stride;
+    const int64_t s = slots.at(i);
     const int p0 = cptr[i], n = cptr[i + 1] - p0;
     for (int t = lane; t < n; t += 64) {
         ccol[p0 + t] = tcol[s + t];
@@ -1215,8 +1236,7 @@ __global__ __launch_bounds__(256) void k_numeric_outer(int count, const int32_t 
                                                        SpgemmArgs g,
                                                        const int32_t *__restrict__ boff,
                                                        const int32_t *__restrict__ cptr,
-                                                       const int64_t *__restrict__ ub_off,
-                                                       int32_t stride,
+                                                       CSlots slots,
                                                        const int32_t *__restrict__ tcol,
                                                        const uint32_t *__restrict__ tmap,
                                                        int32_t *__restrict__ ccol,
@@ -1234,7 +1254,7 @@ __global__ __launch_bounds__(256) void k_numeric_outer(int count, const int32_t 
     // the row's scalars first, all in flight together (wave-uniform: scalar loads)
     const int i = __builtin_amdgcn_readfirstlane(rows ? rows[r] : r);
     const int c0 = cptr[i], cnt = cptr[i + 1] - c0;  // cnt <= min(64, CAPB): the bin's rule
-    const int64_t so = ub_off ? ub_off[i] : int64_t(i) * stride;
+    const int64_t so = slots.at(i);
     const int a_beg = g.ap[i], na = g.ap[i + 1] - a_beg;
     const int avp0 = g.avp[i];
     const int vbase = cvp[i];
@@ -1383,6 +1403,214 @@ __global__ __launch_bounds__(256) void k_numeric_outer(int count, const int32_t 
     }
 }
 
+// The register bin in FP64 for short rows of sparse blocks: row by row over the
+// scalar entries.  G = 4 L lanes own a C block row, L of them each of its four
+// rows.  A row takes its A entries in order (A block j, column n); lane l holds
+// the l-th block of B's block row j and adds a times the block's row n into the
+// C row's entries, which sit compressed in LDS.  Within a step the lanes of a
+// row hold different B blocks, so different C blocks, and the rows are
+// different: no two lanes add to one entry, and every entry sums its products
+// in the order of A's columns (deterministic, no atomics).
+// The MFMA form (k_numeric_outer) multiplies whole 4x4 blocks: at the fill of
+// stencil and interpolation operators (1/4 and less) 1 of 16 to 1 of 64 of its
+// products exist, and it is bound by the VALU work of gathering padded operands
+// (550 instructions per row of A P on 7-pt 128^3, one row per wave).  Here only
+// existing products are formed and 2 or 4 rows share a wave (235 instructions
+// per row); it waits on the chain row pointers -> A blocks -> B rows -> B blocks
+// -> values, so LDS per row (waves per CU) and loads in flight count: 566 us
+// (MFMA) -> 544 with one value load at a time, 500 with four A blocks' loads
+// together, 385 with packed C blocks and 12-byte records.
+// rec, rc: one record per (A block, B block) product of the row.
+constexpr int kRowsA = 16;     // A blocks per row
+constexpr int kRowsAv = 32;    // A values staged in LDS
+// PR: products per row, CAPV: values per C row
+template <int L, int PR, int CAPV>
+__global__ __launch_bounds__(256) void k_numeric_rows(int count, const int32_t *__restrict__ rows,
+                                                      SpgemmArgs g,
+                                                      const int32_t *__restrict__ boff,
+                                                      const int32_t *__restrict__ cptr,
+                                                      CSlots slots,
+                                                      const int32_t *__restrict__ tcol,
+                                                      const uint32_t *__restrict__ tmap,
+                                                      int32_t *__restrict__ ccol,
+                                                      uint16_t *__restrict__ cmap,
+                                                      const int32_t *__restrict__ cvp,
+                                                      double *__restrict__ cval) {
+    constexpr int G = 4 * L, NR = 256 / G;
+    struct Row {
+        double acc[CAPV];            // first (block column, bitmap | first entry << 16) per C block
+        double av[kRowsAv];
+        int2 rec[PR];                // B bitmap | C bitmap << 16, B value offset
+        uint8_t rc[PR];              // first entry of the C block
+        int4 pad;                    // rows start four banks apart
+        int4 ab[kRowsA];             // bitmap | B blocks << 16, first value, first product, first B block
+    };
+    __shared__ Row s_row[NR];
+    const double *__restrict__ aval = static_cast<const double *>(g.av);
+    const double *__restrict__ bval = static_cast<const double *>(g.bv);
+    const int grp = threadIdx.x / G, gl = threadIdx.x % G;
+    const int rr = blockIdx.x * NR + grp;
+    const bool on = rr < count;
+    if (!__ballot(on)) return;  // whole wave; the waves share no LDS
+    Row &s = s_row[grp];
+    int2 *const ck = reinterpret_cast<int2 *>(s.acc);
+    const int i = on ? (rows ? rows[rr] : rr) : 0;
+    const int a_beg = g.ap[i], na = on ? g.ap[i + 1] - a_beg : 0;
+    const int c0 = cptr[i], cnt = on ? cptr[i + 1] - c0 : 0;
+    const int av0 = g.avp[i], nv = on ? g.avp[i + 1] - av0 : 0;
+    const int v0 = cvp[i], nent = on ? cvp[i + 1] - v0 : 0;
+    const int64_t so = slots.at(i);
+    // A blocks, one per lane (na <= kRowsA <= G)
+    int ma = 0, bq0 = 0, blen = 0;
+    if (gl < na) {
+        const int k = g.ac[a_beg + gl];
+        ma = g.am[a_beg + gl];
+        bq0 = g.bp[k];
+        blen = g.bp[k + 1] - bq0;
+    }
+    for (int t = gl; t < min(nv, kRowsAv); t += G) s.av[t] = aval[av0 + t];
+    // C's blocks out of the symbolic temporaries
+    for (int t0 = 0, run = 0; t0 < cnt; t0 += G) {
+        const int t = t0 + gl;
+        int key = 0;
+        uint32_t cm = 0;
+        if (t < cnt) {
+            key = tcol[so + t];
+            cm = tmap[so + t];
+            ccol[c0 + t] = key;
+            cmap[c0 + t] = uint16_t(cm);
+        }
+        int inc = __popc(cm);
+#pragma unroll
+        for (int d = 1; d < G; d <<= 1) {
+            const int v = __shfl_up(inc, d, G);
+            if (gl >= d) inc += v;
+        }
+        if (t < cnt) ck[t] = make_int2(key, int(cm | uint32_t(run + inc - __popc(cm)) << 16));
+        run += __shfl(inc, G - 1, G);
+    }
+    int sums = __popc(uint32_t(ma)) | blen << 16;  // values and products before, in one scan
+    const int own = sums;
+#pragma unroll
+    for (int d = 1; d < kRowsA; d <<= 1) {
+        const int v = __shfl_up(sums, d, G);
+        if (gl >= d) sums += v;
+    }
+    const int ptot = __shfl(sums, na > 0 ? na - 1 : 0, G) >> 16;
+    sums -= own;
+    if (gl < na) s.ab[gl] = make_int4(ma | blen << 16, sums & 0xFFFF, sums >> 16, bq0);
+    wave_sync();
+    // the products' records
+    for (int t = gl; t < ptot; t += G) {
+        int j = 0;
+#pragma unroll
+        for (int step = kRowsA / 2; step >= 1; step >>= 1)
+            if (j + step < na && s.ab[j + step].z <= t) j += step;
+        const int4 ab = s.ab[j];
+        const int q = ab.w + (t - ab.z);
+        const int mb = g.bm[q], bo = boff[q], col = g.bc[q];
+        int lo = 0, n = cnt;
+        while (n > 0) {
+            const int h = n >> 1;
+            if (ck[lo + h].x < col) {
+                lo += h + 1;
+                n -= h + 1;
+            } else {
+                n = h;
+            }
+        }
+        // (a product without entries may have no C block: its record is never used)
+        const uint32_t c = lo < cnt ? uint32_t(ck[lo].y) : 0u;
+        s.rec[t] = make_int2(mb | int(c << 16), bo);
+        s.rc[t] = uint8_t(c >> 16);
+    }
+    wave_sync();
+    for (int t = gl; t < nent; t += G) s.acc[t] = 0.0;
+    wave_sync();
+    const int r = gl / L, l = gl % L;
+    int jmax = na;
+#pragma unroll
+    for (int d = G; d < 64; d <<= 1) jmax = max(jmax, __shfl_xor(jmax, d));
+    auto a_at = [&](uint32_t xa, int a0, int n) {
+        const int ia = a0 + __popc(xa & ((1u << (4 * r + n)) - 1u));
+        return ia < kRowsAv ? s.av[ia] : aval[av0 + ia];
+    };
+    auto b_index = [&](const int2 &rec, int n, uint32_t bn) {
+        return rec.y + __popc(uint32_t(rec.x) & ((1u << (4 * n + __builtin_ctz(bn))) - 1u));
+    };
+    auto add = [&](const int2 &rec, int rc, uint32_t bn, double a, double b) {
+        const int to = rc + __popc((uint32_t(rec.x) >> 16) & ((1u << (4 * r + __builtin_ctz(bn))) - 1u));
+        s.acc[to] = fma(a, b, s.acc[to]);
+    };
+    // a times the entries bn of row n of a B block
+    auto add_row = [&](const int2 &rec, int rc, int n, uint32_t bn, double a) {
+        for (; bn; bn &= bn - 1u) add(rec, rc, bn, a, bval[b_index(rec, n, bn)]);
+    };
+    // four A blocks at a time: the first two B values each will need are loaded
+    // together (a row rarely has a second entry in an A block or a third in a
+    // B block row), so that their latency is paid once per four blocks
+    constexpr int JB = 4;
+    for (int j0 = 0; j0 < jmax; j0 += JB) {
+        double b0[JB], b1[JB];
+#pragma unroll
+        for (int u = 0; u < JB; ++u) {
+            int i0 = 0, i1 = 0;
+            if (j0 + u < na) {
+                const int4 ab = s.ab[j0 + u];
+                const uint32_t nib = (uint32_t(ab.x) >> (4 * r)) & 0xFu;
+                if (l < (ab.x >> 16) && nib) {
+                    const int2 rec = s.rec[ab.z + l];
+                    const int n = __builtin_ctz(nib);
+                    uint32_t bn = (uint32_t(rec.x) >> (4 * n)) & 0xFu;
+                    if (bn) i0 = b_index(rec, n, bn);
+                    bn &= bn - 1u;
+                    if (bn) i1 = b_index(rec, n, bn);
+                }
+            }
+            b0[u] = bval[i0];  // (value 0 where there is none: not used)
+            b1[u] = bval[i1];
+        }
+#pragma unroll
+        for (int u = 0; u < JB; ++u) {
+            if (j0 + u < na) {
+                const int4 ab = s.ab[j0 + u];
+                const uint32_t xa = uint32_t(ab.x) & 0xFFFFu;
+                uint32_t nib = (xa >> (4 * r)) & 0xFu;
+                const int bl = ab.x >> 16;
+                if (l < bl && nib) {
+                    const int2 rec = s.rec[ab.z + l];
+                    const int rc = s.rc[ab.z + l];
+                    const int n = __builtin_ctz(nib);
+                    const double a = a_at(xa, ab.y, n);
+                    uint32_t bn = (uint32_t(rec.x) >> (4 * n)) & 0xFu;
+                    if (bn) {
+                        add(rec, rc, bn, a, b0[u]);
+                        bn &= bn - 1u;
+                        if (bn) {
+                            add(rec, rc, bn, a, b1[u]);
+                            add_row(rec, rc, n, bn & (bn - 1u), a);
+                        }
+                    }
+                    for (nib &= nib - 1u; nib; nib &= nib - 1u) {
+                        const int m = __builtin_ctz(nib);
+                        add_row(rec, rc, m, (uint32_t(rec.x) >> (4 * m)) & 0xFu, a_at(xa, ab.y, m));
+                    }
+                }
+                for (int q = l + L; q < bl; q += L) {
+                    const int2 rec = s.rec[ab.z + q];
+                    const int rc = s.rc[ab.z + q];
+                    for (nib = (xa >> (4 * r)) & 0xFu; nib; nib &= nib - 1u) {
+                        const int m = __builtin_ctz(nib);
+                        add_row(rec, rc, m, (uint32_t(rec.x) >> (4 * m)) & 0xFu, a_at(xa, ab.y, m));
+                    }
+                }
+            }
+            wave_sync();  // a C entry's next product may come from another lane
+        }
+    }
+    for (int t = gl; t < nent; t += G) cval[v0 + t] = s.acc[t];
+}
+
 // The register bin for FP32 / FP16 operands: the product and slot assignment
 // of k_numeric_outer's prologue; the 16-block MFMAs (FP32 accumulation)
 // take 16 C blocks at a time: lane 4b + r works for C block g0 + b, gathers
@@ -1529,14 +1757,15 @@ struct CSizePart {
     int32_t f[5];  // blocks, values, rows per numeric bin; after k_csize_finish: offsets
     int32_t mx;    // largest block count
     int32_t bad;   // a row that broke the register bound (block count -1)
-    int32_t big[3];  // largest values of a bin-1 row, blocks and values of a bin-2 row
+    int32_t big[4];  // largest values of a bin-1 row, blocks and values of a bin-2 row,
+                     // values of a bin-0 row
     unsigned long long sumsq;
 };
 
 struct CSizeTotals {
     RowStats rs;  // rows per numeric bin, largest block count, sum of squares
     int32_t nblk, nnz, bad;
-    int32_t big[3];  // as CSizePart: which numeric launches have rows
+    int32_t big[4];  // as CSizePart: which numeric launches have rows
 };
 
 template <typename FB>
@@ -1544,7 +1773,7 @@ __global__ __launch_bounds__(256) void k_csize_part(int32_t n, FB fb,
                                                     const int32_t *__restrict__ ccnt,
                                                     const int32_t *__restrict__ cnnz,
                                                     CSizePart *__restrict__ parts) {
-    __shared__ int s_f[4][10];
+    __shared__ int s_f[4][11];
     __shared__ unsigned long long s_sq[4];
     const int i = blockIdx.x * 256 + threadIdx.x;
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
@@ -1557,6 +1786,7 @@ __global__ __launch_bounds__(256) void k_csize_part(int32_t n, FB fb,
     const int v1 = __builtin_amdgcn_readlane(wave_incl_max(b == 1 ? v : 0), 63);
     const int b2 = __builtin_amdgcn_readlane(wave_incl_max(b == 2 ? c : 0), 63);
     const int v2 = __builtin_amdgcn_readlane(wave_incl_max(b == 2 ? v : 0), 63);
+    const int v0 = __builtin_amdgcn_readlane(wave_incl_max(b == 0 ? v : 0), 63);
     const bool bad = __ballot(c < 0) != 0ull;
     int nb[3];
 #pragma unroll
@@ -1574,6 +1804,7 @@ __global__ __launch_bounds__(256) void k_csize_part(int32_t n, FB fb,
         s_f[w][7] = v1;
         s_f[w][8] = b2;
         s_f[w][9] = v2;
+        s_f[w][10] = v0;
         s_sq[w] = sq;
     }
     __syncthreads();
@@ -1584,7 +1815,7 @@ __global__ __launch_bounds__(256) void k_csize_part(int32_t n, FB fb,
         p.mx = max(max(s_f[0][5], s_f[1][5]), max(s_f[2][5], s_f[3][5]));
         p.bad = s_f[0][6] | s_f[1][6] | s_f[2][6] | s_f[3][6];
 #pragma unroll
-        for (int q = 0; q < 3; ++q)
+        for (int q = 0; q < 4; ++q)
             p.big[q] = max(max(s_f[0][7 + q], s_f[1][7 + q]), max(s_f[2][7 + q], s_f[3][7 + q]));
         p.sumsq = s_sq[0] + s_sq[1] + s_sq[2] + s_sq[3];
         parts[blockIdx.x] = p;
@@ -1598,11 +1829,11 @@ __global__ __launch_bounds__(rowpass::kFinishThreads) void k_csize_finish(
     int32_t *__restrict__ cptr_end, int32_t *__restrict__ cvp_end) {
     constexpr int NT = rowpass::kFinishThreads, NW = NT / 64;
     __shared__ int s_w[NW][5];
-    __shared__ int s_mx[NW][4], s_bad[NW];
+    __shared__ int s_mx[NW][5], s_bad[NW];
     __shared__ unsigned long long s_sq[NW];
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     int run[5] = {0, 0, 0, 0, 0};
-    int mx[4] = {0, 0, 0, 0}, bad = 0;
+    int mx[5] = {0, 0, 0, 0, 0}, bad = 0;
     unsigned long long sq = 0ull;
     for (int base = 0; base < ng; base += NT) {
         const int gi = base + threadIdx.x;
@@ -1634,7 +1865,7 @@ __global__ __launch_bounds__(rowpass::kFinishThreads) void k_csize_finish(
             for (int q = 0; q < 5; ++q) parts[gi].f[q] = off[q];
             mx[0] = max(mx[0], p.mx);
 #pragma unroll
-            for (int q = 0; q < 3; ++q) mx[1 + q] = max(mx[1 + q], p.big[q]);
+            for (int q = 0; q < 4; ++q) mx[1 + q] = max(mx[1 + q], p.big[q]);
             bad |= p.bad;
             sq += p.sumsq;
         }
@@ -1643,23 +1874,23 @@ __global__ __launch_bounds__(rowpass::kFinishThreads) void k_csize_finish(
     }
     for (int o = 32; o > 0; o >>= 1) {
 #pragma unroll
-        for (int q = 0; q < 4; ++q) mx[q] = max(mx[q], __shfl_xor(mx[q], o));
+        for (int q = 0; q < 5; ++q) mx[q] = max(mx[q], __shfl_xor(mx[q], o));
         bad |= __shfl_xor(bad, o);
         sq += __shfl_xor(sq, o);
     }
     if (lane == 0) {
 #pragma unroll
-        for (int q = 0; q < 4; ++q) s_mx[w][q] = mx[q];
+        for (int q = 0; q < 5; ++q) s_mx[w][q] = mx[q];
         s_bad[w] = bad;
         s_sq[w] = sq;
     }
     __syncthreads();
     if (threadIdx.x == 0) {
-        int m[4] = {0, 0, 0, 0}, b = 0;
+        int m[5] = {0, 0, 0, 0, 0}, b = 0;
         unsigned long long t = 0ull;
         for (int k = 0; k < NW; ++k) {
 #pragma unroll
-            for (int q = 0; q < 4; ++q) m[q] = max(m[q], s_mx[k][q]);
+            for (int q = 0; q < 5; ++q) m[q] = max(m[q], s_mx[k][q]);
             b |= s_bad[k];
             t += s_sq[k];
         }
@@ -1670,6 +1901,7 @@ __global__ __launch_bounds__(rowpass::kFinishThreads) void k_csize_finish(
         tot->big[0] = m[1];
         tot->big[1] = m[2];
         tot->big[2] = m[3];
+        tot->big[3] = m[4];
         tot->rs.sumsq = t;
         tot->nblk = run[0];
         tot->nnz = run[1];
@@ -1777,31 +2009,65 @@ __global__ __launch_bounds__(256) void k_scale_values(int64_t n, double f, doubl
     if (i < n) v[i] *= f;
 }
 
+// Lanes per row of k_numeric_rows for this product, 0 where k_numeric_outer
+// runs instead: rows of more than 16 A blocks or 256 C values, which the row's
+// LDS does not hold, and denser blocks (over 6 of 16 entries), where most of
+// the MFMA's products exist and its one instruction per four blocks wins.
+// Measured at 2 to 4 entries per block: A P of 7-pt 128^3 with trilinear P 385
+// against 566 us, with a PMIS-like P on 101 x 99 x 97 267 against 354 us.  B's
+// block rows of at most 4 blocks on average leave half of eight lanes idle.
+int numeric_rows_lanes(const Mbsr &A, const Mbsr &B, int32_t max_values) {
+    if (A.max_row_blocks > kRowsA || max_values > 256 || A.nblk == 0 || B.nblk == 0) return 0;
+    if (A.avg_nnz > 6.0 || B.avg_nnz > 6.0) return 0;
+    return B.nblk <= 4 * int64_t(B.brow) ? 4 : 8;
+}
+
 // numeric kernels of one value precision; *nslab receives the global slab of
 // the rows over kNumCap blocks (freed by the caller)
 // The FP64 register-bin kernel also copies its rows' block columns and
-// bitmaps from the symbolic temporaries (ub_off, tcol, tmap) to C; the other
+// bitmaps from the symbolic temporaries (slots, tcol, tmap) to C; the other
 // kernels read them from C.
 template <typename VT>
-int launch_numeric(const SpgemmArgs &g, const int32_t *boff, const Mbsr &C, int32_t brow,
+int launch_numeric(const SpgemmArgs &g, const Mbsr &A, const Mbsr &B, const int32_t *boff,
+                   const Mbsr &C, int32_t brow,
                    const int32_t *list, int32_t reg_rows, int32_t lds_rows, int32_t big_rows,
-                   const int64_t *ub_off, int32_t stride, const int32_t *tcol,
-                   const uint32_t *tmap, const int32_t *big, double **nslab, hipStream_t s) {
+                   const CSlots &slots, const int32_t *tcol, const uint32_t *tmap,
+                   const int32_t *big, double **nslab, hipStream_t s) {
     if (reg_rows > 0) {
         if constexpr (std::is_same<VT, double>::value) {
             // accumulators for the bin's longest C row (at most 64 blocks)
             const dim3 grid((reg_rows + 3) / 4);
-            if (C.max_row_blocks <= 16)
+            const int rows_l = numeric_rows_lanes(A, B, big[3]);
+            if (rows_l > 0) {
+                const int per = 256 / (4 * rows_l);
+                const dim3 rgrid((reg_rows + per - 1) / per);
+#define AMGT_NUMERIC_ROWS(L_, P_, V_)                                                          \
+    hipLaunchKernelGGL((k_numeric_rows<L_, P_, V_>), rgrid, dim3(256), 0, s, reg_rows, list,   \
+                       g, boff, C.blk_ptr, slots, tcol, tmap, C.blk_col, C.blk_map,   \
+                       C.val_ptr, C.val)
+#define AMGT_NUMERIC_ROWS_V(L_, P_)                       \
+    do {                                                  \
+        if (big[3] <= 64) AMGT_NUMERIC_ROWS(L_, P_, 64);  \
+        else if (big[3] <= 128) AMGT_NUMERIC_ROWS(L_, P_, 128); \
+        else AMGT_NUMERIC_ROWS(L_, P_, 256);              \
+    } while (0)
+                // (bounded form: at most stride products per row)
+                if (rows_l == 4 && !slots.ub_off && slots.stride <= 32) AMGT_NUMERIC_ROWS_V(4, 32);
+                else if (rows_l == 4) AMGT_NUMERIC_ROWS_V(4, 64);
+                else AMGT_NUMERIC_ROWS_V(8, 64);
+#undef AMGT_NUMERIC_ROWS_V
+#undef AMGT_NUMERIC_ROWS
+            } else if (C.max_row_blocks <= 16)
                 hipLaunchKernelGGL((k_numeric_outer<16>), grid, dim3(256), 0, s, reg_rows, list,
-                                   g, boff, C.blk_ptr, ub_off, stride, tcol, tmap, C.blk_col,
+                                   g, boff, C.blk_ptr, slots, tcol, tmap, C.blk_col,
                                    C.blk_map, C.val_ptr, C.val);
             else if (C.max_row_blocks <= 32)
                 hipLaunchKernelGGL((k_numeric_outer<32>), grid, dim3(256), 0, s, reg_rows, list,
-                                   g, boff, C.blk_ptr, ub_off, stride, tcol, tmap, C.blk_col,
+                                   g, boff, C.blk_ptr, slots, tcol, tmap, C.blk_col,
                                    C.blk_map, C.val_ptr, C.val);
             else
                 hipLaunchKernelGGL((k_numeric_outer<64>), grid, dim3(256), 0, s, reg_rows, list,
-                                   g, boff, C.blk_ptr, ub_off, stride, tcol, tmap, C.blk_col,
+                                   g, boff, C.blk_ptr, slots, tcol, tmap, C.blk_col,
                                    C.blk_map, C.val_ptr, C.val);
         } else
             hipLaunchKernelGGL((k_numeric_reg16<VT>), dim3((reg_rows + 3) / 4), dim3(256), 0, s,
@@ -1905,6 +2171,7 @@ int spgemm(const Mbsr &A, const Mbsr &B, int precision, hipStream_t s, Mbsr *Cp)
     int32_t *retry = nullptr;
     double *nslab = nullptr;
     int32_t *bpop = nullptr, *boff = nullptr;
+    uint16_t *loc = nullptr;
     int st = AMGT_OK;
     auto cleanup = [&]() {
         tmp_free(parts, s);
@@ -1923,6 +2190,7 @@ int spgemm(const Mbsr &A, const Mbsr &B, int precision, hipStream_t s, Mbsr *Cp)
         tmp_free(nslab, s);
         tmp_free(bpop, s);
         tmp_free(boff, s);
+        tmp_free(loc, s);
     };
 #define SG_TRY(expr)               \
     do {                           \
@@ -1947,10 +2215,11 @@ int spgemm(const Mbsr &A, const Mbsr &B, int precision, hipStream_t s, Mbsr *Cp)
     SG_TRY(tmp_alloc_t(&list, size_t(brow) * 3 + 1, s));
     SG_TRY(tmp_alloc_t(&ccnt, size_t(brow) + 1, s));
     SG_TRY(tmp_alloc_t(&cnnz, size_t(brow) + 1, s));
+    if (bounded) SG_TRY(tmp_alloc_t(&loc, size_t(brow), s));
     int64_t total_ub = 0;
     const int32_t *bin = ht.cnt;
     if (bounded) {
-        total_ub = int64_t(brow) * stride;
+        total_ub = (int64_t(brow) + kSymWgRows) * stride;  // whole workgroups
     } else {
         SG_TRY(tmp_alloc_t(&parts, size_t(rowpass::groups(brow)) + 1, s));
         SG_TRY(tmp_alloc_t(&tots, 1, s));
@@ -1971,6 +2240,7 @@ int spgemm(const Mbsr &A, const Mbsr &B, int precision, hipStream_t s, Mbsr *Cp)
                                 {&ht, tots, sizeof(RowStats)}};
         SG_TRY(readback(rb, 2, s));
     }
+    const CSlots slots{ub_off, loc, stride};
     SG_TRY(tmp_alloc_t(&tcol, size_t(total_ub), s));
     SG_TRY(tmp_alloc_t(&tmap, size_t(total_ub), s));
     if (!C.pattern_only && brow > 0) {
@@ -1991,16 +2261,14 @@ int spgemm(const Mbsr &A, const Mbsr &B, int precision, hipStream_t s, Mbsr *Cp)
         }
         SG_HIP(hipGetLastError());
     }
-    constexpr int kSymRows = 4 * kSymRegRows;  // rows per workgroup of k_symbolic_reg
     if (bounded)
-        hipLaunchKernelGGL((k_symbolic_reg<kSymRegRows>), dim3((brow + kSymRows - 1) / kSymRows),
+        hipLaunchKernelGGL((k_symbolic_reg<kSymRegRows>), dim3((brow + kSymWgRows - 1) / kSymWgRows),
                            dim3(256), 0, s, brow, static_cast<const int32_t *>(nullptr), g,
-                           static_cast<const int64_t *>(nullptr), stride, packed, tcol, tmap,
-                           ccnt, cnnz);
+                           slots, packed, tcol, tmap, ccnt, cnnz);
     if (!bounded && bin[0] > 0)
         hipLaunchKernelGGL((k_symbolic_reg<kSymRegRows>),
-                           dim3((bin[0] + kSymRows - 1) / kSymRows), dim3(256), 0, s, bin[0],
-                           list, g, ub_off, 0, packed, tcol, tmap, ccnt, cnnz);
+                           dim3((bin[0] + kSymWgRows - 1) / kSymWgRows), dim3(256), 0, s, bin[0],
+                           list, g, slots, packed, tcol, tmap, ccnt, cnnz);
     if (!bounded && bin[1] > 0) {
         hipLaunchKernelGGL(k_symbolic_wave, dim3((bin[1] + 3) / 4), dim3(256), 0, s, bin[1],
                            list + brow, g, ub_off, tcol, tmap, ccnt, cnnz);
@@ -2099,31 +2367,31 @@ int spgemm(const Mbsr &A, const Mbsr &B, int precision, hipStream_t s, Mbsr *Cp)
     const bool fp64_numeric = !C.pattern_only && precision != AMGT_FLOAT && precision != AMGT_HALF;
     if (brow > 0 && !fp64_numeric)
         hipLaunchKernelGGL(k_compact_c, dim3((brow + 3) / 4), dim3(256), 0, s, brow,
-                           static_cast<const int32_t *>(nullptr), ub_off, stride, C.blk_ptr, tcol,
+                           static_cast<const int32_t *>(nullptr), slots, C.blk_ptr, tcol,
                            tmap, C.blk_col, C.blk_map);
     if (fp64_numeric && lds_rows > 0)
         hipLaunchKernelGGL(k_compact_c, dim3((lds_rows + 3) / 4), dim3(256), 0, s, lds_rows,
-                           list + brow, ub_off, stride, C.blk_ptr, tcol, tmap, C.blk_col,
+                           list + brow, slots, C.blk_ptr, tcol, tmap, C.blk_col,
                            C.blk_map);
     if (fp64_numeric && big_rows > 0)
         hipLaunchKernelGGL(k_compact_c, dim3((big_rows + 3) / 4), dim3(256), 0, s, big_rows,
-                           list + 2 * int64_t(brow), ub_off, stride, C.blk_ptr, tcol, tmap,
+                           list + 2 * int64_t(brow), slots, C.blk_ptr, tcol, tmap,
                            C.blk_col, C.blk_map);
     SG_HIP(hipGetLastError());
     if (!C.pattern_only && brow > 0) {
         switch (precision) {
             case AMGT_FLOAT:
-                st = launch_numeric<float>(g, boff, C, brow, list, reg_rows, lds_rows, big_rows, ub_off, stride, tcol, tmap, ct.big, &nslab, s);
+                st = launch_numeric<float>(g, A, B, boff, C, brow, list, reg_rows, lds_rows, big_rows, slots, tcol, tmap, ct.big, &nslab, s);
                 break;
             case AMGT_HALF:
-                st = launch_numeric<__half>(g, boff, C, brow, list, reg_rows, lds_rows, big_rows, ub_off, stride, tcol, tmap, ct.big, &nslab, s);
+                st = launch_numeric<__half>(g, A, B, boff, C, brow, list, reg_rows, lds_rows, big_rows, slots, tcol, tmap, ct.big, &nslab, s);
                 // the FP16 copies hold A and B times half_scale: undo both (powers of two, exact)
                 if (st == AMGT_OK && C.nnz > 0)
                     hipLaunchKernelGGL(k_scale_values, dim3(unsigned((C.nnz + 255) / 256)), dim3(256),
                                        0, s, C.nnz, 1.0 / (A.half_scale * B.half_scale), C.val);
                 break;
             default:
-                st = launch_numeric<double>(g, boff, C, brow, list, reg_rows, lds_rows, big_rows, ub_off, stride, tcol, tmap, ct.big, &nslab, s);
+                st = launch_numeric<double>(g, A, B, boff, C, brow, list, reg_rows, lds_rows, big_rows, slots, tcol, tmap, ct.big, &nslab, s);
         }
         if (st != AMGT_OK) {
             cleanup();
