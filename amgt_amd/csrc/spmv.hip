@@ -1034,12 +1034,43 @@ __global__ __launch_bounds__(256) void k_spmm(
 // across the lanes first, and the operands of U = 4 blocks are gathered before
 // their MFMAs.  Operand layout (measured on gfx950, block slot b): A_b[i][k] in
 // lane 16k+4b+i, B_b[k][n] in lane 16k+4b+n, D_b[i][n] in lane 16i+4b+n.
-// Multivectors are interleaved (HYPRE multivector storage
-// method 1): entry (row i, vector v) at x[i * kx + v], so the B operand of one
-// instruction is four rows x 16 consecutive right-hand sides (four 128-byte
-// lines) instead of 16 separate 32-byte pieces of column-major vectors.
-// Writes y[row * ky + v] = alpha (A x)[row][v] + beta b[row * kb + v].
-template <int NG, typename VT>
+// X is interleaved (HYPRE multivector storage method 1): entry (row i, vector
+// v) at x[i * kx + v], so the B operand of one instruction is four rows x 16
+// consecutive right-hand sides (four 128-byte lines) instead of 16 separate
+// 32-byte pieces of column-major vectors.  The kernel is bound by these reads
+// out of L2 (27-pt 64^3, k = 32: 27 blocks a row, 1.7 GB): a block's X row is
+// read only if its bitmap has an entry in that column (the outer blocks of a
+// stencil's lines use one of four), by buffer loads whose range check gives 0
+// for the rest, from scalar block data (no per-lane address work).
+// Writes alpha (A x) + beta b: interleaved at y[row * ky + v] (b alike with
+// kb), or (kCm) column-major at y[v * ky + row] through an LDS transpose of the
+// workgroup's 16 rows, which replaces a pass over an interleaved result.
+// MFMA operands from a buffer: 0 past its end
+template <typename VT>
+__device__ __forceinline__ double buf_value(__amdgpu_buffer_rsrc_t rs, uint32_t off);
+template <>
+__device__ __forceinline__ double buf_value<double>(__amdgpu_buffer_rsrc_t rs, uint32_t off) {
+    const auto q = __builtin_amdgcn_raw_buffer_load_b64(rs, off, 0, 0);
+    double v;
+    __builtin_memcpy(&v, &q, 8);
+    return v;
+}
+template <>
+__device__ __forceinline__ double buf_value<float>(__amdgpu_buffer_rsrc_t rs, uint32_t off) {
+    const auto q = __builtin_amdgcn_raw_buffer_load_b32(rs, off, 0, 0);
+    float v;
+    __builtin_memcpy(&v, &q, 4);
+    return double(v);
+}
+template <>
+__device__ __forceinline__ double buf_value<__half>(__amdgpu_buffer_rsrc_t rs, uint32_t off) {
+    const auto q = __builtin_amdgcn_raw_buffer_load_b16(rs, off, 0, 0);
+    __half v;
+    __builtin_memcpy(&v, &q, 2);
+    return double(__half2float(v));
+}
+
+template <int NG, typename VT, bool kCm>
 __global__ __launch_bounds__(256) void k_spmm_mfma_il(
     int32_t brow, int32_t nrows, int32_t ncols, const int32_t *__restrict__ blk_ptr,
     const int32_t *__restrict__ blk_col, const uint16_t *__restrict__ blk_map,
@@ -1047,76 +1078,98 @@ __global__ __launch_bounds__(256) void k_spmm_mfma_il(
     const double *__restrict__ x, int64_t kx, double alpha, double beta, const double *b,
     int64_t kb, double *y, int64_t ky) {
     constexpr int U = 4;
-    const int lane = threadIdx.x & 63;
-    const int br = remap_wg(blockIdx.x, gridDim.x) * 4 + (threadIdx.x >> 6);
-    if (br >= brow) return;  // whole wave
+    constexpr uint32_t kOut = 0xFFFFFFF0u;  // past every buffer: reads 0
+    __shared__ double s_y[kCm ? 16 * NG : 1][17];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int br0 = remap_wg(blockIdx.x, gridDim.x) * 4;
+    const int br = __builtin_amdgcn_readfirstlane(br0 + w);
+    if (!kCm && br >= brow) return;  // whole wave
     const int kk = lane >> 4, bs = (lane >> 2) & 3, nn = lane & 3;
     const int eA = 4 * nn + kk;
     const uint32_t belowA = (1u << eA) - 1u;
-    const int p0 = blk_ptr[br], p1 = blk_ptr[br + 1];
-    int vrel[NG];
-    bool xon[NG];
+    double acc[NG];
+    uint32_t xoff[NG];  // within a block's four X rows
 #pragma unroll
     for (int g = 0; g < NG; ++g) {
+        acc[g] = 0.0;
         const int rhs = 16 * g + 4 * bs + nn;
-        xon[g] = rhs < kn;
-        vrel[g] = k0 + (xon[g] ? rhs : 0);
+        xoff[g] = rhs < kn ? uint32_t(kk * kx + k0 + rhs) * 8u : kOut;
     }
-    double acc[NG];
-#pragma unroll
-    for (int g = 0; g < NG; ++g) acc[g] = 0.0;
-    int voff = val_ptr[br];
-    for (int c0 = p0; c0 < p1; c0 += 64) {
-        const int nb = min(64, p1 - c0);
-        uint32_t mj = 0u;
-        int cj = 0;
-        if (lane < nb) {
-            mj = blk_map[c0 + lane];
-            cj = blk_col[c0 + lane];
-        }
-        int inc = __popc(mj);
-#pragma unroll
-        for (int d = 1; d < 64; d <<= 1) {
-            const int t = __shfl_up(inc, d);
-            if (lane >= d) inc += t;
-        }
-        const int oj = voff + inc - __popc(mj);
-        voff += __shfl(inc, 63);
-        for (int j0 = 0; j0 < nb; j0 += U) {
-            double a[U], bx[U][NG];
-#pragma unroll
-            for (int u = 0; u < U; ++u) {
-                const int j = j0 + u < nb ? j0 + u : nb - 1;
-                const uint32_t m = uint32_t(__shfl(int(mj), j));
-                const int xrow = 4 * __shfl(cj, j) + kk;
-                const int o = __shfl(oj, j);
-                const bool on = j0 + u < nb;
-                a[u] = (on && ((m >> eA) & 1u)) ? double(val[o + __popc(m & belowA)]) : 0.0;
-#pragma unroll
-                for (int g = 0; g < NG; ++g)
-                    bx[u][g] = (on && xon[g] && xrow < ncols) ? x[int64_t(xrow) * kx + vrel[g]] : 0.0;
+    if (br < brow) {
+        const int p0 = blk_ptr[br], p1 = blk_ptr[br + 1];
+        // the row's values from an even index on (a resource starts at 4 bytes)
+        const int odd = val_ptr[br] & 1, v0 = val_ptr[br] - odd, nv = val_ptr[br + 1] - v0;
+        const __amdgpu_buffer_rsrc_t a_rs = __builtin_amdgcn_make_buffer_rsrc(
+            const_cast<VT *>(val + v0), short(0), nv * int(sizeof(VT)), kBufferDword3);
+        int run = odd;
+        for (int c0 = p0; c0 < p1; c0 += 64) {
+            const int nb = min(64, p1 - c0);
+            uint32_t mj = 0u;
+            int cj = 0;
+            if (lane < nb) {
+                mj = blk_map[c0 + lane];
+                cj = blk_col[c0 + lane];
             }
+            const int inc = wave_incl_sum(__popc(mj));
+            const int oj = run + inc - __popc(mj);
+            run += __builtin_amdgcn_readlane(inc, 63);
+            for (int j0 = 0; j0 < nb; j0 += U) {
+                double a[U], bx[U][NG];
 #pragma unroll
-            for (int u = 0; u < U; ++u)
+                for (int u = 0; u < U; ++u) {  // (lanes past nb hold an empty bitmap)
+                    const int j = j0 + u < 64 ? j0 + u : 63;
+                    const uint32_t m =
+                        j0 + u < nb ? uint32_t(__builtin_amdgcn_readlane(int(mj), j)) : 0u;
+                    const int o = __builtin_amdgcn_readlane(oj, j);
+                    const int64_t xr = 4 * int64_t(__builtin_amdgcn_readlane(cj, j));
+                    const uint32_t idx = uint32_t(o + __popc(m & belowA)) * uint32_t(sizeof(VT));
+                    a[u] = buf_value<VT>(a_rs, ((m >> eA) & 1u) ? idx : kOut);
+                    const int64_t left = ncols - xr;  // > 0: a block column inside the matrix
+                    const __amdgpu_buffer_rsrc_t x_rs = __builtin_amdgcn_make_buffer_rsrc(
+                        const_cast<double *>(x + xr * kx), short(0),
+                        int(left < 4 ? left : 4) * int(kx) * 8, kBufferDword3);
+                    const uint32_t cols = m | (m >> 4) | (m >> 8) | (m >> 12);
+                    const bool used = ((cols >> kk) & 1u) != 0u;
 #pragma unroll
-                for (int g = 0; g < NG; ++g)
-                    acc[g] = __builtin_amdgcn_mfma_f64_4x4x4f64(a[u], bx[u][g], acc[g], 0, 0, 0);
+                    for (int g = 0; g < NG; ++g)
+                        bx[u][g] = buf_value<double>(x_rs, used ? xoff[g] : kOut);
+                }
+#pragma unroll
+                for (int u = 0; u < U; ++u)
+#pragma unroll
+                    for (int g = 0; g < NG; ++g)
+                        acc[g] = __builtin_amdgcn_mfma_f64_4x4x4f64(a[u], bx[u][g], acc[g], 0, 0, 0);
+            }
         }
     }
-    const int row = 4 * br + kk;
-    if (row < nrows) {
+    if constexpr (kCm) {
 #pragma unroll
-        for (int g = 0; g < NG; ++g) {
-            if (!xon[g]) continue;
-            double out = alpha * acc[g];
-            if (beta != 0.0) out = fma(beta, b[int64_t(row) * kb + vrel[g]], out);
-            y[int64_t(row) * ky + vrel[g]] = out;
+        for (int g = 0; g < NG; ++g) s_y[16 * g + 4 * bs + nn][4 * w + kk] = acc[g];
+        __syncthreads();
+        const int row = 4 * br0 + (threadIdx.x & 15);
+        if (row >= nrows) return;
+        for (int v = threadIdx.x >> 4; v < kn; v += 16) {
+            double out = alpha * s_y[v][threadIdx.x & 15];
+            if (beta != 0.0) out = fma(beta, b[int64_t(k0 + v) * kb + row], out);
+            y[int64_t(k0 + v) * ky + row] = out;
+        }
+    } else {
+        const int row = 4 * br + kk;
+        if (row < nrows) {
+#pragma unroll
+            for (int g = 0; g < NG; ++g) {
+                const int rhs = 16 * g + 4 * bs + nn;
+                if (rhs >= kn) continue;
+                double out = alpha * acc[g];
+                if (beta != 0.0) out = fma(beta, b[int64_t(row) * kb + k0 + rhs], out);
+                y[int64_t(row) * ky + k0 + rhs] = out;
+            }
         }
     }
 }
 
-// Tiled transposes between the two multivector layouts (32 x 32 tiles in LDS,
-// both sides coalesced).  cm -> il: xi[i * k + v] = x[v * ldx + i].
+// Tiled transpose of a column-major multivector (32 x 32 tiles in LDS, both
+// sides coalesced): xi[i * k + v] = x[v * ldx + i].
 __global__ __launch_bounds__(256) void k_cm_to_il(int32_t n, int32_t k,
                                                   const double *__restrict__ x, int64_t ldx,
                                                   double *__restrict__ xi) {
@@ -1131,29 +1184,6 @@ __global__ __launch_bounds__(256) void k_cm_to_il(int32_t n, int32_t k,
     for (int r = ty; r < 32; r += 8) {
         const int i = i0 + r, v = v0 + tx;
         if (i < n && v < k) xi[int64_t(i) * k + v] = tile[tx][r];
-    }
-}
-
-// il -> cm with the SpMM epilogue: y[v * ldy + i] = alpha yi[i * k + v] + beta b[v * ldb + i]
-__global__ __launch_bounds__(256) void k_il_to_cm(int32_t n, int32_t k,
-                                                  const double *__restrict__ yi, double alpha,
-                                                  double beta, const double *b, int64_t ldb,
-                                                  double *y, int64_t ldy) {
-    __shared__ double tile[32][33];
-    const int i0 = blockIdx.x * 32, v0 = blockIdx.y * 32;
-    const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
-    for (int r = ty; r < 32; r += 8) {
-        const int i = i0 + r, v = v0 + tx;
-        tile[r][tx] = (i < n && v < k) ? yi[int64_t(i) * k + v] : 0.0;
-    }
-    __syncthreads();
-    for (int r = ty; r < 32; r += 8) {
-        const int v = v0 + r, i = i0 + tx;
-        if (v < k && i < n) {
-            double out = alpha * tile[tx][r];
-            if (beta != 0.0) out = fma(beta, b[int64_t(v) * ldb + i], out);
-            y[int64_t(v) * ldy + i] = out;
-        }
     }
 }
 
@@ -1350,8 +1380,8 @@ int launch_spmm_g(const Mbsr &A, const VT *val, int k, double alpha, const doubl
     return AMGT_OK;
 }
 
-// interleaved multivectors: 32 right-hand sides per launch
-template <typename VT>
+// X interleaved, Y interleaved or (kCm) column-major: 32 right-hand sides per launch
+template <typename VT, bool kCm>
 int launch_spmm_il(const Mbsr &A, const VT *val, int k, double alpha, const double *x,
                    int64_t kx, double beta, const double *b, int64_t kb, double *y, int64_t ky,
                    hipStream_t s) {
@@ -1359,11 +1389,11 @@ int launch_spmm_il(const Mbsr &A, const VT *val, int k, double alpha, const doub
     for (int k0 = 0; k0 < k; k0 += 32) {
         const int kn = k - k0 < 32 ? k - k0 : 32;
         if (kn > 16)
-            hipLaunchKernelGGL((k_spmm_mfma_il<2, VT>), dim3(unsigned(grid)), dim3(256), 0, s,
+            hipLaunchKernelGGL((k_spmm_mfma_il<2, VT, kCm>), dim3(unsigned(grid)), dim3(256), 0, s,
                                A.brow, A.nrows, A.ncols, A.blk_ptr, A.blk_col, A.blk_map,
                                A.val_ptr, val, k0, kn, x, kx, alpha, beta, b, kb, y, ky);
         else
-            hipLaunchKernelGGL((k_spmm_mfma_il<1, VT>), dim3(unsigned(grid)), dim3(256), 0, s,
+            hipLaunchKernelGGL((k_spmm_mfma_il<1, VT, kCm>), dim3(unsigned(grid)), dim3(256), 0, s,
                                A.brow, A.nrows, A.ncols, A.blk_ptr, A.blk_col, A.blk_map,
                                A.val_ptr, val, k0, kn, x, kx, alpha, beta, b, kb, y, ky);
         AMGT_HIP(hipGetLastError());
@@ -1372,31 +1402,17 @@ int launch_spmm_il(const Mbsr &A, const VT *val, int k, double alpha, const doub
 }
 
 // column-major multivectors with k >= 8: transpose X to the interleaved
-// layout, run the interleaved MFMA kernel, transpose back with the epilogue
+// layout, run the MFMA kernel with its column-major epilogue
 template <typename VT>
 int launch_spmm_cm_via_il(const Mbsr &A, const VT *val, int k, double alpha, const double *x,
                           int64_t ldx, double beta, const double *b, int64_t ldb, double *y,
                           int64_t ldy, hipStream_t s) {
-    double *xi = nullptr, *yi = nullptr;
+    double *xi = nullptr;
     AMGT_TRY(tmp_alloc_t(&xi, size_t(A.ncols) * size_t(k), s));
-    int st = tmp_alloc_t(&yi, size_t(A.nrows) * size_t(k), s);
-    if (st == AMGT_OK) {
-        const dim3 gx(unsigned((A.ncols + 31) / 32), unsigned((k + 31) / 32));
-        hipLaunchKernelGGL(k_cm_to_il, gx, dim3(256), 0, s, A.ncols, k, x, ldx, xi);
-        st = launch_spmm_il<VT>(A, val, k, 1.0, xi, k, 0.0, nullptr, k, yi, k, s);
-    }
-    if (st == AMGT_OK) {
-        const dim3 gy(unsigned((A.nrows + 31) / 32), unsigned((k + 31) / 32));
-        hipLaunchKernelGGL(k_il_to_cm, gy, dim3(256), 0, s, A.nrows, k, yi, alpha, beta, b, ldb,
-                           y, ldy);
-        hipError_t e = hipGetLastError();
-        if (e != hipSuccess) {
-            set_error(std::string("SpMM transpose: ") + hipGetErrorString(e));
-            st = AMGT_ERR_HIP;
-        }
-    }
+    const dim3 gx(unsigned((A.ncols + 31) / 32), unsigned((k + 31) / 32));
+    hipLaunchKernelGGL(k_cm_to_il, gx, dim3(256), 0, s, A.ncols, k, x, ldx, xi);
+    const int st = launch_spmm_il<VT, true>(A, val, k, alpha, xi, k, beta, b, ldb, y, ldy, s);
     tmp_free(xi, s);
-    tmp_free(yi, s);
     return st;
 }
 
@@ -1710,11 +1726,11 @@ int spmm_interleaved(const Mbsr &A, int precision, int k, double alpha, const do
     if (A.nrows == 0 || k == 0) return AMGT_OK;
     switch (precision) {
         case AMGT_DOUBLE:
-            return launch_spmm_il<double>(A, A.val, k, alpha, x, k, beta, b, k, y, k, s);
+            return launch_spmm_il<double, false>(A, A.val, k, alpha, x, k, beta, b, k, y, k, s);
         case AMGT_FLOAT:
-            return launch_spmm_il<float>(A, A.val32, k, alpha, x, k, beta, b, k, y, k, s);
+            return launch_spmm_il<float, false>(A, A.val32, k, alpha, x, k, beta, b, k, y, k, s);
         case AMGT_HALF:
-            return launch_spmm_il<__half>(A, A.val16, k, alpha / A.half_scale, x, k, beta, b, k,
+            return launch_spmm_il<__half, false>(A, A.val16, k, alpha / A.half_scale, x, k, beta, b, k,
                                           y, k, s);
         default:
             set_error("unknown precision");
