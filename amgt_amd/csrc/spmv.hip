@@ -1168,6 +1168,159 @@ __global__ __launch_bounds__(256) void k_spmm_mfma_il(
     }
 }
 
+// SpMM for sparse blocks: the entries of each of a block row's four rows are
+// listed in LDS (column, value), 16 lanes own a row, RPL right-hand sides each,
+// and a step takes the next entry of all four rows: its X row (consecutive
+// right-hand sides), RPL multiply-adds.  One wave per block row, lists of 32
+// blocks at a time; every row adds its entries in column order.
+// Against the MFMA form: at a fill of 1/4 three of four products of an
+// instruction are zeros and each instruction occupies the SIMD as long as 8 to
+// 16 vector multiply-adds; the list costs 27 steps a row on 27-pt where the
+// block form issues 54 MFMAs and the selection of 27 bitmaps' operands.
+constexpr int kListBlk = 32;   // blocks listed at a time
+constexpr int kListRow = 128;  // entries per row, at most 4 per block
+// inclusive sums within each half of the wave (DPP, as wave_incl_sum)
+__device__ __forceinline__ int half_incl_sum(int v) {
+    v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);
+    return v;
+}
+
+template <int RPL, typename VT, bool kCm>
+__global__ __launch_bounds__(256) void k_spmm_rows(
+    int32_t brow, int32_t nrows, const int32_t *__restrict__ blk_ptr,
+    const int32_t *__restrict__ blk_col, const uint16_t *__restrict__ blk_map,
+    const int32_t *__restrict__ val_ptr, const VT *__restrict__ val, int k0, int kn,
+    const double *__restrict__ x, int64_t kx, double alpha, double beta, const double *b,
+    int64_t kb, double *y, int64_t ky) {
+    constexpr int U = 4;  // entries in flight per row
+    struct List {
+        double val[4][kListRow];
+        int32_t col[4][kListRow];
+        uint16_t to[4 * kListRow];
+    };
+    __shared__ union {
+        List list[4];
+        double y[16 * RPL][17];
+    } sh;
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int br0 = remap_wg(blockIdx.x, gridDim.x) * 4;
+    const int br = __builtin_amdgcn_readfirstlane(br0 + w);
+    if (!kCm && br >= brow) return;  // whole wave
+    const int r = lane >> 4, v16 = lane & 15;
+    double acc[RPL];
+#pragma unroll
+    for (int q = 0; q < RPL; ++q) acc[q] = 0.0;
+    // right-hand sides RPL v16 .. (a lane past the last reads right-hand side
+    // k0, and writes nothing)
+    const int rhs = RPL * v16;
+    const double *xl[RPL];
+#pragma unroll
+    for (int q = 0; q < RPL; ++q) xl[q] = x + k0 + (rhs + q < kn ? rhs + q : 0);
+    // (RPL 2: one 16-byte load where the pairs are aligned and whole)
+    const bool pair = RPL == 2 && ((kx | k0 | kn) & 1) == 0 &&
+                      (reinterpret_cast<uintptr_t>(x) & 15u) == 0;
+    if (br < brow) {
+        List &s = sh.list[w];
+        const int h = lane >> 5;  // rows 2h, 2h + 1 of block lane & 31
+        const int p0 = blk_ptr[br], p1 = blk_ptr[br + 1];
+        int v0 = val_ptr[br];
+        for (int c0 = p0; c0 < p1; c0 += kListBlk) {
+            const int j = c0 + (lane & 31);
+            uint32_t m = 0u;
+            int col = 0;
+            if (j < p1) {
+                m = blk_map[j];
+                col = 4 * blk_col[j];
+            }
+            const int n = __popc(m), ninc = half_incl_sum(n);
+            const int nv = __builtin_amdgcn_readlane(ninc, 31);
+            double av[2];  // the first 128 values, before the lists wait for the bitmaps
+#pragma unroll
+            for (int u = 0; u < 2; ++u)
+                av[u] = 64 * u + lane < nv ? double(val[v0 + 64 * u + lane]) : 0.0;
+            uint32_t bits = (m >> (8 * h)) & 0xFFu;
+            const int c = __popc(bits & 0xFu) | __popc(bits >> 4) << 16;
+            const int cinc = half_incl_sum(c);
+            const int t01 = __builtin_amdgcn_readlane(cinc, 31);
+            const int t23 = __builtin_amdgcn_readlane(cinc, 63);
+            int a0 = (cinc - c) & 0xFFFF, a1 = (cinc - c) >> 16;
+            int src = ninc - n + (h ? __popc(m & 0xFFu) : 0);
+            while (bits) {
+                const int e = __builtin_ctz(bits);
+                bits &= bits - 1u;
+                const int at = (2 * h + (e >> 2)) * kListRow + (e < 4 ? a0++ : a1++);
+                s.col[0][at] = col + (e & 3);
+                s.to[src++] = uint16_t(at);
+            }
+            __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+#pragma unroll
+            for (int u = 0; u < 2; ++u)
+                if (64 * u + lane < nv) s.val[0][s.to[64 * u + lane]] = av[u];
+            for (int t = 128 + lane; t < nv; t += 64) s.val[0][s.to[t]] = double(val[v0 + t]);
+            v0 += nv;
+            __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            const int l0 = t01 & 0xFFFF, l1 = t01 >> 16, l2 = t23 & 0xFFFF, l3 = t23 >> 16;
+            const int len = r == 0 ? l0 : (r == 1 ? l1 : (r == 2 ? l2 : l3));
+            const int steps = max(max(l0, l1), max(l2, l3));
+            for (int t = 0; t < steps; t += U) {
+                double a[U], xv[U][RPL];
+#pragma unroll
+                for (int u = 0; u < U; ++u) {
+                    const int at = min(t + u, kListRow - 1);
+                    const int64_t cc = t + u < len ? s.col[r][at] : 0;
+                    a[u] = s.val[r][at];
+                    if (pair) {
+                        const double2 x2 = *reinterpret_cast<const double2 *>(xl[0] + cc * kx);
+                        xv[u][0] = x2.x;
+                        if constexpr (RPL == 2) xv[u][1] = x2.y;
+                    } else {
+#pragma unroll
+                        for (int q = 0; q < RPL; ++q) xv[u][q] = xl[q][cc * kx];
+                    }
+                }
+#pragma unroll
+                for (int u = 0; u < U; ++u)
+                    if (t + u < len) {
+#pragma unroll
+                        for (int q = 0; q < RPL; ++q) acc[q] = fma(a[u], xv[u][q], acc[q]);
+                    }
+            }
+            __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+        }
+    }
+    if constexpr (kCm) {
+        __syncthreads();  // the lists are done
+#pragma unroll
+        for (int q = 0; q < RPL; ++q) sh.y[rhs + q][4 * w + r] = acc[q];
+        __syncthreads();
+        const int row = 4 * br0 + (threadIdx.x & 15);
+        if (row >= nrows) return;
+        for (int v = threadIdx.x >> 4; v < kn; v += 16) {
+            double out = alpha * sh.y[v][threadIdx.x & 15];
+            if (beta != 0.0) out = fma(beta, b[int64_t(k0 + v) * kb + row], out);
+            y[int64_t(k0 + v) * ky + row] = out;
+        }
+    } else {
+        const int row = 4 * br + r;
+        if (row < nrows) {
+#pragma unroll
+            for (int q = 0; q < RPL; ++q) {
+                if (rhs + q >= kn) continue;
+                double out = alpha * acc[q];
+                if (beta != 0.0) out = fma(beta, b[int64_t(row) * kb + k0 + rhs + q], out);
+                y[int64_t(row) * ky + k0 + rhs + q] = out;
+            }
+        }
+    }
+}
+
 // Tiled transpose of a column-major multivector (32 x 32 tiles in LDS, both
 // sides coalesced): xi[i * k + v] = x[v * ldx + i].
 __global__ __launch_bounds__(256) void k_cm_to_il(int32_t n, int32_t k,
@@ -1380,22 +1533,30 @@ int launch_spmm_g(const Mbsr &A, const VT *val, int k, double alpha, const doubl
     return AMGT_OK;
 }
 
+constexpr double kSpmmRowsMaxNnz = 8.0;
 // X interleaved, Y interleaved or (kCm) column-major: 32 right-hand sides per launch
 template <typename VT, bool kCm>
 int launch_spmm_il(const Mbsr &A, const VT *val, int k, double alpha, const double *x,
                    int64_t kx, double beta, const double *b, int64_t kb, double *y, int64_t ky,
                    hipStream_t s) {
     const int64_t grid = (int64_t(A.brow) + 3) / 4;
+    const bool rows = A.avg_nnz <= kSpmmRowsMaxNnz;
     for (int k0 = 0; k0 < k; k0 += 32) {
         const int kn = k - k0 < 32 ? k - k0 : 32;
-        if (kn > 16)
-            hipLaunchKernelGGL((k_spmm_mfma_il<2, VT, kCm>), dim3(unsigned(grid)), dim3(256), 0, s,
-                               A.brow, A.nrows, A.ncols, A.blk_ptr, A.blk_col, A.blk_map,
-                               A.val_ptr, val, k0, kn, x, kx, alpha, beta, b, kb, y, ky);
-        else
-            hipLaunchKernelGGL((k_spmm_mfma_il<1, VT, kCm>), dim3(unsigned(grid)), dim3(256), 0, s,
-                               A.brow, A.nrows, A.ncols, A.blk_ptr, A.blk_col, A.blk_map,
-                               A.val_ptr, val, k0, kn, x, kx, alpha, beta, b, kb, y, ky);
+#define AMGT_SPMM_ROWS(R_)                                                                       \
+    hipLaunchKernelGGL((k_spmm_rows<R_, VT, kCm>), dim3(unsigned(grid)), dim3(256), 0, s, A.brow, \
+                       A.nrows, A.blk_ptr, A.blk_col, A.blk_map, A.val_ptr, val, k0, kn, x, kx,  \
+                       alpha, beta, b, kb, y, ky)
+#define AMGT_SPMM_MFMA(G_)                                                                       \
+    hipLaunchKernelGGL((k_spmm_mfma_il<G_, VT, kCm>), dim3(unsigned(grid)), dim3(256), 0, s,     \
+                       A.brow, A.nrows, A.ncols, A.blk_ptr, A.blk_col, A.blk_map, A.val_ptr, val, \
+                       k0, kn, x, kx, alpha, beta, b, kb, y, ky)
+        if (rows && kn > 16) AMGT_SPMM_ROWS(2);
+        else if (rows) AMGT_SPMM_ROWS(1);
+        else if (kn > 16) AMGT_SPMM_MFMA(2);
+        else AMGT_SPMM_MFMA(1);
+#undef AMGT_SPMM_ROWS
+#undef AMGT_SPMM_MFMA
         AMGT_HIP(hipGetLastError());
     }
     return AMGT_OK;
