@@ -612,6 +612,124 @@ __global__ __launch_bounds__(256) void k_spmv_blk(
     tile_post(ep, wg);
 }
 
+// Long block rows: one wave per block row, lane (slot s, row r) of 16 x 4 takes
+// row r's nibble of block s, 16 blocks a step.  The lanes are in the order of
+// the values, so a scan of the nibbles' popcounts gives every lane its first
+// value; it loads four consecutive ones (unaligned) and picks each column's by
+// its rank in the nibble: no loop over bits, no LDS, no barrier, 16 partial sums
+// per row reduced by a fixed tree.  The block-lane kernel walks up to 16 bits
+// per lane with dynamic register picks and waits for its workgroup's longest
+// row.  The kernel is bound by the issue of its memory instructions (16 cycles
+// each for 64 addresses), so bitmaps and columns are loaded 64 blocks at a time
+// and handed out by lane permutes, and a lane loads one element of its block's x
+// segment, the four of a block sharing theirs.
+// four consecutive values at any element's address; pick<k>: the k-th, k = 0..3
+template <typename VT> struct Four;
+template <> struct Four<double> {
+    typedef double Two __attribute__((ext_vector_type(2), aligned(8)));
+    Two a, b;
+    __device__ __forceinline__ void load(const double *p) {
+        a = reinterpret_cast<const Two *>(p)[0];
+        b = reinterpret_cast<const Two *>(p)[1];
+    }
+    __device__ __forceinline__ double pick(int k) const {
+        const double lo = (k & 1) ? a.y : a.x, hi = (k & 1) ? b.y : b.x;
+        return (k & 2) ? hi : lo;
+    }
+};
+template <> struct Four<float> {
+    typedef float Vec __attribute__((ext_vector_type(4), aligned(4)));
+    Vec a;
+    __device__ __forceinline__ void load(const float *p) { a = *reinterpret_cast<const Vec *>(p); }
+    __device__ __forceinline__ float pick(int k) const {
+        const float lo = (k & 1) ? a.y : a.x, hi = (k & 1) ? a.w : a.z;
+        return (k & 2) ? hi : lo;
+    }
+};
+template <> struct Four<__half> {
+    typedef uint32_t Vec __attribute__((ext_vector_type(2), aligned(2)));
+    uint64_t a;
+    __device__ __forceinline__ void load(const __half *p) {
+        const Vec v = *reinterpret_cast<const Vec *>(p);
+        a = uint64_t(v.y) << 32 | v.x;
+    }
+    __device__ __forceinline__ __half pick(int k) const {
+        return __ushort_as_half(static_cast<unsigned short>(a >> ((16 * k) & 63)));
+    }
+};
+
+// element c of the four lanes of a quad
+template <int c>
+__device__ __forceinline__ float quad_get(float v) {
+    return __int_as_float(
+        __builtin_amdgcn_update_dpp(0, __float_as_int(v), c * 0x55, 0xf, 0xf, false));
+}
+template <int c>
+__device__ __forceinline__ double quad_get(double v) {
+    return __hiloint2double(
+        __builtin_amdgcn_update_dpp(0, __double2hiint(v), c * 0x55, 0xf, 0xf, false),
+        __builtin_amdgcn_update_dpp(0, __double2loint(v), c * 0x55, 0xf, 0xf, false));
+}
+
+template <typename VT, typename AT, typename EP>
+__global__ __launch_bounds__(256) void k_spmv_long(
+    int32_t brow, int32_t nrows, int32_t ncols, int32_t nnz, const int32_t *__restrict__ blk_ptr,
+    const int32_t *__restrict__ blk_col, const uint16_t *__restrict__ blk_map,
+    const int32_t *__restrict__ val_ptr, const VT *__restrict__ val, const double *__restrict__ x,
+    EP ep, double *y) {
+    constexpr int U = 4;
+    const int lane = threadIdx.x & 63;
+    const int br = __builtin_amdgcn_readfirstlane(remap_wg(blockIdx.x, gridDim.x) * 4 +
+                                                  int(threadIdx.x >> 6));
+    if (br >= brow) return;  // whole wave
+    const int r = lane & 3, s = lane >> 2;
+    const int p0 = blk_ptr[br], p1 = blk_ptr[br + 1];
+    int voff = val_ptr[br];
+    AT acc = AT(0);
+    for (int jb = p0; jb < p1; jb += 16 * U) {
+        const int j = min(jb + lane, p1 - 1);  // clamped: unconditional loads
+        uint32_t mj = blk_map[j];
+        const int cj = blk_col[j];
+        if (jb + lane >= p1) mj = 0u;
+        uint32_t nib[U];
+        int from[U];
+        Four<VT> v[U];
+        AT xs[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            nib[u] = 0u;
+            if (jb + 16 * u >= p1) continue;  // wave-uniform
+            const int addr = (16 * u + s) << 2;
+            nib[u] = (uint32_t(__builtin_amdgcn_ds_bpermute(addr, int(mj))) >> (4 * r)) & 0xFu;
+            const int col = __builtin_amdgcn_ds_bpermute(addr, cj);
+            xs[u] = AT(x[min(4 * col + r, ncols - 1)]);
+            const int cn = __popc(nib[u]);
+            const int inc = wave_incl_sum(cn);
+            const int o = voff + inc - cn;
+            voff += __builtin_amdgcn_readlane(inc, 63);
+            const int at = min(o, nnz - 4);  // four values inside the array (nnz >= 4)
+            from[u] = o - at;
+            v[u].load(val + at);
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            if (jb + 16 * u >= p1) continue;
+            const AT xq[4] = {quad_get<0>(xs[u]), quad_get<1>(xs[u]), quad_get<2>(xs[u]),
+                              quad_get<3>(xs[u])};
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+                const int k = from[u] + __popc(nib[u] & ((1u << c) - 1u));  // 0..3 for an entry
+                const AT t = mul_acc<VT, AT>(acc, v[u].pick(k), double(xq[c]));
+                acc = ((nib[u] >> c) & 1u) ? t : acc;
+            }
+        }
+    }
+#pragma unroll
+    for (int d = 32; d >= 4; d >>= 1) acc += __shfl_xor(acc, d);
+    const int row = 4 * br + r;
+    if (s == 0 && row < nrows) y[row] = ep(row, double(acc));
+}
+
 // Balanced variant (counterpart of bsr_spmv_balanced_tc_fp64,
 // csr_matvec_device.c:556-613, with the split of BSR_BALANCED_PREPROCESS_GPU
 // :1269-1300): workgroup t owns blocks [t*CAPB, (t+1)*CAPB) whatever rows they
@@ -1421,6 +1539,16 @@ int launch_spmv_blk_g(const Mbsr &A, const VT *val, const double *x, EP ep, doub
     return AMGT_OK;
 }
 
+template <typename VT, typename AT, typename EP>
+int launch_spmv_long(const Mbsr &A, const VT *val, const double *x, EP ep, double *y,
+                     hipStream_t s) {
+    hipLaunchKernelGGL((k_spmv_long<VT, AT, EP>), dim3(unsigned((int64_t(A.brow) + 3) / 4)),
+                       dim3(256), 0, s, A.brow, A.nrows, A.ncols, int32_t(A.nnz), A.blk_ptr,
+                       A.blk_col, A.blk_map, A.val_ptr, val, x, ep, y);
+    AMGT_HIP(hipGetLastError());
+    return AMGT_OK;
+}
+
 // Tile tables and carry buffer of the balanced kernel: the handle's own
 // (spmv_prepare) or a caller's workspace (spmv_balanced_ws).
 struct BalTables {
@@ -1446,6 +1574,24 @@ int launch_spmv_bal_g(const Mbsr &A, const BalTables &tb, const VT *val, const d
                        tb.lo, tb.head, tb.carry, ep, y);
     AMGT_HIP(hipGetLastError());
     return AMGT_OK;
+}
+
+// Whether an average tile of `rows` block rows stays within 90 % of the block
+// kernel's 512 blocks and 85 % of its 2048 values, so that few tiles overflow to
+// its walk over global memory (the counts vary more for values).
+bool blk_tile_fits(const Mbsr &A, int rows) {
+    const double brow = A.brow > 0 ? double(A.brow) : 1.0;
+    return double(A.nblk) / brow * rows <= 460.0 && double(A.nnz) / brow * rows <= 1740.0;
+}
+
+// Whether the block kind runs its long-row kernel: rows of which eight do not
+// fit a tile.  Measured (us, FP64 / FP32 / FP16, tile of 8 rows against long):
+// coarse operators of 60 blocks a row 31.5 / 27 / 24 against 21 / 16 / 13 (62k
+// rows), 421 / 383 / 336 against 247 / 217 / 183 (1M rows); 44 blocks, 231
+// values a row 26 / 21 / 19 against 21 / 16 / 13; where eight rows fit the tile
+// wins: 43 blocks, 196 values a row 31.5 / 27 / 28 against 46 / 35 / 32.
+bool spmv_long_rows(const Mbsr &A, int lanes) {
+    return lanes == 64 && A.nnz >= 4 && !blk_tile_fits(A, 8);
 }
 
 // y[row] = ep(row, (A x)[row]) with the handle's kernel kind and lanes setting
@@ -1474,6 +1620,7 @@ int launch_spmv_t(const Mbsr &A, const VT *val, int lanes, const double *x, EP e
         val_aligned) {
         // lanes selects the tile: 4 -> 64 block rows (2 blocks per thread),
         // 8 -> 128 (4 per thread), 16 -> 32, 32 -> 16, 64 -> 8 block rows
+        if (spmv_long_rows(A, lanes)) return launch_spmv_long<VT, AT>(A, val, x, ep, y, s);
         switch (lanes) {
             case 4: return launch_spmv_blk_g<64, 2, VT, AT>(A, val, x, ep, y, s);
             case 8: return launch_spmv_blk_g<128, 4, VT, AT>(A, val, x, ep, y, s);
@@ -1533,7 +1680,13 @@ int launch_spmm_g(const Mbsr &A, const VT *val, int k, double alpha, const doubl
     return AMGT_OK;
 }
 
-constexpr double kSpmmRowsMaxNnz = 8.0;
+// Entries per block up to which k_spmm_rows runs instead of k_spmm_mfma_il.
+// Measured on 16384 block rows of 27 random blocks, k = 8 / 16 / 32 (us, rows
+// against MFMA): 2.1 entries 19 / 23 / 30 against 31 / 32 / 45; 4.0 entries 29 /
+// 31 / 43 against 31 / 32 / 44; 6.0 entries 40 / 41 / 57 against 31 / 31 / 44.
+// Stencils, whose rows have equal lengths, gain more: 27-pt 64^3 (4.1 entries),
+// k = 32, 133 against 167.
+constexpr double kSpmmRowsMaxNnz = 4.5;
 // X interleaved, Y interleaved or (kCm) column-major: 32 right-hand sides per launch
 template <typename VT, bool kCm>
 int launch_spmm_il(const Mbsr &A, const VT *val, int k, double alpha, const double *x,
@@ -1629,12 +1782,11 @@ int spmv_default_lanes(const Mbsr &A) {
     }
     if (A.spmv_kernel == kSpmvBalanced) return 16;  // tiles of 256 blocks
     if (A.spmv_kernel == kSpmvBlock) {
-        // block-lane tiles of 512 blocks: the most block rows per tile (64, 32,
-        // 16 or 8, lanes 4 / 16 / 32 / 64) whose average load stays within 90 %
-        // of the capacity, so that few tiles overflow to the global-memory walk
-        if (avg * 64.0 <= 460.0) return 4;
-        if (avg * 32.0 <= 460.0) return 16;
-        if (avg * 16.0 <= 460.0) return 32;
+        // block-lane tiles: the most block rows per tile (64, 32, 16 or 8, lanes
+        // 4 / 16 / 32 / 64) that fit
+        if (blk_tile_fits(A, 64)) return 4;
+        if (blk_tile_fits(A, 32)) return 16;
+        if (blk_tile_fits(A, 16)) return 32;
         return 64;
     }
     // enough slots that a typical block row takes about two block steps

@@ -244,6 +244,38 @@ def test_default_kernel_from_statistics(dev):
         assert M.info()["spmv_kernel"] == want
 
 
+# block rows of 1 to 130 blocks (edges of the 16-block steps and the 64-block
+# loads), rows of more values than eight of a tile hold, ragged columns
+@pytest.mark.parametrize("prec,tol", [(L.AMGT_DOUBLE, 1e-12), (L.AMGT_FLOAT, 2e-6),
+                                      (L.AMGT_HALF, 2e-3)])
+@pytest.mark.parametrize("n", [1203, 1204])
+def test_spmv_long_rows(dev, n, prec, tol):
+    rng = np.random.default_rng(n)
+    counts = [1, 15, 16, 17, 63, 64, 65, 128, 130, 0, 48, 100, 127]  # blocks per block row
+    dens = [1.0, 0.2]
+    rows, cols, m = [], [], 4 * len(counts) - 2
+    for br, c in enumerate(counts):
+        for bc in rng.permutation((n + 3) // 4)[:c]:
+            full = rng.random(16) < dens[br % 2]
+            full[int(rng.integers(0, 8))] = True
+            for e in np.flatnonzero(full):
+                r, k = 4 * br + e // 4, 4 * bc + e % 4
+                if r < m and k < n:
+                    rows.append(r)
+                    cols.append(k)
+    S = sp.csr_matrix((rng.standard_normal(len(rows)), (rows, cols)), shape=(m, n))
+    I, J, A = S.indptr.astype(np.int32), S.indices.astype(np.int32), S.data
+    ref = O.csr2mbsr(m, n, I, J, A)
+    M = make(dev, m, n, I, J, A)
+    M.set_precision(prec)
+    M.set_spmv_kernel(L.AMGT_SPMV_BLOCK)
+    M.set_spmv_lanes(64)
+    x, b = rng.standard_normal(n), rng.standard_normal(m)
+    exp = O.mbsr_spmv(ref, -1.0, x, 1.0, b)
+    y = M.spmv(T(x, dev), alpha=-1.0, beta=1.0, b=T(b, dev)).cpu().numpy()
+    assert np.all(np.abs(y - exp) <= tol * row_scale(m, n, I, J, A, x, 1.0, b))
+
+
 @pytest.mark.parametrize("prec,tol", [(L.AMGT_FLOAT, 2e-6), (L.AMGT_HALF, 2e-3)])
 def test_spmv_balanced_low_precision(dev, prec, tol):
     (m, n), I, J, A = CASES["skewed"]()
