@@ -21,6 +21,7 @@
 // the mBSR handles have ascending columns).
 #include "internal.hpp"
 
+#include <algorithm>
 #include <vector>
 
 namespace amgt {
@@ -511,7 +512,7 @@ __global__ __launch_bounds__(kThreads) void k_extpi_row(
 //    of row i1 that are P columns (a lane per entry of row i1, its column
 //    looked up in the LDS table), so every weight receives its terms in the
 //    host's order;
-//  * the diagonal, the truncation sort and rescale on lane 0, in order.
+//  * the diagonal and the row sums in order, the truncation by ranks.
 // capacities: WA entries of row i (A and S), WT distinct P columns kept in
 // LDS, WH table slots: at most WT + 64 candidate columns (the insertions stop
 // once WT is passed) plus WA strong F neighbours ever enter the table, which
@@ -529,8 +530,8 @@ struct WaveRow {
     double pw[WT];
     double jdist[WA];
     double jdiag[WA];
-    int32_t jinfo[WA];  // >= 0: P position; -1 skip/diag; -2 strong F (distribute);
-                         // -3 add a_ij to the diagonal
+    int32_t jinfo[WA];  // >= 0: P position; -1 none; -2 strong F (distribute); at the
+                         // end, with jdist, the kept columns and weights
     int32_t jsgn[WA];
     int32_t jb1[WA];    // strong F neighbour: its row's range in J / A
     int32_t je1[WA];
@@ -592,7 +593,10 @@ __global__ __launch_bounds__(64) void k_extpi_wave(
         s.hkey[t] = -1;
         s.hval[t] = INT_MAX;
     }
-    if (lane == 0) s.sc[2] = 0;  // distinct candidate columns
+    if (lane == 0) {
+        s.sc[0] = -1;  // the diagonal's place
+        s.sc[2] = 0;   // distinct candidate columns
+    }
     __syncthreads();
     // candidates in the host's order (par_lr_interp.c:1501-1560)
     int T = 0;
@@ -745,10 +749,10 @@ __global__ __launch_bounds__(64) void k_extpi_wave(
                     dist = s.aval[jj] / sum;
                     if (qi >= 0 && (sgn * aqi) < 0) dterm = dist * aqi;
                 } else {
-                    info = -3;
+                    dterm = s.aval[jj];
                 }
             } else if (cf[i1] != -3) {
-                info = -3;
+                dterm = s.aval[jj];
             }
         }
         s.jinfo[jj] = info;
@@ -779,47 +783,71 @@ __global__ __launch_bounds__(64) void k_extpi_wave(
         }
         __syncthreads();  // the next entry's terms may go to the same weights
     }
-    if (lane == 0) {
-        double diagonal = 0.0;
-        for (int jj = 0; jj < la; ++jj)
-            if (s.acol[jj] == i) {
-                diagonal = s.aval[jj];
-                break;
+    // the diagonal in row order (every lane the same sum; 0.0 for the entries
+    // that add nothing)
+    double diagonal = 0.0;
+    for (int t = lane; t < la; t += 64)
+        if (s.acol[t] == i) s.sc[0] = t;
+    __syncthreads();
+    if (s.sc[0] >= 0) diagonal = s.aval[s.sc[0]];
+    for (int jj = 0; jj < la; ++jj) diagonal += s.jdiag[jj];
+    if (diagonal != 0)
+        for (int q = lane; q < c; q += 64) s.pw[q] /= -diagonal;
+    __syncthreads();
+    // truncation (par_csr_matrix.c:3130-3215): where the kept weights are
+    // distinct in magnitude, sorted order is the order of the ranks, which the
+    // lanes count (the host's quicksort on one lane took most of a long row's
+    // time); else the quicksort
+    const bool trunc = max_elmts > 0 && c > max_elmts;
+    const int cc = trunc ? max_elmts : c;
+    int32_t *kcol = s.pcol;
+    double *kw = s.pw;
+    if (trunc) {  // uniform
+        double row_sum = 0.0;
+        for (int q = 0; q < c; ++q) row_sum += s.pw[q];
+        bool tie = max_elmts > WA;  // the kept entries' LDS
+        if (!tie)
+            for (int q = lane; q < c; q += 64) {
+                const double a = fabs(s.pw[q]);
+                int above = 0, same = 0;
+                for (int t = 0; t < c; ++t) {
+                    const double b = fabs(s.pw[t]);
+                    above += b > a ? 1 : 0;
+                    same += b == a ? 1 : 0;
+                }
+                if (above < max_elmts) {
+                    if (same != 1) {
+                        tie = true;
+                    } else {
+                        s.jinfo[above] = s.pcol[q];
+                        s.jdist[above] = s.pw[q];
+                    }
+                }
             }
-        for (int jj = 0; jj < la; ++jj) {
-            const int info = s.jinfo[jj];
-            if (info == -2) {
-                diagonal += s.jdiag[jj];
-            } else if (info == -3) {
-                diagonal += s.aval[jj];
-            }
-        }
-        s.sc[0] = 0;
-        if (diagonal != 0)
-            for (int q = 0; q < c; ++q) s.pw[q] /= -diagonal;
-        int cc = c;
-        if (max_elmts > 0 && c > max_elmts) {
-            double row_sum = 0.0;
-            for (int q = 0; q < c; ++q) row_sum += s.pw[q];
+        if (__ballot(tie) == 0ull) {
+            kcol = s.jinfo;
+            kw = s.jdist;
+        } else if (lane == 0) {
             qsort2_abs(s.pcol, s.pw, 0, c - 1);
-            double scale = 0.0;
-            for (int q = 0; q < max_elmts; ++q) scale += s.pw[q];
-            if (scale != 0. && scale != row_sum) {
-                scale = row_sum / scale;
-                for (int q = 0; q < max_elmts; ++q) s.pw[q] *= scale;
-            }
-            cc = max_elmts;
         }
-        s.sc[1] = cc;
+        __syncthreads();
+        double scale = 0.0;
+        for (int q = 0; q < max_elmts; ++q) scale += kw[q];
+        if (scale != 0. && scale != row_sum) {
+            scale = row_sum / scale;
+            __syncthreads();
+            for (int q = lane; q < max_elmts; q += 64) kw[q] *= scale;
+        }
+    }
+    __syncthreads();
+    if (lane == 0) {
         out.cnt[i] = cc;
         use[i] = 0;
     }
-    __syncthreads();
-    const int cc = s.sc[1];
     const int64_t o = out.at(i);
     for (int q = lane; q < cc; q += 64) {
-        out.sj[o + q] = s.pcol[q];
-        out.sw[o + q] = s.pw[q];
+        out.sj[o + q] = kcol[q];
+        out.sw[o + q] = kw[q];
     }
 }
 
@@ -927,15 +955,15 @@ __global__ __launch_bounds__(kThreads) void k_extpi_group(
     int32_t n, const int32_t *__restrict__ I, const int32_t *__restrict__ J,
     const double *__restrict__ A, const int32_t *__restrict__ SI, const int32_t *__restrict__ SJ,
     const int32_t *__restrict__ cf, const int8_t *__restrict__ dneg, int max_elmts, RowSlots out,
-    int32_t *__restrict__ use, int code, int overflow_code, int32_t *__restrict__ ovf) {
+    int32_t *__restrict__ use, int per, int code, int overflow_code, int32_t *__restrict__ ovf) {
     constexpr int NG = kThreads / G, WH = 8 * G, WT = 4 * G;
     __shared__ GroupRow<G> s_row[NG];
     __shared__ int32_t s_list[kThreads];
     __shared__ int s_wc[kThreads / 64];
     const int tid = threadIdx.x, lane = tid & 63;
-    // this kernel's rows among the workgroup's, packed
-    const int row = blockIdx.x * kThreads + tid;
-    const bool mine = row < n && use[row] == code;
+    // this kernel's rows among the workgroup's `per`, packed
+    const int row = blockIdx.x * per + tid;
+    const bool mine = tid < per && row < n && use[row] == code;
     const uint64_t bal = __ballot(mine);
     if (lane == 0) s_wc[tid >> 6] = __popcll(bal);
     __syncthreads();
@@ -1675,10 +1703,17 @@ int amgt_amg_extpi_interp(int32_t n, const int32_t *A_i, const int32_t *A_j,
     };
     // (after the lists of round 0 are written: an overflow changes the row's code)
     auto group_rows = [&]() -> int {
+        // rows per workgroup: up to 256 (its groups then take rows of this kernel
+        // only, one after the other), fewer on small levels, where the time is that
+        // of one group's rows (512^2 5-pt, level 3, 3481 rows of 27: 797 us with
+        // 256, the wave kernel 327)
 #define AMGT_EXTPI_GROUP(G_, CODE_)                                                            \
-    if (h.c[CODE_ - 1] > 0)                                                                    \
-    hipLaunchKernelGGL((k_extpi_group<G_>), g, b, 0, s, n, A_i, A_j, A_data, S_i, S_j,         \
-                       cf_marker, dneg, max_elmts, slots, use, CODE_, kTier64, ovf)
+    if (h.c[CODE_ - 1] > 0) {                                                                  \
+        const int per = std::max(kThreads / G_, std::min(kThreads, (n + 2047) / 2048));        \
+        hipLaunchKernelGGL((k_extpi_group<G_>), dim3(unsigned((n + per - 1) / per)), b, 0, s,  \
+                           n, A_i, A_j, A_data, S_i, S_j, cf_marker, dneg, max_elmts, slots,   \
+                           use, per, CODE_, kTier64, ovf);                                     \
+    }
         AMGT_EXTPI_GROUP(8, kGroup8);
         AMGT_EXTPI_GROUP(16, kGroup16);
         AMGT_EXTPI_GROUP(32, kGroup32);
