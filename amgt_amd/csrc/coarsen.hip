@@ -20,6 +20,7 @@
 // The diagonal of a row is found by column (HYPRE keeps it first; exports of
 // the mBSR handles have ascending columns).
 #include "internal.hpp"
+#include "rowpass.hpp"
 
 #include <algorithm>
 #include <vector>
@@ -58,7 +59,45 @@ __device__ __forceinline__ int64_t diag_pos(const int32_t *__restrict__ I,
 }
 
 // ---- strength (par_strength.c:75-528, one function) ---------------------------
+// A thread per row; the entries of the workgroup's 256 rows are staged in LDS
+// with coalesced loads where they fit (7-pt: 1792 of kStageEntries), and the
+// strong columns leave through LDS.  (Threads walking their rows in memory: 81
+// us to count and 188 us to fill on 7-pt 128^3, 176 MB read by each.)
+constexpr int kStageEntries = 2048;
+
 #pragma clang fp contract(off)
+// row entries [b, e) of j / a; strong columns to out (kFill), their number
+// returned; d: the diagonal's position or -1
+template <bool kFill>
+__device__ __forceinline__ int strong_entries(const int32_t *j, const double *a, int64_t b,
+                                              int64_t e, int64_t d, double theta,
+                                              double max_row_sum, int32_t *out) {
+    const double diag = d >= 0 ? a[d] : 0.0;
+    double row_scale = 0.0, row_sum = diag;
+    for (int64_t p = b; p < e; ++p) {
+        if (p == d) continue;
+        const double v = a[p];
+        if (diag < 0) row_scale = v > row_scale ? v : row_scale;
+        else row_scale = v < row_scale ? v : row_scale;
+        row_sum += v;
+    }
+    int c = 0;
+    // a row too dominant by the row-sum test keeps only weak dependencies
+    if (!(fabs(row_sum) > fabs(diag) * max_row_sum && max_row_sum < 1.0)) {
+        const double thr = theta * row_scale;
+        for (int64_t p = b; p < e; ++p) {
+            if (p == d) continue;
+            const double v = a[p];
+            const bool weak = diag < 0 ? (v <= thr) : (v >= thr);
+            if (!weak) {
+                if (kFill) out[c] = j[p];
+                ++c;
+            }
+        }
+    }
+    return c;
+}
+
 template <bool kFill>
 __global__ __launch_bounds__(kThreads) void k_strength(int32_t n, const int32_t *__restrict__ I,
                                                       const int32_t *__restrict__ J,
@@ -66,33 +105,36 @@ __global__ __launch_bounds__(kThreads) void k_strength(int32_t n, const int32_t 
                                                       double max_row_sum, int32_t *__restrict__ cnt,
                                                       const int32_t *__restrict__ SI,
                                                       int32_t *__restrict__ SJ) {
-    const int i = blockIdx.x * kThreads + threadIdx.x;
-    if (i >= n) return;
-    const int64_t d = diag_pos(I, J, i);
-    const double diag = d >= 0 ? A[d] : 0.0;
-    double row_scale = 0.0, row_sum = diag;
-    for (int64_t p = I[i]; p < I[i + 1]; ++p) {
-        if (p == d) continue;
-        const double a = A[p];
-        if (diag < 0) row_scale = a > row_scale ? a : row_scale;
-        else row_scale = a < row_scale ? a : row_scale;
-        row_sum += a;
-    }
-    int c = 0;
-    int64_t out = kFill ? SI[i] : 0;
-    // a row too dominant by the row-sum test keeps only weak dependencies
-    if (!(fabs(row_sum) > fabs(diag) * max_row_sum && max_row_sum < 1.0)) {
-        const double thr = theta * row_scale;
-        for (int64_t p = I[i]; p < I[i + 1]; ++p) {
-            if (p == d) continue;
-            const double a = A[p];
-            const bool weak = diag < 0 ? (a <= thr) : (a >= thr);
-            if (!weak) {
-                if (kFill) SJ[out++] = J[p];
-                ++c;
-            }
+    __shared__ double s_a[kStageEntries];
+    __shared__ int32_t s_j[kStageEntries];
+    __shared__ int32_t s_out[kFill ? kStageEntries : 1];
+    const int r0 = blockIdx.x * kThreads, i = r0 + threadIdx.x;
+    const int e0 = I[r0], ne = I[min(r0 + kThreads, n)] - e0;
+    if (ne <= kStageEntries) {  // uniform
+        for (int t = threadIdx.x; t < ne; t += kThreads) {
+            s_j[t] = J[e0 + t];
+            s_a[t] = A[e0 + t];
         }
+        __syncthreads();
+        const int o0 = kFill ? SI[r0] : 0;
+        if (i < n) {
+            const int b = I[i] - e0, e = I[i + 1] - e0;
+            int d = -1;
+            for (int p = b; p < e && d < 0; ++p) d = s_j[p] == i ? p : -1;
+            const int c = strong_entries<kFill>(s_j, s_a, b, e, d, theta, max_row_sum,
+                                                kFill ? s_out + (SI[i] - o0) : nullptr);
+            if (!kFill) cnt[i] = c;
+        }
+        if constexpr (kFill) {
+            __syncthreads();
+            const int no = SI[min(r0 + kThreads, n)] - o0;
+            for (int t = threadIdx.x; t < no; t += kThreads) SJ[o0 + t] = s_out[t];
+        }
+        return;
     }
+    if (i >= n) return;
+    const int c = strong_entries<kFill>(J, A, I[i], I[i + 1], diag_pos(I, J, i), theta,
+                                        max_row_sum, kFill ? SJ + SI[i] : nullptr);
     if (!kFill) cnt[i] = c;
 }
 
@@ -106,16 +148,22 @@ __global__ __launch_bounds__(kThreads) void k_col_count(int32_t n, const int32_t
 }
 
 // x_{k} = a^k x_0 mod m of the Park-Miller generator (random.c:43-101); all
-// products stay below 2^62
+// products stay below 2^62.  m = 2^31 - 1, so 2^31 = 1 (mod m) and a product is
+// reduced by adding its upper and lower 31 bits (twice), without a division.
+__device__ __forceinline__ uint64_t pm_mod(uint64_t v) {
+    constexpr uint64_t kM = 2147483647u;
+    v = (v & kM) + (v >> 31);
+    v = (v & kM) + (v >> 31);
+    return v >= kM ? v - kM : v;
+}
 __device__ __forceinline__ uint64_t pm_jump(uint64_t x0, uint64_t k) {
-    constexpr uint64_t kA = 16807u, kM = 2147483647u;
-    uint64_t r = 1u, b = kA;
+    uint64_t r = 1u, b = 16807u;
     while (k) {
-        if (k & 1u) r = (r * b) % kM;
-        b = (b * b) % kM;
+        if (k & 1u) r = pm_mod(r * b);
+        b = pm_mod(b * b);
         k >>= 1;
     }
-    return (r * x0) % kM;
+    return pm_mod(r * x0);
 }
 
 // measures and the initial graph (par_coarsen.c:2230-2400, IndepSetInit with
@@ -208,40 +256,38 @@ __global__ __launch_bounds__(kThreads) void k_pmis_set(int32_t n, const double *
 }
 
 // C and F points (par_coarsen.c:2583-2666): a graph node of measure < 1 is F;
-// a node outside the set that depends on a C point is F
+// a node outside the set that depends on a C point is F.  Then the subgraph
+// update (:2690-2760): decided nodes leave, *any = 1 if one stays.  (A row's
+// measure is read and written by its own thread only.)  Clears `lost` for the
+// next pass.
 __global__ __launch_bounds__(kThreads) void k_pmis_cf(int32_t n, const int32_t *__restrict__ SI,
                                                      const int32_t *__restrict__ SJ,
-                                                     const double *__restrict__ measure,
-                                                     int32_t *__restrict__ cf) {
+                                                     double *__restrict__ measure,
+                                                     int32_t *__restrict__ cf,
+                                                     int32_t *__restrict__ lost,
+                                                     int32_t *__restrict__ any) {
     const int i = blockIdx.x * kThreads + threadIdx.x;
     if (i >= n) return;
     const double mi = measure[i];
     if (!(mi > 0)) return;
-    if (mi < 1) cf[i] = -1;
-    if (cf[i] > 0) return;
-    for (int p = SI[i]; p < SI[i + 1]; ++p)
-        if (cf[SJ[p]] > 0) {
-            cf[i] = -1;
-            break;
-        }
-}
-
-// subgraph update (par_coarsen.c:2690-2760)
-__global__ __launch_bounds__(kThreads) void k_pmis_update(int32_t n, double *__restrict__ measure,
-                                                         const int32_t *__restrict__ cf,
-                                                         int32_t *__restrict__ any) {
-    const int i = blockIdx.x * kThreads + threadIdx.x;
-    if (i >= n) return;
-    if (!(measure[i] > 0)) return;
-    if (cf[i] != 0) measure[i] = 0.0;
+    lost[i] = 0;
+    int c = cf[i];
+    if (mi < 1) cf[i] = c = -1;
+    if (c <= 0) {
+        for (int p = SI[i]; p < SI[i + 1]; ++p)
+            if (cf[SJ[p]] > 0) {
+                cf[i] = c = -1;
+                break;
+            }
+    }
+    if (c != 0) measure[i] = 0.0;
     else *any = 1;
 }
 
-__global__ __launch_bounds__(kThreads) void k_is_coarse(int32_t n, const int32_t *__restrict__ cf,
-                                                       int32_t *__restrict__ flag) {
-    const int i = blockIdx.x * kThreads + threadIdx.x;
-    if (i < n) flag[i] = cf[i] >= 0 ? 1 : 0;
-}
+struct NotCoarse {
+    const int32_t *cf;
+    __device__ int64_t operator()(int i) const { return cf[i] >= 0 ? 0 : 1; }
+};
 
 // ---- extended+i interpolation (par_lr_interp.c:1025-1928, one process) -----------
 // upper bound of a row's entries: 1 for C, 0 for isolated, else the strong C
@@ -1507,14 +1553,16 @@ int amgt_amg_pmis(int32_t n, const int32_t *S_i, const int32_t *S_j, int cf_init
     *n_coarse = 0;
     if (n == 0) return AMGT_OK;
     Tmp tmp(s);
-    int32_t *cnt = nullptr, *lost = nullptr, *any = nullptr, *flag = nullptr, *scan = nullptr;
+    // one flag per pass: whether a node stayed undecided
+    constexpr int kFlags = 64;
+    int32_t *cnt = nullptr, *lost = nullptr, *any = nullptr;
     double *measure = nullptr;
-    AMGT_TRY(tmp.get(&cnt, n));
-    AMGT_TRY(tmp.get(&lost, n));
-    AMGT_TRY(tmp.get(&any, 1));
+    AMGT_TRY(tmp.get(&cnt, size_t(n) * 2));  // cnt and lost, cleared together
+    lost = cnt + n;
+    AMGT_TRY(tmp.get(&any, kFlags));
     AMGT_TRY(tmp.get(&measure, n));
-    AMGT_HIP(hipMemsetAsync(cnt, 0, sizeof(int32_t) * size_t(n), s));
-    AMGT_HIP(hipMemsetAsync(any, 0, sizeof(int32_t), s));
+    AMGT_HIP(hipMemsetAsync(cnt, 0, sizeof(int32_t) * 2 * size_t(n), s));
+    AMGT_HIP(hipMemsetAsync(any, 0, sizeof(int32_t) * kFlags, s));
     const dim3 g(grid_of(n)), b(kThreads);
     hipLaunchKernelGGL(k_col_count, g, b, 0, s, n, S_i, S_j, cnt);
     if (cf_init == 1)
@@ -1522,34 +1570,49 @@ int amgt_amg_pmis(int32_t n, const int32_t *S_i, const int32_t *S_j, int cf_init
     else
         hipLaunchKernelGGL(k_pmis_init, g, b, 0, s, n, S_i, cnt, measure, cf_marker, any);
     AMGT_HIP(hipGetLastError());
-    int32_t h_any = 0;
-    const Readback rb_any[1] = {{&h_any, any, sizeof(int32_t)}};
-    AMGT_TRY(readback(rb_any, 1, s));
-    // every pass decides at least the nodes of largest measure, so the loop
-    // ends within n passes
-    for (int iter = 0; h_any && iter <= n; ++iter) {
+    // Every pass decides at least the nodes of largest measure, so the loop
+    // ends within n passes.  A pass after the last one changes nothing, so on
+    // small levels, where waiting for the flag costs more than a pass, every
+    // second flag is read (and none after the start: an empty graph is as good
+    // as any).
+    const int per_check = n <= 65536 ? 2 : 1;
+    int32_t h_any = 1;
+    if (per_check == 1) {
+        const Readback rb[1] = {{&h_any, any, sizeof(int32_t)}};
+        AMGT_TRY(readback(rb, 1, s));
+    }
+    int flag = 0;  // the last pass's flag
+    for (int64_t iter = 0; h_any && iter <= int64_t(n) + 1; ++iter) {
         if (!cf_init || iter) {
-            AMGT_HIP(hipMemsetAsync(lost, 0, sizeof(int32_t) * size_t(n), s));
             hipLaunchKernelGGL(k_pmis_clear, g, b, 0, s, n, S_i, S_j, measure, lost);
             hipLaunchKernelGGL(k_pmis_set, g, b, 0, s, n, measure, lost, cf_marker);
         }
-        hipLaunchKernelGGL(k_pmis_cf, g, b, 0, s, n, S_i, S_j, measure, cf_marker);
-        AMGT_HIP(hipMemsetAsync(any, 0, sizeof(int32_t), s));
-        hipLaunchKernelGGL(k_pmis_update, g, b, 0, s, n, measure, cf_marker, any);
+        if (++flag == kFlags) {
+            AMGT_HIP(hipMemsetAsync(any, 0, sizeof(int32_t) * kFlags, s));
+            flag = 0;
+        }
+        hipLaunchKernelGGL(k_pmis_cf, g, b, 0, s, n, S_i, S_j, measure, cf_marker, lost,
+                           any + flag);
         AMGT_HIP(hipGetLastError());
-        AMGT_TRY(readback(rb_any, 1, s));
+        if (iter % per_check == per_check - 1) {
+            const Readback rb[1] = {{&h_any, any + flag, sizeof(int32_t)}};
+            AMGT_TRY(readback(rb, 1, s));
+        }
     }
     if (h_any) {
         set_error("PMIS did not converge");
         return AMGT_ERR_INPUT;
     }
-    AMGT_TRY(tmp.get(&flag, n));
-    AMGT_TRY(tmp.get(&scan, size_t(n) + 1));
-    hipLaunchKernelGGL(k_is_coarse, g, b, 0, s, n, cf_marker, flag);
-    AMGT_HIP(hipGetLastError());
-    AMGT_TRY(exclusive_scan_i32(flag, scan, n, s));
-    const Readback rb[1] = {{n_coarse, scan + n, sizeof(int32_t)}};
-    return readback(rb, 1, s);
+    rowpass::Part *parts = nullptr;
+    RowStats *tot = nullptr;
+    RowStats ht{};
+    AMGT_TRY(tmp.get(&parts, size_t(rowpass::groups(n))));
+    AMGT_TRY(tmp.get(&tot, 1));
+    AMGT_TRY(rowpass::count(n, NotCoarse{cf_marker}, 0, 0, parts, tot, s));
+    const Readback rb[1] = {{&ht, tot, sizeof(RowStats)}};
+    AMGT_TRY(readback(rb, 1, s));
+    *n_coarse = ht.cnt[0];
+    return AMGT_OK;
 }
 
 int amgt_amg_extpi_interp(int32_t n, const int32_t *A_i, const int32_t *A_j,
