@@ -72,7 +72,7 @@ def interpolation_batched(grids, device):
     being a zero Dirichlet value.  Up to 8 entries per row, ascending columns,
     no stored zeros.  Returns (I, J, A, ncoarse, coarse grids)."""
     import ctypes
-    from .mbsr import _stream_ptr, copy_from_device_ptr
+    from .mbsr import _stream_ptr, copies_from_device_ptrs
     flat = (ctypes.c_int32 * (3 * len(grids)))(*[int(v) for g in grids for v in g])
     nf, nc, nnz = ctypes.c_int32(), ctypes.c_int32(), ctypes.c_int64()
     pi, pj, pa = ctypes.c_void_p(), ctypes.c_void_p(), ctypes.c_void_p()
@@ -80,9 +80,9 @@ def interpolation_batched(grids, device):
                                            ctypes.byref(nnz), ctypes.byref(pi), ctypes.byref(pj),
                                            ctypes.byref(pa), _stream_ptr(None)),
             "amgt_interp_trilinear")
-    I = copy_from_device_ptr(pi.value, nf.value + 1, torch.int32, device)
-    J = copy_from_device_ptr(pj.value, nnz.value, torch.int32, device)
-    A = copy_from_device_ptr(pa.value, nnz.value, torch.float64, device)
+    I, J, A = copies_from_device_ptrs([(pi.value, nf.value + 1, torch.int32),
+                                       (pj.value, nnz.value, torch.int32),
+                                       (pa.value, nnz.value, torch.float64)], device)
     cgrids = [tuple((int(x) + 1) // 2 for x in gr) for gr in grids]
     return I, J, A, int(nc.value), cgrids
 

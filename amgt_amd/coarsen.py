@@ -16,7 +16,7 @@ import ctypes
 import torch
 
 from . import _lib as L
-from .mbsr import _stream_ptr, copy_from_device_ptr
+from .mbsr import _stream_ptr, copies_from_device_ptrs
 
 
 def _p(t: torch.Tensor | None) -> ctypes.c_void_p:
@@ -45,8 +45,8 @@ def strength(n: int, I: torch.Tensor, J: torch.Tensor, A: torch.Tensor, theta: f
     L.check(lib.amgt_amg_strength(n, _p(I), _p(J), _p(A), float(theta), float(max_row_sum),
                                   ctypes.byref(nnz), ctypes.byref(si), ctypes.byref(sj),
                                   _stream_ptr(stream)), "amgt_amg_strength")
-    SI = copy_from_device_ptr(si.value, n + 1, torch.int32, I.device, stream)
-    SJ = copy_from_device_ptr(sj.value, nnz.value, torch.int32, I.device, stream)
+    SI, SJ = copies_from_device_ptrs([(si.value, n + 1, torch.int32),
+                                      (sj.value, nnz.value, torch.int32)], I.device, stream)
     return SI, SJ
 
 
@@ -108,9 +108,9 @@ def extpi_interp(n: int, I: torch.Tensor, J: torch.Tensor, A: torch.Tensor, SI: 
                                       int(max_elmts), ctypes.byref(nc), ctypes.byref(nnz),
                                       ctypes.byref(pi), ctypes.byref(pj), ctypes.byref(pa),
                                       _stream_ptr(stream)), "amgt_amg_extpi_interp")
-    PI = copy_from_device_ptr(pi.value, n + 1, torch.int32, I.device, stream)
-    PJ = copy_from_device_ptr(pj.value, nnz.value, torch.int32, I.device, stream)
-    PA = copy_from_device_ptr(pa.value, nnz.value, torch.float64, I.device, stream)
+    PI, PJ, PA = copies_from_device_ptrs([(pi.value, n + 1, torch.int32),
+                                          (pj.value, nnz.value, torch.int32),
+                                          (pa.value, nnz.value, torch.float64)], I.device, stream)
     return PI, PJ, PA, int(nc.value)
 
 
@@ -128,7 +128,7 @@ def rap_host_order(n: int, nc: int, I: torch.Tensor, J: torch.Tensor, A: torch.T
                                         ctypes.byref(nnz), ctypes.byref(ci), ctypes.byref(cj),
                                         ctypes.byref(ca), _stream_ptr(stream)),
             "amgt_amg_rap_host_order")
-    CI = copy_from_device_ptr(ci.value, nc + 1, torch.int32, I.device, stream)
-    CJ = copy_from_device_ptr(cj.value, nnz.value, torch.int32, I.device, stream)
-    CA = copy_from_device_ptr(ca.value, nnz.value, torch.float64, I.device, stream)
+    CI, CJ, CA = copies_from_device_ptrs([(ci.value, nc + 1, torch.int32),
+                                          (cj.value, nnz.value, torch.int32),
+                                          (ca.value, nnz.value, torch.float64)], I.device, stream)
     return CI, CJ, CA

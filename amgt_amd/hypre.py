@@ -24,7 +24,7 @@ import ctypes
 import torch
 
 from . import _lib as L
-from .mbsr import MBSRMatrix, _need_cuda, _ptr, _stream_ptr, copy_from_device_ptr
+from .mbsr import MBSRMatrix, _need_cuda, _ptr, _stream_ptr, copies_from_device_ptrs
 
 AMGT_DOUBLE = L.AMGT_DOUBLE
 AMGT_FLOAT = L.AMGT_FLOAT
@@ -114,9 +114,11 @@ def hypreDevice_CSRSpGemm(A: CSRMatrix, B: CSRMatrix, stream=None) -> CSRMatrix:
         ctypes.byref(cache), _stream_ptr(stream))
     L.check(st, "hypreDevice_CSRSpGemm")
     dev = A.i.device
-    I = copy_from_device_ptr(ci.value, A.num_rows + 1, torch.int32, dev, stream)
-    J = copy_from_device_ptr(cj.value, nnzC.value, torch.int32, dev, stream)
-    D = copy_from_device_ptr(cd.value, nnzC.value, torch.float64, dev, stream) if cd.value else None
+    items = [(ci.value, A.num_rows + 1, torch.int32), (cj.value, nnzC.value, torch.int32)]
+    if cd.value:
+        items.append((cd.value, nnzC.value, torch.float64))
+    I, J, *D = copies_from_device_ptrs(items, dev, stream)
+    D = D[0] if D else None
     C = CSRMatrix(I, J, D, A.num_rows, B.num_cols)
     C.bsr_mat = cache
     C.coasen_level = A.coasen_level

@@ -71,21 +71,32 @@ def _need_rows_len(t, name, k, n, device):
         raise ValueError(f"{name} has shape {tuple(t.shape)}, ({k}, >= {n}) needed")
 
 
+def copies_from_device_ptrs(items, device, stream=None, free=True):
+    """Copies of library-owned device arrays, items = (pointer, entries, dtype),
+    as new tensors.  With `free` the arrays are given back to the library allocator: one synchronisation
+    after all the copies, none without."""
+    out = []
+    sp = _stream_ptr(stream)
+    for ptr, n, dtype in items:
+        t = torch.empty(n, dtype=dtype, device=device)
+        if n and ptr:
+            rc = L.hip().hipMemcpyAsync(ctypes.c_void_p(t.data_ptr()), ctypes.c_void_p(ptr),
+                                        n * t.element_size(), L.HIP_MEMCPY_D2D, sp)
+            if rc != 0:
+                raise RuntimeError(f"hipMemcpyAsync failed ({rc})")
+        out.append(t)
+    if free and any(ptr for ptr, _, _ in items):
+        torch.cuda.current_stream().synchronize() if stream is None else stream.synchronize()
+        for ptr, _, _ in items:
+            if ptr:
+                L.check(L.load().amgt_free(ctypes.c_void_p(ptr)), "amgt_free")
+    return out
+
+
 def copy_from_device_ptr(ptr: int, n: int, dtype, device, stream=None, free=True):
     """Copies n elements at a library-owned device pointer into a new tensor and
     (optionally) frees the pointer through the library allocator."""
-    out = torch.empty(n, dtype=dtype, device=device)
-    sp = _stream_ptr(stream)
-    if n and ptr:
-        nbytes = n * out.element_size()
-        rc = L.hip().hipMemcpyAsync(ctypes.c_void_p(out.data_ptr()), ctypes.c_void_p(ptr), nbytes,
-                                    L.HIP_MEMCPY_D2D, sp)
-        if rc != 0:
-            raise RuntimeError(f"hipMemcpyAsync failed ({rc})")
-    if free and ptr:
-        torch.cuda.current_stream().synchronize() if stream is None else stream.synchronize()
-        L.check(L.load().amgt_free(ctypes.c_void_p(ptr)), "amgt_free")
-    return out
+    return copies_from_device_ptrs([(ptr, n, dtype)], device, stream, free)[0]
 
 
 class MBSRMatrix:
@@ -356,10 +367,11 @@ class MBSRMatrix:
                                        ctypes.byref(pi), ctypes.byref(pj), ctypes.byref(pv))
         L.check(st, "amgt_mbsr_to_csr")
         nrows = self.info()["nrows"]
-        I = copy_from_device_ptr(pi.value, nrows + 1, torch.int32, self.device, stream)
-        J = copy_from_device_ptr(pj.value, nnz.value, torch.int32, self.device, stream)
-        V = (copy_from_device_ptr(pv.value, nnz.value, torch.float64, self.device, stream)
-             if pv.value else None)
+        items = [(pi.value, nrows + 1, torch.int32), (pj.value, nnz.value, torch.int32)]
+        if pv.value:
+            items.append((pv.value, nnz.value, torch.float64))
+        I, J, *V = copies_from_device_ptrs(items, self.device, stream)
+        V = V[0] if V else None
         return I, J, V
 
 
