@@ -172,24 +172,56 @@ int tmp_alloc(void **p, size_t bytes, hipStream_t s) {
 
 void tmp_free(void *p, hipStream_t s) { pool_free(p, s); }
 
+// The items' words, gathered into the pinned area (mapped memory; visible to
+// the host after the stream synchronisation).
+namespace {
+constexpr int kReadItems = 4;
+struct ReadArgs {
+    const uint32_t *src[kReadItems];
+    int32_t end[kReadItems];   // words up to and including the item
+    int32_t off[kReadItems];   // the item's first word in the area
+};
+__global__ __launch_bounds__(64) void k_readback(ReadArgs a, uint32_t *__restrict__ area) {
+    for (int w = threadIdx.x; w < a.end[kReadItems - 1]; w += 64) {
+        int k = 0;
+        while (w >= a.end[k]) ++k;
+        const int at = w - (k ? a.end[k - 1] : 0);
+        area[a.off[k] + at] = a.src[k][at];
+    }
+}
+}  // namespace
+
 int readback(const Readback *items, int n, hipStream_t s) {
     // one pinned area per host thread, allocated on first use, kept for the process
+    // (portable: every GPU of the process may write it)
     thread_local unsigned char *area = nullptr;
     if (!area) {
         void *p = nullptr;
-        AMGT_HIP(hipHostMalloc(&p, kReadbackBytes, hipHostMallocDefault));
+        AMGT_HIP(hipHostMalloc(&p, kReadbackBytes, hipHostMallocPortable | hipHostMallocMapped));
         area = static_cast<unsigned char *>(p);
     }
+    uint32_t *dev_area = nullptr;
+    AMGT_HIP(hipHostGetDevicePointer(reinterpret_cast<void **>(&dev_area), area, 0));
+    // One small kernel gathers the items: an asynchronous copy per item costs a
+    // launch of its own each.
+    ReadArgs ra{};
     size_t off = 0;
+    int32_t words = 0;
     for (int k = 0; k < n; ++k) {
         const size_t b = items[k].bytes;
-        if (off + b > kReadbackBytes) {
-            set_error("readback: more than kReadbackBytes requested");
+        if (off + b > kReadbackBytes || k >= kReadItems || (b & 3) != 0) {
+            set_error("readback: more than kReadbackBytes or items requested");
             return AMGT_ERR_ARG;
         }
-        AMGT_HIP(hipMemcpyAsync(area + off, items[k].src, b, hipMemcpyDeviceToHost, s));
+        words += int32_t(b / 4);
+        ra.src[k] = static_cast<const uint32_t *>(items[k].src);
+        ra.end[k] = words;
+        ra.off[k] = int32_t(off / 4);
         off = (off + b + 15) & ~size_t(15);
     }
+    for (int k = n; k < kReadItems; ++k) ra.end[k] = words;
+    hipLaunchKernelGGL(k_readback, dim3(1), dim3(64), 0, s, ra, dev_area);
+    AMGT_HIP(hipGetLastError());
     AMGT_HIP(hipStreamSynchronize(s));
     off = 0;
     for (int k = 0; k < n; ++k) {

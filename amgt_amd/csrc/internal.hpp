@@ -89,11 +89,12 @@ int tmp_alloc_t(T **p, size_t n, hipStream_t s) {
     return tmp_alloc(reinterpret_cast<void **>(p), sizeof(T) * (n ? n : 1), s);
 }
 
-// Device->host readbacks of sizes and counters, all at once: each item is
-// copied into a pinned per-thread staging area, one stream synchronisation
-// covers them, then they are copied to their destinations.  (A copy into
-// pageable memory waits for the stream and stages through a driver buffer
-// on its own: about 12 us each on MI355X, against one sync for a batch.)
+// Device->host readbacks of sizes and counters, all at once: a small kernel
+// gathers the items (at most four, whole 4-byte words) into a pinned
+// per-thread staging area, one stream synchronisation covers them, then they
+// are copied to their destinations.  (A copy into pageable memory waits for
+// the stream and stages through a driver buffer on its own: about 12 us each
+// on MI355X; asynchronous copies into pinned memory still cost a launch each.)
 // At most kReadbackBytes in total; every caller synchronises before it
 // returns, so the area is free again.
 struct Readback {
