@@ -327,23 +327,27 @@ __device__ __forceinline__ double round_out<double>(double x) {
 //
 // rows / ub_off NULL: the bounded form, every block row 0 .. count-1, where the
 // host's bound (stride = largest A row times largest B row, at most 64) holds
-// every row's products.  The workgroup's rows share its part of the temporaries
-// and pack their blocks there, row i from loc[i] on (CSlots): with a slot of
-// `stride` entries per row the ten blocks of an average row cost several cache
-// lines each way.  A row
-// that breaks the bound writes no structure and a block count of -1, which
+// every row's products: row i has a slot of `stride` entries.  Where the row
+// kernel of the numeric pass follows (loc not NULL), a wave's rows pack their
+// blocks instead, row i from loc[i] on (CSlots): the ten blocks of an average
+// row in a slot of 28 cost several cache lines each way (A P on 7-pt 128^3:
+// numeric pass 500 -> 385 us, symbolic pass + 13); the MFMA kernel, one row per
+// wave, only waits for loc (+ 15 to 30 us at 200000 block rows).  A row that breaks the bound writes no structure and a block count of -1, which
 // the size pass reports as an error.
 constexpr int kSymRegRows = 2;  // rows per wave of k_symbolic_reg
 constexpr int kSymWgRows = 4 * kSymRegRows;  // rows per workgroup
 
 // Where the symbolic pass left a block row's C blocks: at ub_off[i], or in the
-// bounded form at loc[i] in the part of the row's workgroup.
+// bounded form (ub_off NULL) in the row's slot, or packed at loc[i] of the slots
+// of the rows that shared a wave.
 struct CSlots {
     const int64_t *ub_off;
     uint16_t *loc;
     int32_t stride;
     __device__ __forceinline__ int64_t at(int i) const {
-        return ub_off ? ub_off[i] : int64_t(i / kSymRegRows) * kSymRegRows * stride + loc[i];
+        if (ub_off) return ub_off[i];
+        if (!loc) return int64_t(i) * stride;
+        return int64_t(i / kSymRegRows) * kSymRegRows * stride + loc[i];
     }
 };
 template <int RPW>
@@ -508,6 +512,8 @@ __global__ __launch_bounds__(256) void k_symbolic_reg(int count, const int32_t *
         int64_t slot;
         if (ub_off) {
             slot = ub_off[i[u]];
+        } else if (!slots.loc) {
+            slot = int64_t(i[u]) * stride;
         } else {
             if (lane == 0) slots.loc[i[u]] = uint16_t(at);
             slot = int64_t(r0) * stride + at;
@@ -2009,17 +2015,24 @@ __global__ __launch_bounds__(256) void k_scale_values(int64_t n, double f, doubl
     if (i < n) v[i] *= f;
 }
 
-// Lanes per row of k_numeric_rows for this product, 0 where k_numeric_outer
-// runs instead: rows of more than 16 A blocks or 256 C values, which the row's
-// LDS does not hold, and denser blocks (over 6 of 16 entries), where most of
-// the MFMA's products exist and its one instruction per four blocks wins.
-// Measured at 2 to 4 entries per block: A P of 7-pt 128^3 with trilinear P 385
-// against 566 us, with a PMIS-like P on 101 x 99 x 97 267 against 354 us.  B's
-// block rows of at most 4 blocks on average leave half of eight lanes idle.
-int numeric_rows_lanes(const Mbsr &A, const Mbsr &B, int32_t max_values) {
-    if (A.max_row_blocks > kRowsA || max_values > 256 || A.nblk == 0 || B.nblk == 0) return 0;
+// Lanes per row of k_numeric_rows for this FP64 product, 0 where
+// k_numeric_outer runs instead.  A row's LDS holds 16 A blocks.  The row kernel
+// pays per scalar product (about pa * pb of them per scalar row; twice with 8
+// lanes, which put 2 instead of 4 rows in a wave), the MFMA kernel a fixed part
+// and its steps of four blocks per A block, so the line rises with A's blocks.
+// B's block rows of at most 4 blocks leave half of eight lanes idle.  Measured,
+// product of 200000 block rows with itself, rows / MFMA kernel in us: 3 blocks
+// of 2, 4, 5, 6, 8 entries 259/318, 281/317, 294/318, 332/317, 338/315 (line at
+// 5.7 entries); 5 blocks 339/382, 412/392, 442/394, 533/398, 620/420 (3.3);
+// 7 blocks of 2, 4, 6 entries 391/430, 554/454, 686/488 (2.5); numeric pass of
+// A P on 7-pt 128^3, trilinear P (23 products per scalar row, 4 lanes) 385/566.
+int numeric_rows_lanes(const Mbsr &A, const Mbsr &B) {
+    if (A.max_row_blocks > kRowsA || A.nblk == 0 || B.nblk == 0) return 0;
     if (A.avg_nnz > 6.0 || B.avg_nnz > 6.0) return 0;
-    return B.nblk <= 4 * int64_t(B.brow) ? 4 : 8;
+    const int lanes = B.nblk <= 4 * int64_t(B.brow) ? 4 : 8;
+    const double pa = double(A.nnz) / (4.0 * A.brow), pb = double(B.nnz) / (4.0 * B.brow);
+    const double blocks = double(A.nblk) / A.brow;
+    return pa * pb <= (lanes == 4 ? 16.0 : 11.0) + 1.25 * blocks ? lanes : 0;
 }
 
 // numeric kernels of one value precision; *nslab receives the global slab of
@@ -2032,13 +2045,13 @@ int launch_numeric(const SpgemmArgs &g, const Mbsr &A, const Mbsr &B, const int3
                    const Mbsr &C, int32_t brow,
                    const int32_t *list, int32_t reg_rows, int32_t lds_rows, int32_t big_rows,
                    const CSlots &slots, const int32_t *tcol, const uint32_t *tmap,
-                   const int32_t *big, double **nslab, hipStream_t s) {
+                   const int32_t *big, int rows_l, double **nslab, hipStream_t s) {
     if (reg_rows > 0) {
         if constexpr (std::is_same<VT, double>::value) {
             // accumulators for the bin's longest C row (at most 64 blocks)
             const dim3 grid((reg_rows + 3) / 4);
-            const int rows_l = numeric_rows_lanes(A, B, big[3]);
-            if (rows_l > 0) {
+            // (C rows over 256 values do not fit the row kernel's LDS)
+            if (rows_l > 0 && big[3] <= 256) {
                 const int per = 256 / (4 * rows_l);
                 const dim3 rgrid((reg_rows + per - 1) / per);
 #define AMGT_NUMERIC_ROWS(L_, P_, V_)                                                          \
@@ -2215,7 +2228,11 @@ int spgemm(const Mbsr &A, const Mbsr &B, int precision, hipStream_t s, Mbsr *Cp)
     SG_TRY(tmp_alloc_t(&list, size_t(brow) * 3 + 1, s));
     SG_TRY(tmp_alloc_t(&ccnt, size_t(brow) + 1, s));
     SG_TRY(tmp_alloc_t(&cnnz, size_t(brow) + 1, s));
-    if (bounded) SG_TRY(tmp_alloc_t(&loc, size_t(brow), s));
+    // lanes of the FP64 row kernel, 0: another kernel
+    const int rows_l = !C.pattern_only && precision != AMGT_FLOAT && precision != AMGT_HALF
+                           ? numeric_rows_lanes(A, B)
+                           : 0;
+    if (bounded && rows_l > 0) SG_TRY(tmp_alloc_t(&loc, size_t(brow), s));
     int64_t total_ub = 0;
     const int32_t *bin = ht.cnt;
     if (bounded) {
@@ -2381,17 +2398,17 @@ int spgemm(const Mbsr &A, const Mbsr &B, int precision, hipStream_t s, Mbsr *Cp)
     if (!C.pattern_only && brow > 0) {
         switch (precision) {
             case AMGT_FLOAT:
-                st = launch_numeric<float>(g, A, B, boff, C, brow, list, reg_rows, lds_rows, big_rows, slots, tcol, tmap, ct.big, &nslab, s);
+                st = launch_numeric<float>(g, A, B, boff, C, brow, list, reg_rows, lds_rows, big_rows, slots, tcol, tmap, ct.big, rows_l, &nslab, s);
                 break;
             case AMGT_HALF:
-                st = launch_numeric<__half>(g, A, B, boff, C, brow, list, reg_rows, lds_rows, big_rows, slots, tcol, tmap, ct.big, &nslab, s);
+                st = launch_numeric<__half>(g, A, B, boff, C, brow, list, reg_rows, lds_rows, big_rows, slots, tcol, tmap, ct.big, rows_l, &nslab, s);
                 // the FP16 copies hold A and B times half_scale: undo both (powers of two, exact)
                 if (st == AMGT_OK && C.nnz > 0)
                     hipLaunchKernelGGL(k_scale_values, dim3(unsigned((C.nnz + 255) / 256)), dim3(256),
                                        0, s, C.nnz, 1.0 / (A.half_scale * B.half_scale), C.val);
                 break;
             default:
-                st = launch_numeric<double>(g, A, B, boff, C, brow, list, reg_rows, lds_rows, big_rows, slots, tcol, tmap, ct.big, &nslab, s);
+                st = launch_numeric<double>(g, A, B, boff, C, brow, list, reg_rows, lds_rows, big_rows, slots, tcol, tmap, ct.big, rows_l, &nslab, s);
         }
         if (st != AMGT_OK) {
             cleanup();

@@ -115,6 +115,48 @@ def test_spgemm_register_bound(dev, kb_b):
     assert GC.info()["max_row_blocks"] == int(cnt.max())
 
 
+def _filled_blocks_csr(nbr, nbc, counts, fill, seed, cut=0):
+    """CSR of 4 nbr - cut rows: block row i has counts(i) blocks of fill(i) entries."""
+    rng = np.random.default_rng(seed)
+    rows, cols = [], []
+    for i in range(nbr):
+        for bc in rng.permutation(nbc)[:counts(i)]:
+            e = rng.permutation(16)[:fill(i)]
+            rows.append(4 * i + e // 4)
+            cols.append(4 * int(bc) + e % 4)
+    m = 4 * nbr - cut
+    r, c = np.concatenate(rows), np.concatenate(cols)
+    keep = r < m
+    S = sp.csr_matrix((rng.uniform(-1.0, 1.0, int(keep.sum())), (r[keep], c[keep])),
+                      shape=(m, 4 * nbc))
+    S.sort_indices()
+    return S.indptr.astype(np.int32), S.indices.astype(np.int32), S.data
+
+
+# (A: longest block row, entries per block, entries per block of row 5; B: longest
+# block row, entries per block, blocks of row 3)
+@pytest.mark.parametrize("ca,fa,fa5,cb,fb,cb3", [
+    (8, 2, 2, 4, 1, 4),     # 4 lanes, at most 32 products
+    (16, 1, 1, 4, 2, 4),    # 4 lanes, 16 A blocks, 64 products
+    (16, 1, 16, 4, 2, 4),   # one row over the A values staged, C row over 64 values
+    (16, 1, 16, 4, 5, 4),   # ... over 128 values
+    (16, 1, 16, 4, 5, 0),   # ... an empty B row
+    (9, 1, 1, 7, 2, 7),     # 8 lanes, 63 products
+    (9, 1, 16, 7, 3, 7),    # 8 lanes, C row over 256 values: the MFMA kernel
+    (5, 2, 2, 4, 2, 20),    # rows by list (100 products possible)
+    (17, 1, 1, 3, 1, 3),    # 17 A blocks: the MFMA kernel
+    (3, 5, 5, 3, 5, 3),     # below the line of 3-block rows
+    (3, 6, 6, 3, 6, 3),     # above it
+])
+def test_spgemm_short_sparse_rows(dev, ca, fa, fa5, cb, fb, cb3):
+    AI, AJ, AA = _filled_blocks_csr(67, 41, lambda i: ca if i == 5 else i % (ca + 1),
+                                    lambda i: fa5 if i == 5 else fa, 21, cut=3)
+    BI, BJ, BA = _filled_blocks_csr(41, 53, lambda i: cb3 if i == 3 else cb - i % 2,
+                                    lambda i: fb, 22)
+    check_product(dev, 4 * 67 - 3, 4 * 41, 4 * 53, AI, AJ, AA, BI, BJ, BA,
+                  f"short rows {ca}x{fa} {cb}x{fb}")
+
+
 def test_spgemm_stencils(dev):
     for kind, dims in [(7, (10, 9, 8)), (27, (7, 6, 5)), (7, (33, 31, 1)), (9, (20, 17, 1))]:
         I, J, A = W.stencil(kind, *dims)
