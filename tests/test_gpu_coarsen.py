@@ -191,6 +191,40 @@ def test_extpi_wave_tiers_match_oracle(dev, n, per_row):
     assert np.array_equal(PA.cpu().numpy(), rPA)
 
 
+@pytest.mark.parametrize("per_row", [7, 8, 15, 16, 31, 32])
+@pytest.mark.parametrize("mixed", [False, True])
+def test_extpi_group_edges_match_oracle(dev, per_row, mixed):
+    """Rows of exactly 8, 9, 16, 17, 32 and 33 entries: the last and the first
+    rows of the 8-, 16- and 32-lane kernels (mixed: beside tridiagonal rows, so
+    that few rows of a workgroup are theirs); random columns overflow their
+    candidate tables.  P unlimited and truncated equals the oracle's exactly."""
+    n = 1501
+    I, J, A = _rand_long(n, per_row, per_row)
+    if mixed:
+        M = sp.csr_matrix((A, J, I), shape=(n, n)).tolil()
+        T3 = sp.diags([-1.0, 2.5, -1.0], [-1, 0, 1], (n, n)).tolil()
+        for i in range(n):
+            if i % 9:
+                M.rows[i], M.data[i] = T3.rows[i], T3.data[i]
+        M = M.tocsr()
+        M.sort_indices()
+        I, J, A = M.indptr.astype(np.int32), M.indices.astype(np.int32), M.data.copy()
+    print(f"[extpi groups] per_row={per_row} mixed={mixed}", flush=True)
+    dI, dJ, dA = T(I, dev), T(J, dev), T(A, dev)
+    SI, SJ = C.strength(n, dI, dJ, dA, 0.25, 0.9)
+    rSI, rSJ = O.amg_strength(n, I, J, A, 0.25, 0.9)
+    assert np.array_equal(SI.cpu().numpy(), rSI) and np.array_equal(SJ.cpu().numpy(), rSJ)
+    cf, nc = C.pmis(n, SI, SJ, 0)
+    rcf, rnc = O.amg_pmis(n, rSI, rSJ, 0)
+    assert nc == rnc and np.array_equal(cf.cpu().numpy(), rcf)
+    for pmx in (0, 4):
+        PI, PJ, PA, _ = C.extpi_interp(n, dI, dJ, dA, SI, SJ, cf, pmx)
+        rPI, rPJ, rPA, _ = O.amg_extpi(n, I, J, A, rSI, rSJ, rcf, pmx)
+        assert np.array_equal(PI.cpu().numpy(), rPI), pmx
+        assert np.array_equal(PJ.cpu().numpy(), rPJ), pmx
+        assert np.array_equal(PA.cpu().numpy(), rPA), pmx
+
+
 def test_pmis_cf_init_rejected(dev):
     import ctypes
     from amgt_amd import _lib as L

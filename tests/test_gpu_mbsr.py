@@ -454,6 +454,41 @@ def test_spmm_low_precision_and_transposed(dev, prec, tol):
         assert np.all(np.abs(Y[v] - exp) <= tol * scale)
 
 
+@pytest.mark.parametrize("prec,tol", [(L.AMGT_DOUBLE, 1e-12), (L.AMGT_FLOAT, 2e-6),
+                                      (L.AMGT_HALF, 2e-3)])
+@pytest.mark.parametrize("k", [2, 7, 16, 17, 18, 33])
+@pytest.mark.parametrize("fill", [3, 6])
+def test_spmm_block_lists(dev, prec, tol, k, fill):
+    """Block rows of 0 to 65 blocks, around the 32 block list entries of the
+    row kernel (3 entries per block) and beside it the matrix-core kernel (6):
+    both layouts, sizes not multiples of 4."""
+    rng = np.random.default_rng(fill)
+    counts = [1, 31, 0, 32, 33, 64, 65, 2, 63, 16]
+    n, m, rows, cols = 4 * 90 - 1, 4 * len(counts) - 3, [], []
+    for br, c in enumerate(counts):
+        for bc in rng.permutation(90)[:c]:
+            e = rng.permutation(16)[:fill]
+            rows += list(4 * br + e // 4)
+            cols += list(4 * int(bc) + e % 4)
+    ok = (np.array(rows) < m) & (np.array(cols) < n)
+    S = sp.csr_matrix((rng.standard_normal(len(rows))[ok],
+                       (np.array(rows)[ok], np.array(cols)[ok])), shape=(m, n))
+    I, J, A = S.indptr.astype(np.int32), S.indices.astype(np.int32), S.data
+    ref = O.csr2mbsr(m, n, I, J, A)
+    M = make(dev, m, n, I, J, A)
+    M.set_precision(prec)
+    X, B = rng.standard_normal((k, n)), rng.standard_normal((k, m))
+    Y = M.spmm(T(X, dev), alpha=-1.0, beta=1.0, B=T(B, dev)).cpu().numpy()
+    Z = torch.full((m, k), float("nan"), dtype=torch.float64, device=dev)
+    M.spmm_interleaved(T(X.T, dev), Z, alpha=-1.0, beta=1.0, B=T(B.T, dev))
+    Z = Z.cpu().numpy()
+    for v in range(k):
+        exp = O.mbsr_spmv(ref, -1.0, X[v], 1.0, B[v])
+        scale = row_scale(m, n, I, J, A, X[v], 1.0, B[v])
+        assert np.all(np.abs(Y[v] - exp) <= tol * scale), v
+        assert np.all(np.abs(Z[:, v] - exp) <= tol * scale), v
+
+
 def test_full_size_c2_spmv(dev):
     """3D 7-point 128^3 (2,097,152 rows): bit-exact structure and FP64 SpMV vs the oracle."""
     from amgt_amd import workloads as W
