@@ -100,9 +100,10 @@ struct ConvTotals {
     unsigned long long sumsq;
 };
 
-// A tile (kList: the single block rows of listed tiles, row w % kTileRows of tile
-// tiles[w / kTileRows], written to the row's own slot with its block count in
-// cnt).  Every entry's place in its block row is the number of smaller
+// A tile (kList: a tile over the capacity, in two parts: workgroup 2 k takes the
+// rows of tile tiles[k] before its last, at most start - 1 entries, workgroup
+// 2 k + 1 the last one alone, if it fits, written to its own slot with its block
+// count in rel).  Every entry's place in its block row is the number of smaller
 // keys there, counted over an LDS copy of the row's keys (four per read; rows
 // padded to a multiple of four with keys above all others).  The blocks of the
 // tile go to tmp_col / tmp_map from the tile's first entry on, packed; rel = a
@@ -117,7 +118,7 @@ __global__ __launch_bounds__(kTileThreads) void k_conv_tile(
     const int32_t *__restrict__ J, const double *__restrict__ A,
     const int32_t *__restrict__ tile_lo, const int32_t *__restrict__ tiles,
     double *__restrict__ val, int32_t *__restrict__ tmp_col,
-    uint16_t *__restrict__ tmp_map, int32_t *__restrict__ rel_or_cnt,
+    uint16_t *__restrict__ tmp_map, int32_t *__restrict__ rel,
     TilePart *__restrict__ parts, int values_only) {
     constexpr int NW = kTileThreads / 64, EPT = kTileCap / kTileThreads;
     constexpr int kPad = kTileCap + 3 * kTileRows;
@@ -131,10 +132,14 @@ __global__ __launch_bounds__(kTileThreads) void k_conv_tile(
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
     int t0, rows, part;  // first block row, block rows, index in parts
     if constexpr (kList) {
-        part = tiles[blockIdx.x / kTileRows];
-        t0 = tile_lo[part] + int(blockIdx.x % kTileRows);
-        if (t0 >= tile_lo[part + 1]) return;
-        rows = 1;
+        part = tiles[blockIdx.x >> 1];
+        t0 = tile_lo[part];
+        rows = tile_lo[part + 1] - t0 - 1;
+        if (blockIdx.x & 1) {
+            t0 += rows;
+            rows = 1;
+        }
+        if (rows <= 0 || rows > kTileRows) return;
     } else {
         part = blockIdx.x;
         t0 = tile_lo[part];
@@ -301,9 +306,9 @@ __global__ __launch_bounds__(kTileThreads) void k_conv_tile(
             const int lo = s_I[4 * br];
             return lo < n ? s_first[s_rid[lo] >> 2] : total;
         };
-        if constexpr (kList) {
+        if (kList && (blockIdx.x & 1)) {
             if (lane == 0) {
-                rel_or_cnt[t0] = total;
+                rel[t0] = total;
                 if (s_err) atomicOr(&parts[part].mx_flags, uint32_t(s_err));
             }
         } else {
@@ -315,21 +320,37 @@ __global__ __launch_bounds__(kTileThreads) void k_conv_tile(
             for (int u = 0; u < 2; ++u) {
                 const int c = max(u == 0 ? f1 - f0 : f2 - f1, 0);
                 if (2 * lane + u >= rows) continue;
-                rel_or_cnt[t0 + 2 * lane + u] = u == 0 ? f0 : f1;
+                rel[t0 + 2 * lane + u] = u == 0 ? f0 : f1;
                 sq += static_cast<unsigned long long>(c) * unsigned(c);
                 mx = max(mx, c);
             }
             for (int d = 32; d > 0; d >>= 1) sq += __shfl_xor(sq, d);
             mx = wave_incl_max(mx);
-            if (lane == 63)
-                parts[part] = TilePart{total, uint32_t(mx) << 8 | uint32_t(s_err), sq};
+            if (lane == 63) {
+                const uint32_t flags = uint32_t(mx) << 8 | uint32_t(s_err);
+                if constexpr (kList) {  // (the last row's workgroup adds its errors)
+                    parts[part].blocks = total;
+                    parts[part].sumsq = sq;
+                    atomicOr(&parts[part].mx_flags, flags);
+                } else {
+                    parts[part] = TilePart{total, flags, sq};
+                }
+            }
         }
     }
 }
 
-// ---- block rows of kTileCap + 1 to CAP entries in listed tiles: a workgroup per
-// row (workgroup w: row w % kTileRows of tile tiles[w / kTileRows]), LDS bitonic
-// sort of CAP keys.
+// ---- block rows of kTileCap + 1 to CAP entries: the last row of a listed tile
+// (no other row of a tile can be that long), a workgroup each.  Where the CSR rows
+// ascend, as they mostly do, they are four sorted runs, and an entry's place is
+// its place in its run plus the smaller keys of the other three, by binary search;
+// otherwise a bitonic sort.  Bound by the latency of the steps in one workgroup
+// (bitonic: 78 barriers for 4096 keys).  1024 threads for every length: a second
+// launch of 256 threads for up to 2048 entries follows instead of overlapping
+// (few rows of 1000 to 8000 entries, whole conversion: 525 against 441 us with the
+// bitonic sort, 327 with ranks; 1250 block rows of 1200 entries 318 -> 190, 225
+// of 3600 216 -> 160).  One workgroup per listed tile, not per row of it: those
+// rows took 5500 us when most workgroups were empty.
 template <int THREADS, int CAP>
 __global__ __launch_bounds__(THREADS) void k_sort_block(
     int32_t nrows, int32_t ncols, int32_t nnz, const int32_t *__restrict__ I,
@@ -341,11 +362,11 @@ __global__ __launch_bounds__(THREADS) void k_sort_block(
     __shared__ uint32_t s_key[CAP];
     __shared__ int32_t s_aux[CAP];  // source index, then block rank
     __shared__ int32_t s_wave_tot[THREADS / 64];
-    __shared__ int s_err;
+    __shared__ int s_err, s_descends;
+    constexpr int EPT = CAP / THREADS;
     const int t = threadIdx.x;
-    const int tile = tiles[blockIdx.x / kTileRows];
-    const int br = tile_lo[tile] + int(blockIdx.x % kTileRows);
-    if (br >= tile_lo[tile + 1]) return;
+    const int br = tile_lo[tiles[blockIdx.x] + 1] - 1;
+    if (br < 0) return;
     const int r0 = 4 * br;
     const int s = entry_at(I, r0, nnz);
     const int n = entry_at(I, min(r0 + 4, nrows), nnz) - s;
@@ -356,7 +377,7 @@ __global__ __launch_bounds__(THREADS) void k_sort_block(
     }
     int np = 64;
     while (np < n) np <<= 1;
-    if (t == 0) s_err = 0;
+    if (t == 0) s_err = s_descends = 0;
     int err = 0;
     for (int i = t; i < np; i += THREADS) {
         if (i < n) {
@@ -368,7 +389,52 @@ __global__ __launch_bounds__(THREADS) void k_sort_block(
         }
     }
     __syncthreads();
-    for (int k = 2; k <= np; k <<= 1) {
+    // ascending: every key above the one before it in its CSR row (also no duplicates)
+    for (int i = t; i < n; i += THREADS) {
+        if (i == 0) continue;
+        const uint32_t a = s_key[i - 1], b = s_key[i];
+        if (((a ^ b) & 12u) == 0u && a >= b) s_descends = 1;
+    }
+    __syncthreads();
+    if (!s_descends) {
+        int run[5];
+#pragma unroll
+        for (int q = 0; q < 5; ++q)
+            run[q] = min(max(entry_at(I, min(r0 + q, nrows), nnz) - s, 0), n);
+        uint32_t key[EPT];
+        int rank[EPT];
+#pragma unroll
+        for (int u = 0; u < EPT; ++u) {
+            const int i = t + u * THREADS;
+            key[u] = i < n ? s_key[i] : 0u;
+            rank[u] = i;
+            const int own = int(key[u] >> 2) & 3;
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                // i counts the runs before its own in full: take back their keys
+                // above, and add the smaller keys of the runs after it
+                if (i >= n || q == own) continue;
+                int lo = run[q], hi = run[q + 1];
+                while (lo < hi) {
+                    const int mid = (lo + hi) >> 1;
+                    if (s_key[mid] < key[u]) lo = mid + 1;
+                    else hi = mid;
+                }
+                rank[u] += q < own ? lo - run[q + 1] : lo - run[q];
+            }
+        }
+        __syncthreads();
+#pragma unroll
+        for (int u = 0; u < EPT; ++u) {
+            const int i = t + u * THREADS;
+            if (i < n) {
+                s_key[rank[u]] = key[u];
+                s_aux[rank[u]] = s + i;
+            }
+        }
+        __syncthreads();
+    }
+    for (int k = 2; s_descends && k <= np; k <<= 1) {
         for (int j = k >> 1; j > 0; j >>= 1) {
             for (int i = t; i < np; i += THREADS) {
                 int p = i ^ j;
@@ -438,35 +504,21 @@ __global__ __launch_bounds__(THREADS) void k_sort_block(
     if (t == 0 && s_err) atomicOr(err_out, s_err);
 }
 
-// Block counts of the rows of listed tiles (cnt) -> the tile's part and the
-// rows' first blocks within the tile, in place; a workgroup per tile.
-__global__ __launch_bounds__(64) void k_conv_list_sum(const int32_t *__restrict__ tile_lo,
-                                                      const int32_t *__restrict__ tiles,
-                                                      int32_t *__restrict__ cnt,
-                                                      TilePart *__restrict__ parts) {
-    const int t = tiles[blockIdx.x], lane = threadIdx.x;
-    int run = 0, mx = 0;
-    unsigned long long sq = 0ull;
-    for (int b0 = tile_lo[t]; b0 < tile_lo[t + 1]; b0 += 64) {
-        const int br = b0 + lane;
-        const bool in = br < tile_lo[t + 1];
-        const int c = in ? cnt[br] : 0;
-        const int incl = wave_incl_sum(c);
-        if (in) cnt[br] = run + incl - c;
-        run += __builtin_amdgcn_readlane(incl, 63);
-        mx = max(mx, c);
-        sq += static_cast<unsigned long long>(c) * unsigned(c);
-    }
-    for (int d = 32; d > 0; d >>= 1) {
-        sq += __shfl_xor(sq, d);
-        mx = max(mx, __shfl_xor(mx, d));
-    }
-    if (lane == 0) {
-        TilePart &p = parts[t];
-        p.blocks = run;
-        p.mx_flags = (p.mx_flags & 0xffu) | uint32_t(mx) << 8;
-        p.sumsq = sq;
-    }
+// Adds the last row of every listed tile (its block count in rel) to the tile's
+// part; rel then holds the row's first block within the tile.
+__global__ __launch_bounds__(kTileThreads) void k_conv_list_sum(
+    int32_t ntiles, const int32_t *__restrict__ tile_lo, const int32_t *__restrict__ tiles,
+    int32_t *__restrict__ rel, TilePart *__restrict__ parts) {
+    const int k = blockIdx.x * kTileThreads + threadIdx.x;
+    if (k >= ntiles) return;
+    const int t = tiles[k], br = tile_lo[t + 1] - 1;
+    TilePart p = parts[t];
+    const uint32_t c = uint32_t(rel[br]);
+    rel[br] = p.blocks;
+    p.blocks += int32_t(c);
+    p.sumsq += static_cast<unsigned long long>(c) * c;
+    p.mx_flags = max(p.mx_flags >> 8, c) << 8 | (p.mx_flags & 0xffu);
+    parts[t] = p;
 }
 
 // One workgroup: the tiles' first blocks, the totals and the list of the tiles
@@ -568,21 +620,14 @@ __global__ __launch_bounds__(kTileThreads) void k_conv_pack(
         val_ptr[brow] = I[nrows];
     }
     const int blocks = parts[t].blocks;
-    if (!(parts[t].mx_flags & TilePart::kOver)) {
-        const int from = I[4 * t0];
-        for (int k = threadIdx.x; k < blocks; k += kTileThreads) {
-            blk_col[to + k] = tmp_col[from + k];
-            blk_map[to + k] = tmp_map[from + k];
-        }
-        return;
-    }
-    for (int r = 0; r < rows; ++r) {  // each row in its own slot
-        const int from = I[4 * (t0 + r)], f = rel[t0 + r];
-        const int c = (r + 1 < rows ? rel[t0 + r + 1] : blocks) - f;
-        for (int k = threadIdx.x; k < c; k += kTileThreads) {
-            blk_col[to + f + k] = tmp_col[from + k];
-            blk_map[to + f + k] = tmp_map[from + k];
-        }
+    // a listed tile's last row has its blocks in its own slot
+    const bool over = (parts[t].mx_flags & TilePart::kOver) != 0u;
+    const int body = over ? rel[t0 + rows - 1] : blocks;
+    const int from = I[4 * t0], from_last = I[4 * (t0 + rows - 1)] - body;
+    for (int k = threadIdx.x; k < blocks; k += kTileThreads) {
+        const int at = (k < body ? from : from_last) + k;
+        blk_col[to + k] = tmp_col[at];
+        blk_map[to + k] = tmp_map[at];
     }
 }
 
@@ -683,18 +728,18 @@ int sort_tiles(int32_t nrows, int32_t ncols, int64_t nnz, const int32_t *I, cons
         set_error("CSR->mBSR: row pointers must ascend");
         return AMGT_ERR_INPUT;
     }
-    if (ht->over > 0) {  // the rows of the tiles over the capacity, one by one
-        const int32_t nt = ht->over;
-        const dim3 grid(unsigned(nt) * unsigned(kTileRows));
-        hipLaunchKernelGGL((k_conv_tile<true>), grid, dim3(kTileThreads), 0, s, nrows, ncols, nz, I,
-                           J, A, w.tile_lo, w.tiles, val, w.tmp_col, w.tmp_map, w.rel, w.parts,
-                           values_only);
-        hipLaunchKernelGGL((k_sort_block<1024, 8192>), grid, dim3(1024), 0, s, nrows, ncols, nz, I,
-                           J, A, w.tile_lo, w.tiles, val, w.tmp_col, w.tmp_map, w.rel,
+    if (ht->over > 0) {  // the tiles over the capacity, their last rows by themselves
+        const unsigned nt = unsigned(ht->over);
+        hipLaunchKernelGGL((k_conv_tile<true>), dim3(2 * nt), dim3(kTileThreads), 0, s, nrows,
+                           ncols, nz, I, J, A, w.tile_lo, w.tiles, val, w.tmp_col, w.tmp_map,
+                           w.rel, w.parts, values_only);
+        hipLaunchKernelGGL((k_sort_block<1024, 8192>), dim3(nt), dim3(1024), 0, s, nrows, ncols,
+                           nz, I, J, A, w.tile_lo, w.tiles, val, w.tmp_col, w.tmp_map, w.rel,
                            w.err, values_only);
         if (!values_only)
-            hipLaunchKernelGGL(k_conv_list_sum, dim3(unsigned(nt)), dim3(64), 0, s,
-                               w.tile_lo, w.tiles, w.rel, w.parts);
+            hipLaunchKernelGGL(k_conv_list_sum, dim3((nt + kTileThreads - 1) / kTileThreads),
+                               dim3(kTileThreads), 0, s, ht->over, w.tile_lo, w.tiles, w.rel,
+                               w.parts);
         AMGT_HIP(hipGetLastError());
         AMGT_TRY(totals(ends));
         if (ht->err & kErrBig) {

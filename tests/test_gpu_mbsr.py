@@ -115,6 +115,31 @@ def test_conversion_tile_edges(dev, m, n, lens):
     assert np.array_equal(M.arrays()["val"].cpu().numpy(), 2.0 * ref["val"])
 
 
+@pytest.mark.parametrize("ascending", [False, True])
+def test_conversion_tiles_of_short_and_long_rows(dev, ascending):
+    """Over a million entries in block rows of 300 beside 850, 1024, 1025 and 1900:
+    tiles over the capacity whose last block row does or does not fit one; columns
+    at random or ascending (long rows sorted by ranks)."""
+    rng = np.random.default_rng(77)
+    lens = np.array([75, 212, 256, 475] * 230 + [75, 213] * 700 + [0, 257])
+    lens = np.repeat(lens, 4)
+    lens[4 * 2 + 1] += 1  # 1025 entries
+    m, n = len(lens) - 1, 6000
+    lens = lens[:m]
+    I = np.zeros(m + 1, np.int32)
+    I[1:] = np.cumsum(lens)
+    cols = [rng.permutation(n)[:k] for k in lens]
+    J = np.concatenate([np.sort(c) if ascending else c for c in cols]).astype(np.int32)
+    A = rng.standard_normal(len(J))
+    ref = O.csr2mbsr(m, n, I, J, A)
+    M = make(dev, m, n, I, J, A)
+    assert M.info()["max_row_blocks"] == int(np.diff(ref["blk_ptr"]).max())
+    assert M.info()["stand"] == pytest.approx(O.mbsr_stats(ref)[0], rel=1e-12)
+    check_structure(M, ref)
+    M.update_values(T(I, dev), T(J, dev), T(-3.0 * A, dev))
+    assert np.array_equal(M.arrays()["val"].cpu().numpy(), -3.0 * ref["val"])
+
+
 def test_conversion_pattern_only_and_empty(dev):
     (m, n), I, J, A = CASES["rand_rect"]()
     M = make(dev, m, n, I, J, None)
