@@ -1584,14 +1584,21 @@ bool blk_tile_fits(const Mbsr &A, int rows) {
     return double(A.nblk) / brow * rows <= 460.0 && double(A.nnz) / brow * rows <= 1740.0;
 }
 
-// Whether the block kind runs its long-row kernel: rows of which eight do not
-// fit a tile.  Measured (us, FP64 / FP32 / FP16, tile of 8 rows against long):
-// coarse operators of 60 blocks a row 31.5 / 27 / 24 against 21 / 16 / 13 (62k
-// rows), 421 / 383 / 336 against 247 / 217 / 183 (1M rows); 44 blocks, 231
-// values a row 26 / 21 / 19 against 21 / 16 / 13; where eight rows fit the tile
-// wins: 43 blocks, 196 values a row 31.5 / 27 / 28 against 46 / 35 / 32.
+// Whether the block kind runs its long-row kernel: rows of which eight overflow
+// the tile of 512 blocks or 2048 values (half a standard deviation above the
+// average: neighbouring rows are alike), so that the block kernel walks global
+// memory per value, and at least 2.25 values per block: the long-row kernel pays
+// per block.  Measured (us, FP64 / FP32 / FP16, block against long-row kernel):
+// coarse operators of 60 blocks of 6.5 values a row 31.5 / 27 / 24 against
+// 21 / 16 / 13 (62k rows), 421 / 383 / 336 against 247 / 217 / 183 (1M rows);
+// 120k rows of 100 blocks of 1, 2, 3, 4 values 29, 39, 46, 55 against 42 (FP64),
+// 24, 32, 37, 43 against 30 (FP16); of 60 blocks of 1 to 4 values, which fit,
+// 17 to 18.5 / 14 to 15 / 14 to 15 against 27 / 20 / 17, and of 6, which do not,
+// 34 / 31 / 29 against 27 / 21 / 19.
 bool spmv_long_rows(const Mbsr &A, int lanes) {
-    return lanes == 64 && A.nnz >= 4 && !blk_tile_fits(A, 8);
+    if (lanes != 64 || A.nnz < 4 || A.brow <= 0 || A.nblk == 0 || A.avg_nnz < 2.25) return false;
+    const double blocks = double(A.nblk) / A.brow, spread = 1.0 + 0.5 * A.stand / blocks;
+    return 8.0 * blocks * spread > 512.0 || 8.0 * double(A.nnz) / A.brow * spread > 2048.0;
 }
 
 // y[row] = ep(row, (A x)[row]) with the handle's kernel kind and lanes setting
