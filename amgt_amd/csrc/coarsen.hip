@@ -919,7 +919,7 @@ __global__ __launch_bounds__(64) void k_extpi_wave(
 //    of the group runs the host's quicksort.
 // Issue-bound by the probe loops, which diverge: the first form, which walked
 // each lane's own columns three times (37 loops), took 1140 us on 7-pt 128^3
-// (1.5 M F rows), the thread kernel 4845 us.
+// (1.5 M F rows), this one 906, the thread kernel 4845 us.
 constexpr int kTerms = 4;  // terms of one neighbour kept in LDS
 template <int G>
 struct GroupRow {

@@ -14,8 +14,9 @@
 // kTileCap): rank sort of each row's keys in LDS, coalesced loads and stores,
 // the tile's blocks packed.  Then one workgroup scans the tiles' block counts
 // and the packed blocks are copied to their places.  Tiles over the capacity (a
-// block row of more than 256 entries) are left to a second pass, a workgroup per
-// block row (rank sort up to kTileCap entries, LDS bitonic up to 8192).
+// block row of more than 256 entries) are left to a second pass: the rows before
+// the last as a tile, the last by itself (as a tile up to kTileCap entries, a
+// workgroup of 1024 threads up to 8192).
 // Larger block rows return AMGT_ERR_UNSUPPORTED.
 #include "internal.hpp"
 #include "rowpass.hpp"

@@ -19,7 +19,8 @@
 //    v_mfma_f64_4x4x4f64 (four independent 4x4x4 products: the A block
 //    replicated, B block g in block slot g) and added to the C slots of their
 //    block columns.  A B row never repeats a block column, so the four slots
-//    are distinct: no atomics, deterministic results.
+//    are distinct: no atomics, deterministic results.  Short FP64 rows of sparse
+//    blocks instead go scalar row by scalar row (k_numeric_rows).
 // 5. accumulators are compressed to the mBSR value layout.
 #include "internal.hpp"
 #include "rowpass.hpp"

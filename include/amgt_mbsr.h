@@ -108,6 +108,7 @@ int amgt_mbsr_set_spmv_lanes(amgt_mbsr_t A, int lanes);
  *   AMGT_SPMV_STAGED    a workgroup stages its tile of block rows in LDS, lanes walk it
  *   AMGT_SPMV_BLOCK     lane per 4x4 block over an LDS-staged tile of block rows, whole
  *                       x segments, per-row partial sums reduced in LDS
+ *                       (64 lanes, long rows of filled blocks: a wave per block row)
  *   AMGT_SPMV_BALANCED  the block kernel over equal tiles of blocks whatever rows they
  *                       belong to; rows cut by tile edges are finished by a second pass
  *                       (bsr_spmv_balanced_tc_fp64 + BSR_BALANCED_PREPROCESS_GPU,
@@ -124,7 +125,8 @@ int amgt_mbsr_autotune(amgt_mbsr_t A, void *stream);
  * up to 350k with <= 8, with lanes per block row so that about 2^18 lanes share the
  * walk; else the balanced kernel when the spread of blocks per block row is >= 12
  * (tiles of 256 blocks), else the block-lane kernel with the largest tile whose average
- * load fits 90 % of its 512 blocks.  Fitted to amgt_mbsr_spmv_sweep over every
+ * load fits 90 % of its 512 blocks and, unless the blocks are nearly full, its 2048
+ * values.  Fitted to amgt_mbsr_spmv_sweep over every
  * operator of the AMG hierarchies of the benchmark configurations.  Resets settings made
  * with amgt_mbsr_set_spmv_kernel / _lanes or amgt_mbsr_autotune. */
 int amgt_mbsr_tune_from_stats(amgt_mbsr_t A);
