@@ -1577,11 +1577,18 @@ int launch_spmv_bal_g(const Mbsr &A, const BalTables &tb, const VT *val, const d
 }
 
 // Whether an average tile of `rows` block rows stays within 90 % of the block
-// kernel's 512 blocks and 85 % of its 2048 values, so that few tiles overflow to
-// its walk over global memory (the counts vary more for values).
+// kernel's 512 blocks, so that few tiles overflow to its walk over global memory,
+// and within its 2048 values (200k rows of 7 blocks of 5, 6, 8 values, tile of 64
+// against 32 rows: 35, 39, 41 against 22, 22, 24 us FP64).  No margin for the
+// values: 7-pt operators fill 1784 of 64 rows, 31 us on 128^3, 45 with 32 rows.
+// Nearly full blocks, of which a tile of 2048 values has work for less than 170
+// lanes, go by the blocks alone (7 blocks of 16 values 48 against 56 us, 14 44
+// against 58), unless eight rows overflow, where the long-row kernel is (25 blocks
+// of 16 values 47 against 32).
 bool blk_tile_fits(const Mbsr &A, int rows) {
-    const double brow = A.brow > 0 ? double(A.brow) : 1.0;
-    return double(A.nblk) / brow * rows <= 460.0 && double(A.nnz) / brow * rows <= 1740.0;
+    const double brow = A.brow > 0 ? double(A.brow) : 1.0, values = double(A.nnz) / brow;
+    if (double(A.nblk) / brow * rows > 460.0) return false;
+    return values * rows <= 2048.0 || (A.avg_nnz > 12.0 && values * 8.0 <= 2048.0);
 }
 
 // Whether the block kind runs its long-row kernel: rows of which eight overflow
