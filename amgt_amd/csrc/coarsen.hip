@@ -1635,8 +1635,7 @@ int amgt_amg_extpi_interp(int32_t n, const int32_t *A_i, const int32_t *A_j,
     // so that the output kernel takes a thread per slot); otherwise the slots
     // are sized by the rows' upper bounds.
     constexpr int kMaxSlot = 16;
-    int shift = 0;
-    while ((1 << shift) < max_elmts) ++shift;
+    int shift = 0;  // of the fixed slots
     RowSlots slots{};
     int32_t *flag = nullptr, *f2c = nullptr, *cnt = nullptr, *use = nullptr, *ovf = nullptr;
     int8_t *dneg = nullptr;
@@ -1652,6 +1651,7 @@ int amgt_amg_extpi_interp(int32_t n, const int32_t *A_i, const int32_t *A_j,
     AMGT_TRY(tmp.get(&tot, 1));
     int64_t total_slots = 0;
     if (max_elmts > 0 && max_elmts <= kMaxSlot) {
+        while ((1 << shift) < max_elmts) ++shift;
         slots.stride = 1 << shift;
         total_slots = int64_t(n) << shift;
     } else {

@@ -225,6 +225,21 @@ def test_extpi_group_edges_match_oracle(dev, per_row, mixed):
         assert np.array_equal(PA.cpu().numpy(), rPA), pmx
 
 
+@pytest.mark.parametrize("limit", [2**30, 2**30 + 1, 2**31 - 1])
+def test_extpi_limits_up_to_int_max(dev, limit):
+    """A limit above every row's length, INT_MAX included, truncates nothing: P equals
+    the unlimited one."""
+    print(f"[extpi limit] {limit}", flush=True)
+    n = 900
+    I, J, A = _rand_long(n, 9, 3)
+    dI, dJ, dA = T(I, dev), T(J, dev), T(A, dev)
+    SI, SJ = C.strength(n, dI, dJ, dA, 0.25, 0.9)
+    cf, _ = C.pmis(n, SI, SJ, 0)
+    P = C.extpi_interp(n, dI, dJ, dA, SI, SJ, cf, limit)
+    U = C.extpi_interp(n, dI, dJ, dA, SI, SJ, cf, 0)
+    assert all(torch.equal(a, b) for a, b in zip(P[:3], U[:3])) and P[3] == U[3]
+
+
 def test_pmis_cf_init_rejected(dev):
     import ctypes
     from amgt_amd import _lib as L
