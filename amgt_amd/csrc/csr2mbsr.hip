@@ -754,8 +754,9 @@ int sort_tiles(int32_t nrows, int32_t ncols, int64_t nnz, const int32_t *I, cons
 
 }  // namespace
 
-int csr_to_mbsr(int32_t nrows, int32_t ncols, int64_t nnz, const int32_t *rowptr,
-                const int32_t *colidx, const double *A, hipStream_t s, Mbsr *out) {
+// (its last kernel may be pending on return)
+static int convert(int32_t nrows, int32_t ncols, int64_t nnz, const int32_t *rowptr,
+                   const int32_t *colidx, const double *A, hipStream_t s, Mbsr *out) {
     Mbsr &m = *out;
     m = Mbsr();
     m.nrows = nrows;
@@ -817,6 +818,16 @@ int csr_to_mbsr(int32_t nrows, int32_t ncols, int64_t nnz, const int32_t *rowptr
     m.avg_nnz = nblk ? double(nnz) / double(nblk) : 0.0;
     m.max_row_blocks = ht.max_blocks;
     m.spmv_kernel = default_spmv_kernel(m);
+    return AMGT_OK;
+}
+
+int csr_to_mbsr(int32_t nrows, int32_t ncols, int64_t nnz, const int32_t *rowptr,
+                const int32_t *colidx, const double *A, hipStream_t s, Mbsr *out) {
+    AMGT_TRY(convert(nrows, ncols, nnz, rowptr, colidx, A, s, out));
+    // k_conv_pack reads the caller's row pointers and writes the handle's arrays:
+    // wait, so that the caller may free or change its arrays and use the handle on
+    // any stream (no stream of another user would know of this one's work)
+    AMGT_HIP(hipStreamSynchronize(s));
     return AMGT_OK;
 }
 

@@ -110,7 +110,9 @@ class MBSRMatrix:
     @classmethod
     def from_csr(cls, rowptr: torch.Tensor, colidx: torch.Tensor, values, nrows: int, ncols: int,
                  stream=None) -> "MBSRMatrix":
-        """CSR2BSR_GPU (csr_matvec_device.c:1201-1267).  values may be None (pattern only)."""
+        """CSR2BSR_GPU (csr_matvec_device.c:1201-1267).  values may be None (pattern only).
+        On return the matrix is whole, for use on any stream, and the tensors are no longer
+        read."""
         _need_cuda(rowptr, "rowptr", torch.int32)
         _need_cuda(colidx, "colidx", torch.int32)
         _need_cuda(values, "values", torch.float64)

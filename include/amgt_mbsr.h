@@ -83,7 +83,9 @@ int amgt_set_mixed_precision(int enable);
 
 /* ---- mBSR handle ---- */
 /* CSR2BSR_GPU, csr_matvec_device.c:1201-1267.  Rows may be in any column
- * order (HYPRE keeps the diagonal first).  d_val may be NULL (pattern only). */
+ * order (HYPRE keeps the diagonal first).  d_val may be NULL (pattern only).
+ * Synchronises the stream: on return the handle is whole, for use on any stream, and
+ * the CSR arrays are no longer read. */
 int amgt_mbsr_create_from_csr(int32_t nrows, int32_t ncols, int64_t nnz, const int32_t *d_rowptr,
                               const int32_t *d_colidx, const double *d_val, void *stream,
                               amgt_mbsr_t *out);

@@ -140,6 +140,37 @@ def test_conversion_tiles_of_short_and_long_rows(dev, ascending):
     assert np.array_equal(M.arrays()["val"].cpu().numpy(), -3.0 * ref["val"])
 
 
+def test_conversion_complete_on_return(dev):
+    """On a side stream: when from_csr returns, none of its work is pending; after it or
+    update_values the CSR tensors may be overwritten on another stream and the handle
+    used there without an event."""
+    (m, n), I, J, A = (262144, 262144), *O.stencil(7, 64, 64, 64)
+    ref = O.csr2mbsr(m, n, I, J, A)
+    side = torch.cuda.Stream()
+    for lens in (None, 300):
+        if lens:  # a tile over the capacity as well
+            m, n = 800, 2000
+            I = np.arange(m + 1, dtype=np.int32) * lens
+            J = np.concatenate([np.random.default_rng(r).permutation(n)[:lens]
+                                for r in range(m)]).astype(np.int32)
+            A = np.random.default_rng(5).standard_normal(len(J))
+            ref = O.csr2mbsr(m, n, I, J, A)
+        print(f"[conversion on a side stream] {m} rows", flush=True)
+        dI, dJ, dA = T(I, dev), T(J, dev), T(A, dev)
+        torch.cuda.synchronize()
+        M = MBSRMatrix.from_csr(dI, dJ, dA, m, n, stream=side)
+        assert side.query()
+        for t in (dI, dJ, dA):
+            t.zero_()
+        check_structure(M, ref)
+        dI, dJ, dA = T(I, dev), T(J, dev), T(2.0 * A, dev)
+        torch.cuda.synchronize()
+        M.update_values(dI, dJ, dA, stream=side)
+        for t in (dI, dJ, dA):
+            t.zero_()
+        assert np.array_equal(M.arrays()["val"].cpu().numpy(), 2.0 * ref["val"])
+
+
 def test_conversion_pattern_only_and_empty(dev):
     (m, n), I, J, A = CASES["rand_rect"]()
     M = make(dev, m, n, I, J, None)
