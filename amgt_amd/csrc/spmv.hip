@@ -1290,13 +1290,18 @@ __global__ __launch_bounds__(256) void k_spmm_mfma_il(
 // listed in LDS (column, value), 16 lanes own a row, RPL right-hand sides each,
 // and a step takes the next entry of all four rows: its X row (consecutive
 // right-hand sides), RPL multiply-adds.  One wave per block row, lists of 32
-// blocks at a time; every row adds its entries in column order.
+// blocks at a time; every row adds its entries in column order.  Where one row is
+// much longer than the others (the lanes of those would wait for it), all 64
+// lanes take the rows in turn, 16 lanes every fourth entry, and the four parts of
+// a row's sum are added at the end: 60000 block rows of 27 blocks whose 4 entries
+// are in one row, k = 8 / 16 / 32: 213 / 215 / 363 us without, 78 / 78 / 110 with
+// (the MFMA form 98 / 98 / 144).  The turns of four loads decide.
 // Against the MFMA form: at a fill of 1/4 three of four products of an
 // instruction are zeros and each instruction occupies the SIMD as long as 8 to
 // 16 vector multiply-adds; the list costs 27 steps a row on 27-pt where the
 // block form issues 54 MFMAs and the selection of 27 bitmaps' operands.
-constexpr int kListBlk = 32;   // blocks listed at a time
-constexpr int kListRow = 128;  // entries per row, at most 4 per block
+constexpr int kListBlk = 32;                // blocks listed at a time
+constexpr int kListCap = 16 * kListBlk;     // entries of them, at most
 // inclusive sums within each half of the wave (DPP, as wave_incl_sum)
 __device__ __forceinline__ int half_incl_sum(int v) {
     v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);
@@ -1315,10 +1320,10 @@ __global__ __launch_bounds__(256) void k_spmm_rows(
     const double *__restrict__ x, int64_t kx, double alpha, double beta, const double *b,
     int64_t kb, double *y, int64_t ky) {
     constexpr int U = 4;  // entries in flight per row
-    struct List {
-        double val[4][kListRow];
-        int32_t col[4][kListRow];
-        uint16_t to[4 * kListRow];
+    struct List {  // the four rows' entries one after the other
+        double val[kListCap];
+        int32_t col[kListCap];
+        uint16_t to[kListCap];
     };
     __shared__ union {
         List list[4];
@@ -1329,9 +1334,11 @@ __global__ __launch_bounds__(256) void k_spmm_rows(
     const int br = __builtin_amdgcn_readfirstlane(br0 + w);
     if (!kCm && br >= brow) return;  // whole wave
     const int r = lane >> 4, v16 = lane & 15;
-    double acc[RPL];
+    double acc[RPL];       // row r
+    double even[4][RPL];   // this 16 lanes' part of the rows' sums, even split
+    bool split = false;
 #pragma unroll
-    for (int q = 0; q < RPL; ++q) acc[q] = 0.0;
+    for (int q = 0; q < RPL; ++q) acc[q] = even[0][q] = even[1][q] = even[2][q] = even[3][q] = 0.0;
     // right-hand sides RPL v16 .. (a lane past the last reads right-hand side
     // k0, and writes nothing)
     const int rhs = RPL * v16;
@@ -1365,34 +1372,34 @@ __global__ __launch_bounds__(256) void k_spmm_rows(
             const int cinc = half_incl_sum(c);
             const int t01 = __builtin_amdgcn_readlane(cinc, 31);
             const int t23 = __builtin_amdgcn_readlane(cinc, 63);
-            int a0 = (cinc - c) & 0xFFFF, a1 = (cinc - c) >> 16;
+            const int l0 = t01 & 0xFFFF, l1 = t01 >> 16, l2 = t23 & 0xFFFF, l3 = t23 >> 16;
+            const int e1 = l0, e2 = l0 + l1, e3 = e2 + l2;  // first entries of rows 1 to 3
+            int a0 = (h ? e2 : 0) + ((cinc - c) & 0xFFFF), a1 = (h ? e3 : e1) + ((cinc - c) >> 16);
             int src = ninc - n + (h ? __popc(m & 0xFFu) : 0);
             while (bits) {
                 const int e = __builtin_ctz(bits);
                 bits &= bits - 1u;
-                const int at = (2 * h + (e >> 2)) * kListRow + (e < 4 ? a0++ : a1++);
-                s.col[0][at] = col + (e & 3);
+                const int at = e < 4 ? a0++ : a1++;
+                s.col[at] = col + (e & 3);
                 s.to[src++] = uint16_t(at);
             }
             __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
             __builtin_amdgcn_wave_barrier();
 #pragma unroll
             for (int u = 0; u < 2; ++u)
-                if (64 * u + lane < nv) s.val[0][s.to[64 * u + lane]] = av[u];
-            for (int t = 128 + lane; t < nv; t += 64) s.val[0][s.to[t]] = double(val[v0 + t]);
+                if (64 * u + lane < nv) s.val[s.to[64 * u + lane]] = av[u];
+            for (int t = 128 + lane; t < nv; t += 64) s.val[s.to[t]] = double(val[v0 + t]);
             v0 += nv;
             __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
             __builtin_amdgcn_wave_barrier();
-            const int l0 = t01 & 0xFFFF, l1 = t01 >> 16, l2 = t23 & 0xFFFF, l3 = t23 >> 16;
-            const int len = r == 0 ? l0 : (r == 1 ? l1 : (r == 2 ? l2 : l3));
             const int steps = max(max(l0, l1), max(l2, l3));
-            for (int t = 0; t < steps; t += U) {
-                double a[U], xv[U][RPL];
+            // entries t + u * stride (u < U) below end; their X rows' parts
+            auto load = [&](int t, int stride, int end, double (&a)[U], double (&xv)[U][RPL]) {
 #pragma unroll
                 for (int u = 0; u < U; ++u) {
-                    const int at = min(t + u, kListRow - 1);
-                    const int64_t cc = t + u < len ? s.col[r][at] : 0;
-                    a[u] = s.val[r][at];
+                    const int e = t + u * stride, at = min(e, kListCap - 1);
+                    const int64_t cc = e < end ? s.col[at] : 0;
+                    a[u] = s.val[at];
                     if (pair) {
                         const double2 x2 = *reinterpret_cast<const double2 *>(xl[0] + cc * kx);
                         xv[u][0] = x2.x;
@@ -1402,15 +1409,51 @@ __global__ __launch_bounds__(256) void k_spmm_rows(
                         for (int q = 0; q < RPL; ++q) xv[u][q] = xl[q][cc * kx];
                     }
                 }
+            };
+            double a[U], xv[U][RPL];
+            const int even_turns = (l0 + 4 * U - 1) / (4 * U) + (l1 + 4 * U - 1) / (4 * U) +
+                                   (l2 + 4 * U - 1) / (4 * U) + (l3 + 4 * U - 1) / (4 * U);
+            if (4 * ((steps + U - 1) / U) <= 5 * even_turns) {  // (wave-uniform)
+                const int beg = r == 0 ? 0 : (r == 1 ? e1 : (r == 2 ? e2 : e3));
+                const int end = r == 0 ? e1 : (r == 1 ? e2 : (r == 2 ? e3 : nv));
+                for (int t = 0; t < steps; t += U) {
+                    load(beg + t, 1, end, a, xv);
 #pragma unroll
-                for (int u = 0; u < U; ++u)
-                    if (t + u < len) {
+                    for (int u = 0; u < U; ++u)
+                        if (beg + t + u < end) {
 #pragma unroll
-                        for (int q = 0; q < RPL; ++q) acc[q] = fma(a[u], xv[u][q], acc[q]);
+                            for (int q = 0; q < RPL; ++q) acc[q] = fma(a[u], xv[u][q], acc[q]);
+                        }
+                }
+            } else {
+                split = true;
+                const int from[5] = {0, e1, e2, e3, nv};
+#pragma unroll
+                for (int k = 0; k < 4; ++k)
+                    for (int t = from[k]; t < from[k + 1]; t += 4 * U) {
+                        load(t + r, 4, from[k + 1], a, xv);
+#pragma unroll
+                        for (int u = 0; u < U; ++u)
+                            if (t + r + 4 * u < from[k + 1]) {
+#pragma unroll
+                                for (int q = 0; q < RPL; ++q)
+                                    even[k][q] = fma(a[u], xv[u][q], even[k][q]);
+                            }
                     }
             }
             __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
             __builtin_amdgcn_wave_barrier();
+        }
+    }
+    if (split) {  // rows r of the four lane groups' parts
+#pragma unroll
+        for (int q = 0; q < RPL; ++q) {
+            const bool up = (r & 2) != 0, odd = (r & 1) != 0;
+            const double p0 = (up ? even[2][q] : even[0][q]) +
+                              __shfl_xor(up ? even[0][q] : even[2][q], 32);
+            const double p1 = (up ? even[3][q] : even[1][q]) +
+                              __shfl_xor(up ? even[1][q] : even[3][q], 32);
+            acc[q] += (odd ? p1 : p0) + __shfl_xor(odd ? p0 : p1, 16);
         }
     }
     if constexpr (kCm) {

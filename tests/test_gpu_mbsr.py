@@ -545,6 +545,45 @@ def test_spmm_block_lists(dev, prec, tol, k, fill):
         assert np.all(np.abs(Z[:, v] - exp) <= tol * scale), v
 
 
+@pytest.mark.parametrize("prec,tol", [(L.AMGT_DOUBLE, 1e-12), (L.AMGT_FLOAT, 2e-6),
+                                      (L.AMGT_HALF, 2e-3)])
+@pytest.mark.parametrize("k", [8, 17, 32, 33])
+def test_spmm_uneven_rows(dev, prec, tol, k):
+    """Block rows whose entries lie in one or two of the four rows, up to 65 blocks (several
+    lists, even and uneven ones in one block row), lengths around multiples of 16 and 4."""
+    rng = np.random.default_rng(k)
+    # (blocks, entries per block of the long row, the long row, from block: even before)
+    shapes = [(27, 4, 0, 0), (32, 4, 3, 0), (33, 4, 1, 0), (65, 4, 2, 0), (65, 4, 0, 32),
+              (16, 1, 2, 0), (17, 1, 3, 0), (5, 4, 1, 0), (1, 4, 3, 0), (64, 3, 2, 20), (0, 0, 0, 0)]
+    n, m, rows, cols = 4 * 90 - 2, 4 * len(shapes) - 1, [], []
+    for br, (c, f, lr, even) in enumerate(shapes):
+        for j, bc in enumerate(np.sort(rng.permutation(90)[:c])):
+            if j < even:
+                rows += [4 * br, 4 * br + 1, 4 * br + 2, 4 * br + 3]
+                cols += list(4 * int(bc) + rng.permutation(4))
+            else:
+                rows += [4 * br + lr] * f + ([4 * br + (lr + 1) % 4] if j % 5 == 0 else [])
+                cols += list(4 * int(bc) + rng.permutation(4)[:f]) + ([4 * int(bc)] if j % 5 == 0 else [])
+    ok = (np.array(rows) < m) & (np.array(cols) < n)
+    S = sp.csr_matrix((rng.standard_normal(len(rows))[ok],
+                       (np.array(rows)[ok], np.array(cols)[ok])), shape=(m, n))
+    I, J, A = S.indptr.astype(np.int32), S.indices.astype(np.int32), S.data
+    ref = O.csr2mbsr(m, n, I, J, A)
+    M = make(dev, m, n, I, J, A)
+    assert M.info()["avg_nnz"] <= 4.5  # the row kernel
+    M.set_precision(prec)
+    X, B = rng.standard_normal((k, n)), rng.standard_normal((k, m))
+    Y = M.spmm(T(X, dev), alpha=-1.0, beta=1.0, B=T(B, dev)).cpu().numpy()
+    Z = torch.full((m, k), float("nan"), dtype=torch.float64, device=dev)
+    M.spmm_interleaved(T(X.T, dev), Z, alpha=-1.0, beta=1.0, B=T(B.T, dev))
+    Z = Z.cpu().numpy()
+    for v in range(k):
+        exp = O.mbsr_spmv(ref, -1.0, X[v], 1.0, B[v])
+        scale = row_scale(m, n, I, J, A, X[v], 1.0, B[v])
+        assert np.all(np.abs(Y[v] - exp) <= tol * scale), v
+        assert np.all(np.abs(Z[:, v] - exp) <= tol * scale), v
+
+
 def test_full_size_c2_spmv(dev):
     """3D 7-point 128^3 (2,097,152 rows): bit-exact structure and FP64 SpMV vs the oracle."""
     from amgt_amd import workloads as W
