@@ -13,6 +13,7 @@
 // x, b, y are FP64.
 #include "internal.hpp"
 
+#include <algorithm>
 #include <string>
 #include <type_traits>
 
@@ -1743,20 +1744,29 @@ int launch_spmm_g(const Mbsr &A, const VT *val, int k, double alpha, const doubl
     return AMGT_OK;
 }
 
-// Entries per block up to which k_spmm_rows runs instead of k_spmm_mfma_il.
-// Measured on 16384 block rows of 27 random blocks, k = 8 / 16 / 32 (us, rows
-// against MFMA): 2.1 entries 19 / 23 / 30 against 31 / 32 / 45; 4.0 entries 29 /
-// 31 / 43 against 31 / 32 / 44; 6.0 entries 40 / 41 / 57 against 31 / 31 / 44.
-// Stencils, whose rows have equal lengths, gain more: 27-pt 64^3 (4.1 entries),
-// k = 32, 133 against 167.
-constexpr double kSpmmRowsMaxNnz = 4.5;
+// Whether k_spmm_rows runs instead of k_spmm_mfma_il.  The row kernel costs a fixed
+// part per block row (its lists) and its entries, the MFMA form its blocks, so
+// the line in entries per block rises with the blocks of a row.  Measured on 20000
+// to 100000 block rows of random blocks, k = 8 / 32 (us, rows against MFMA): 4
+// blocks of 2 entries 53 / 64 against 37 / 49; 7 of 2 58 / 77 against 53 / 70; 13 of
+// 2 70 / 92 against 78 / 116, of 3 81 / 111 against 79 / 117, of 4 94 / 135 against
+// 80 / 127; 20 of 3 62 / 86 against 72 / 106, of 4 72 / 103 against 72 / 106, of 5
+// 83 / 120 against 73 / 106; 27 of 4 87 / 128 against 96 / 139, of 5 103 / 151 against
+// 95 / 139; 60 of 4 63 / 94 against 74 / 106, of 5 76 / 113 against 74 / 106.
+// Stencils, whose rows have equal lengths, alike: 5-pt (5 blocks of 4) 163 / 270
+// against 104 / 205, 9-pt (9 of 4) 95 / 150 against 75 / 144, 27-pt 64^3 (25 of 4.1)
+// 90 / 123 against 107 / 149.
+bool spmm_by_rows(const Mbsr &A) {
+    const double blocks = A.brow > 0 ? double(A.nblk) / A.brow : 0.0;
+    return blocks > 0.0 && A.avg_nnz <= std::min(4.5, 6.2 - 42.0 / blocks);
+}
 // X interleaved, Y interleaved or (kCm) column-major: 32 right-hand sides per launch
 template <typename VT, bool kCm>
 int launch_spmm_il(const Mbsr &A, const VT *val, int k, double alpha, const double *x,
                    int64_t kx, double beta, const double *b, int64_t kb, double *y, int64_t ky,
                    hipStream_t s) {
     const int64_t grid = (int64_t(A.brow) + 3) / 4;
-    const bool rows = A.avg_nnz <= kSpmmRowsMaxNnz;
+    const bool rows = spmm_by_rows(A);
     for (int k0 = 0; k0 < k; k0 += 32) {
         const int kn = k - k0 < 32 ? k - k0 : 32;
 #define AMGT_SPMM_ROWS(R_)                                                                       \
