@@ -59,39 +59,59 @@ __device__ __forceinline__ int64_t diag_pos(const int32_t *__restrict__ I,
 }
 
 // ---- strength (par_strength.c:75-528, one function) ---------------------------
-// A thread per row; the entries of the workgroup's 256 rows are staged in LDS
-// with coalesced loads where they fit (7-pt: 1792 of kStageEntries), and the
-// strong columns leave through LDS.  (Threads walking their rows in memory: 81
-// us to count and 188 us to fill on 7-pt 128^3, 176 MB read by each.)
+// A thread per row; the entries of the workgroup's `per` rows are staged in LDS
+// with coalesced loads, as many rows at a time as fit (7-pt: all 256, 1792 of
+// kStageEntries), and the strong columns leave through LDS; a row that does not
+// fit by itself is walked in memory.  (Threads walking their rows in memory: 81 us
+// to count and 188 us to fill on 7-pt 128^3, 176 MB read by each; whole calls
+// 360 -> 196 us, 27-pt 64^3 547 -> 154.)  A workgroup's parts follow each other, so
+// small levels give it fewer rows (125-pt 30^3: 248 us walked, 961 with 256 rows a
+// workgroup, 142 with 16).
 constexpr int kStageEntries = 2048;
 
 #pragma clang fp contract(off)
 // row entries [b, e) of j / a; strong columns to out (kFill), their number
 // returned; d: the diagonal's position or -1
-template <bool kFill>
-__device__ __forceinline__ int strong_entries(const int32_t *j, const double *a, int64_t b,
-                                              int64_t e, int64_t d, double theta,
-                                              double max_row_sum, int32_t *out) {
+template <bool kFill, typename P>
+__device__ __forceinline__ int strong_entries(const int32_t *j, const double *a, P b, P e, P d,
+                                              double theta, double max_row_sum, int32_t *out) {
     const double diag = d >= 0 ? a[d] : 0.0;
     double row_scale = 0.0, row_sum = diag;
-    for (int64_t p = b; p < e; ++p) {
-        if (p == d) continue;
-        const double v = a[p];
-        if (diag < 0) row_scale = v > row_scale ? v : row_scale;
-        else row_scale = v < row_scale ? v : row_scale;
-        row_sum += v;
+    // eight entries' loads at a time, ahead of the chains of sums and of the stores
+    // (which could alias them)
+    constexpr int U = 8;
+    for (P p0 = b; p0 < e; p0 += U) {
+        double v[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) v[u] = a[p0 + u < e ? p0 + u : p0];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const bool on = p0 + u < e && p0 + u != d;
+            const bool beyond = diag < 0 ? v[u] > row_scale : v[u] < row_scale;
+            row_scale = on && beyond ? v[u] : row_scale;
+            row_sum = on ? row_sum + v[u] : row_sum;
+        }
     }
     int c = 0;
     // a row too dominant by the row-sum test keeps only weak dependencies
     if (!(fabs(row_sum) > fabs(diag) * max_row_sum && max_row_sum < 1.0)) {
         const double thr = theta * row_scale;
-        for (int64_t p = b; p < e; ++p) {
-            if (p == d) continue;
-            const double v = a[p];
-            const bool weak = diag < 0 ? (v <= thr) : (v >= thr);
-            if (!weak) {
-                if (kFill) out[c] = j[p];
-                ++c;
+        for (P p0 = b; p0 < e; p0 += U) {
+            double v[U];
+            int32_t k[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const P p = p0 + u < e ? p0 + u : p0;
+                v[u] = a[p];
+                k[u] = kFill ? j[p] : 0;
+            }
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const bool weak = diag < 0 ? (v[u] <= thr) : (v[u] >= thr);
+                if (p0 + u < e && p0 + u != d && !weak) {
+                    if (kFill) out[c] = k[u];
+                    ++c;
+                }
             }
         }
     }
@@ -99,7 +119,8 @@ __device__ __forceinline__ int strong_entries(const int32_t *j, const double *a,
 }
 
 template <bool kFill>
-__global__ __launch_bounds__(kThreads) void k_strength(int32_t n, const int32_t *__restrict__ I,
+__global__ __launch_bounds__(kThreads) void k_strength(int32_t n, int32_t per,
+                                                      const int32_t *__restrict__ I,
                                                       const int32_t *__restrict__ J,
                                                       const double *__restrict__ A, double theta,
                                                       double max_row_sum, int32_t *__restrict__ cnt,
@@ -108,34 +129,55 @@ __global__ __launch_bounds__(kThreads) void k_strength(int32_t n, const int32_t 
     __shared__ double s_a[kStageEntries];
     __shared__ int32_t s_j[kStageEntries];
     __shared__ int32_t s_out[kFill ? kStageEntries : 1];
-    const int r0 = blockIdx.x * kThreads, i = r0 + threadIdx.x;
-    const int e0 = I[r0], ne = I[min(r0 + kThreads, n)] - e0;
-    if (ne <= kStageEntries) {  // uniform
-        for (int t = threadIdx.x; t < ne; t += kThreads) {
-            s_j[t] = J[e0 + t];
-            s_a[t] = A[e0 + t];
+    __shared__ int32_t s_I[kThreads + 1];
+    __shared__ int32_t s_d[kThreads];  // the diagonals' places
+    const int r0 = blockIdx.x * per, m = min(per, n - r0), tid = threadIdx.x;  // per <= kThreads
+    for (int t = tid; t <= m; t += kThreads) s_I[t] = I[r0 + t];
+    s_d[tid] = INT_MAX;
+    __syncthreads();
+    for (int ra = 0; ra < m;) {  // rows ra .. rb - 1 of the workgroup's (uniform)
+        const int e0 = s_I[ra];
+        int rb = s_I[m] - e0 <= kStageEntries ? m : ra;
+        for (int hi = m; rb < hi;) {
+            const int mid = (rb + hi + 1) >> 1;
+            if (s_I[mid] - e0 <= kStageEntries) rb = mid;
+            else hi = mid - 1;
         }
-        __syncthreads();
-        const int o0 = kFill ? SI[r0] : 0;
-        if (i < n) {
-            const int b = I[i] - e0, e = I[i + 1] - e0;
-            int d = -1;
-            for (int p = b; p < e && d < 0; ++p) d = s_j[p] == i ? p : -1;
-            const int c = strong_entries<kFill>(s_j, s_a, b, e, d, theta, max_row_sum,
-                                                kFill ? s_out + (SI[i] - o0) : nullptr);
+        const bool staged = rb > ra;
+        rb = max(rb, ra + 1);
+        const bool mine = tid >= ra && tid < rb;
+        const int i = r0 + tid, ne = s_I[rb] - e0;
+        if (staged) {
+            for (int t = tid; t < ne; t += kThreads) {
+                const int j = J[e0 + t], q = j - r0;
+                s_j[t] = j;
+                s_a[t] = A[e0 + t];
+                if (q >= ra && q < rb && e0 + t >= s_I[q] && e0 + t < s_I[q + 1])
+                    atomicMin(&s_d[q], t);
+            }
+            __syncthreads();
+            const int o0 = kFill ? SI[r0 + ra] : 0;
+            if (mine) {
+                const int d = s_d[tid];
+                const int c = strong_entries<kFill>(s_j, s_a, s_I[tid] - e0, s_I[tid + 1] - e0,
+                                                    d == INT_MAX ? -1 : d, theta, max_row_sum,
+                                                    kFill ? s_out + (SI[i] - o0) : nullptr);
+                if (!kFill) cnt[i] = c;
+            }
+            if constexpr (kFill) {
+                __syncthreads();
+                const int no = SI[r0 + rb] - o0;
+                for (int t = tid; t < no; t += kThreads) SJ[o0 + t] = s_out[t];
+            }
+            if (rb < m) __syncthreads();  // (uniform; the next part takes the place)
+        } else if (mine) {
+            const int c = strong_entries<kFill, int64_t>(J, A, I[i], I[i + 1], diag_pos(I, J, i),
+                                                         theta, max_row_sum,
+                                                         kFill ? SJ + SI[i] : nullptr);
             if (!kFill) cnt[i] = c;
         }
-        if constexpr (kFill) {
-            __syncthreads();
-            const int no = SI[min(r0 + kThreads, n)] - o0;
-            for (int t = threadIdx.x; t < no; t += kThreads) SJ[o0 + t] = s_out[t];
-        }
-        return;
+        ra = rb;
     }
-    if (i >= n) return;
-    const int c = strong_entries<kFill>(J, A, I[i], I[i + 1], diag_pos(I, J, i), theta,
-                                        max_row_sum, kFill ? SJ + SI[i] : nullptr);
-    if (!kFill) cnt[i] = c;
 }
 
 // ---- PMIS (par_coarsen.c:2101-2813 on one process) ------------------------------
@@ -1508,8 +1550,12 @@ int amgt_amg_strength(int32_t n, const int32_t *A_i, const int32_t *A_j, const d
         set_error("allocation of S row pointer failed");
         return AMGT_ERR_ALLOC;
     }
+    // rows per workgroup: 1024 workgroups if there are rows for them (eight each)
+    int32_t per = 8;
+    while (per < kThreads && int64_t(n) >= int64_t(2 * per) * 1024) per *= 2;
+    const dim3 wgs(unsigned((int64_t(n) + per - 1) / per));
     if (n > 0) {
-        hipLaunchKernelGGL((k_strength<false>), dim3(grid_of(n)), dim3(kThreads), 0, s, n, A_i, A_j,
+        hipLaunchKernelGGL((k_strength<false>), wgs, dim3(kThreads), 0, s, n, per, A_i, A_j,
                            A_data, theta, max_row_sum, cnt, nullptr, nullptr);
         AMGT_HIP(hipGetLastError());
     }
@@ -1530,8 +1576,7 @@ int amgt_amg_strength(int32_t n, const int32_t *A_i, const int32_t *A_j, const d
         return AMGT_ERR_ALLOC;
     }
     if (n > 0) {
-        hipLaunchKernelGGL((k_strength<true>), dim3(grid_of(n)), dim3(kThreads), 0, s, n, A_i, A_j,
-                           A_data, theta, max_row_sum, nullptr, si, sjj);
+        hipLaunchKernelGGL((k_strength<true>), wgs, dim3(kThreads), 0, s, n, per, A_i, A_j, A_data, theta, max_row_sum, nullptr, si, sjj);
         AMGT_HIP(hipGetLastError());
     }
     *nnzS = total;

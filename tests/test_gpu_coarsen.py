@@ -225,6 +225,36 @@ def test_extpi_group_edges_match_oracle(dev, per_row, mixed):
         assert np.array_equal(PA.cpu().numpy(), rPA), pmx
 
 
+@pytest.mark.parametrize("n", [3001, 40003, 270001])
+@pytest.mark.parametrize("diagonal", ["ascending", "first", "none"])
+def test_strength_parts(dev, n, diagonal):
+    """Rows of 2047, 2048 and 2049 entries (the part a workgroup stages) and of 600 and 1449
+    (two parts) among tridiagonal and empty ones, 8, 32 and 256 rows per workgroup: S
+    equals the oracle's for both row-sum limits."""
+    print(f"[strength parts] n={n} diagonal={diagonal}", flush=True)
+    rng = np.random.default_rng(n)
+    lens = np.full(n, 3)
+    lens[::11] = 0
+    for at, group in ((8, [2048, 0, 1, 2047, 1, 2049, 3, 2]), (64, [600, 1448, 2, 1449, 600, 7, 2100, 5]),
+                      (1032, [700, 700, 700, 700, 0, 0, 2048, 2]), (n - 9, [3, 3, 2000, 47, 1, 3, 3, 2049, 600])):
+        lens[at:at + len(group)] = group
+    rows = np.repeat(np.arange(n), lens)
+    off = np.arange(len(rows)) - np.repeat(np.cumsum(lens) - lens, lens)
+    J = (rows + off * (n // 2600) + (0 if diagonal != "none" else 1)) % n
+    A = -rng.uniform(0.1, 1.0, len(J)) * np.where(rng.random(len(J)) < 0.1, -1.0, 1.0)
+    A[J == rows] = rng.choice([-2.0, 2.0, 0.5], int((J == rows).sum()))
+    if diagonal == "ascending":
+        o = np.lexsort((J, rows))
+        J, A = J[o], A[o]
+    I = np.zeros(n + 1, np.int32)
+    I[1:] = np.cumsum(lens)
+    J = J.astype(np.int32)
+    for theta, mrs in ((0.25, 1.0), (0.5, 0.9)):
+        SI, SJ = C.strength(n, T(I, dev), T(J, dev), T(A, dev), theta, mrs)
+        rSI, rSJ = O.amg_strength(n, I, J, A, theta, mrs)
+        assert np.array_equal(SI.cpu().numpy(), rSI) and np.array_equal(SJ.cpu().numpy(), rSJ)
+
+
 @pytest.mark.parametrize("limit", [2**30, 2**30 + 1, 2**31 - 1])
 def test_extpi_limits_up_to_int_max(dev, limit):
     """A limit above every row's length, INT_MAX included, truncates nothing: P equals
