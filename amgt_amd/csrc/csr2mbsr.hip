@@ -37,9 +37,16 @@ enum : int { kErrDup = 1, kErrCol = 2, kErrBig = 4, kErrPtr = 8 };
 constexpr int kTileThreads = 256;
 constexpr int kTileCap = 1024;   // entries of a tile
 constexpr int kTileRows = 128;   // block rows of a tile, at most
+constexpr int kRowCap = 8192;    // entries of a block row, at most
 // entries between the starts of two tiles: the tile's last block row must fit
 // behind them (257 or 513 entries); 768 for block rows of at most 128 on average
 constexpr int kTileStart = 768, kTileStartLong = 512, kTileLongRow = 128;
+// Block rows over this many entries: places by binary search of their CSR rows
+// where those ascend, instead of counting all keys (few rows of 700 beside 7-pt
+// ones: the tile took 75 us, the latency of one workgroup's counting).
+constexpr int kLongRank = 192;
+// CSR rows over this many entries per lane are numbered by the whole workgroup
+constexpr int kFillTurns = 32, kFillList = kTileCap / kFillTurns;
 
 // row pointer i, kept inside [0, nnz]: the pointers are verified only with the
 // readback after the sorts, so no load may follow a wrong one out of the arrays
@@ -77,12 +84,13 @@ __global__ __launch_bounds__(kTileThreads) void k_conv_cut(int32_t nrows, int32_
                                                            int32_t *__restrict__ tile_lo,
                                                            int32_t *__restrict__ err) {
     const int br = blockIdx.x * kTileThreads + threadIdx.x;
+    int bad = 0;
+    for (int r = 4 * br; br < brow && r < min(4 * br + 4, nrows); ++r) bad |= I[r + 1] < I[r];
+    bad = __syncthreads_or(bad);
+    // err[0] collects the errors of the listed tiles, err[1 + k] those seen here
+    if (threadIdx.x == 0) err[1 + blockIdx.x] = bad ? kErrPtr : 0;
+    if (br == 0) err[0] = 0;
     if (br > brow) return;
-    if (br < brow) {
-        bool bad = false;
-        for (int r = 4 * br; r < min(4 * br + 4, nrows); ++r) bad |= I[r + 1] < I[r];
-        if (bad) atomicOr(err, kErrPtr);
-    }
     const int before = br > 0 ? entry_at(I, 4 * (br - 1), nnz) / start + (br - 1) / rows : -1;
     const int key = br < brow ? entry_at(I, 4 * br, nnz) / start + br / rows : ntiles;
     for (int t = before + 1; t <= key; ++t) tile_lo[t] = br;
@@ -129,7 +137,8 @@ __global__ __launch_bounds__(kTileThreads) void k_conv_tile(
     __shared__ int s_I[4 * kTileRows + 1];             // row starts within the tile
     __shared__ int s_ps[kTileRows + 1];                // padded block row starts
     __shared__ int s_first[kTileRows + 1];
-    __shared__ int s_wt[NW], s_err;
+    __shared__ int s_wt[NW], s_err, s_longest, s_descends;
+    __shared__ int s_list[kFillList], s_nlist;         // CSR rows filled by all threads
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
     int t0, rows, part;  // first block row, block rows, index in parts
     if constexpr (kList) {
@@ -154,7 +163,11 @@ __global__ __launch_bounds__(kTileThreads) void k_conv_tile(
     const int base = entry_at(I, 4 * t0, nnz);
     const int n = entry_at(I, 4 * t0 + nr, nnz) - base;
     if (n < 0 || n > kTileCap) {  // uniform
-        if (!kList && tid == 0) parts[part] = TilePart{0, TilePart::kOver, 0ull};
+        if (!kList && tid == 0) {
+            const int last = base + n - entry_at(I, 4 * (t0 + rows - 1), nnz);
+            parts[part] =
+                TilePart{0, TilePart::kOver | (last > kRowCap ? uint32_t(kErrBig) : 0u), 0ull};
+        }
         return;  // (kList: k_sort_block's row)
     }
     int cj[EPT];
@@ -174,7 +187,7 @@ __global__ __launch_bounds__(kTileThreads) void k_conv_tile(
         s_sorted[t] = kPadKey;
         s_rid[t] = 0;
     }
-    if (tid == 0) s_err = 0;
+    if (tid == 0) s_err = s_descends = s_nlist = 0;
     __syncthreads();
     if (w == 0) {  // padded starts of the block rows, two per lane
         int len[2];
@@ -190,15 +203,32 @@ __global__ __launch_bounds__(kTileThreads) void k_conv_tile(
             const int at = incl - len[1] - (u == 0 ? len[0] : 0);
             if (2 * lane + u <= rows) s_ps[2 * lane + u] = at;
         }
+        const int longest = wave_incl_max(max(len[0], len[1]));
         if (lane == 63 && rows == kTileRows) s_ps[rows] = incl;
+        if (lane == 63) s_longest = longest;
     }
     {  // the entries' rows: a power of two of lanes per row
         int lpr = kTileThreads;
         while (lpr > 1 && nr * lpr > kTileThreads) lpr >>= 1;
-        for (int row = tid / lpr; row < nr; row += kTileThreads / lpr)
+        for (int row = tid / lpr; row < nr; row += kTileThreads / lpr) {
+            if (s_I[row + 1] - s_I[row] > kFillTurns * lpr) {
+                if (tid % lpr == 0) {
+                    const int at = atomicAdd(&s_nlist, 1);
+                    if (at < kFillList) s_list[at] = row;  // (always, for ascending pointers)
+                }
+                continue;
+            }
             for (int e = s_I[row] + tid % lpr; e < s_I[row + 1]; e += lpr) s_rid[e] = uint16_t(row);
+        }
     }
     __syncthreads();
+    if (s_nlist > 0) {  // uniform
+        for (int k = 0; k < min(s_nlist, kFillList); ++k) {
+            const int row = s_list[k];
+            for (int e = s_I[row] + tid; e < s_I[row + 1]; e += kTileThreads) s_rid[e] = uint16_t(row);
+        }
+        __syncthreads();
+    }
     uint32_t key[EPT];
     int rid[EPT];
     int err = 0;
@@ -221,20 +251,66 @@ __global__ __launch_bounds__(kTileThreads) void k_conv_tile(
         }
     }
     __syncthreads();
+    // long block rows: whether their CSR rows ascend from the second entry on
+    // (ascending columns, or the diagonal first)
+    if (s_longest > kLongRank) {  // uniform
+#pragma unroll
+        for (int k = 0; k < EPT; ++k) {
+            const int e = tid + k * kTileThreads;
+            if (e >= n || e - 1 <= s_I[rid[k]]) continue;
+            const int br = rid[k] >> 2, at = s_ps[br] + (e - s_I[4 * br]);
+            if (s_ps[br + 1] - s_ps[br] > kLongRank && at > 0 && at < kPad && s_key[at - 1] >= key[k])
+                s_descends = 1;
+        }
+        __syncthreads();
+    }
+    const bool search = s_longest > kLongRank && s_descends == 0;
 #pragma unroll
     for (int k = 0; k < EPT; ++k) {
         const int e = tid + k * kTileThreads;
         if (e >= n) continue;
         const int br = rid[k] >> 2;
         int rank = 0;
-        const int j1 = min(s_ps[br + 1], kPad);
-        for (int j = s_ps[br]; j < j1; j += 4) {
-            const uint4 kk = *reinterpret_cast<const uint4 *>(&s_key[j]);
-            rank += kk.x < key[k] ? 1 : 0;
-            rank += kk.y < key[k] ? 1 : 0;
-            rank += kk.z < key[k] ? 1 : 0;
-            rank += kk.w < key[k] ? 1 : 0;
+        int j1 = min(s_ps[br + 1], kPad);
+        if (search && j1 - s_ps[br] > kLongRank) {
+            // the four CSR rows' smaller keys: the first, and a binary search of the rest
+            const int off = s_ps[br] - s_I[4 * br];
+            int lo[4], len[4];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const int b = s_I[min(4 * br + q, nr)];
+                len[q] = s_I[min(4 * br + q + 1, nr)] - b - 1;
+                lo[q] = b + 1 + off;
+                if (len[q] >= 0) rank += s_key[min(unsigned(b + off), unsigned(kPad - 1))] < key[k];
+                rank -= lo[q];
+            }
+            while (max(max(len[0], len[1]), max(len[2], len[3])) > 0) {
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    if (len[q] <= 0) continue;
+                    const int half = len[q] >> 1;
+                    const bool up = s_key[min(unsigned(lo[q] + half), unsigned(kPad - 1))] < key[k];
+                    lo[q] = up ? lo[q] + half + 1 : lo[q];
+                    len[q] = up ? len[q] - half - 1 : half;
+                }
+            }
+#pragma unroll
+            for (int q = 0; q < 4; ++q) rank += lo[q];
+            j1 = 0;  // (no counting below)
         }
+        auto below = [&](const uint4 &kk) {
+            return (kk.x < key[k] ? 1 : 0) + (kk.y < key[k] ? 1 : 0) + (kk.z < key[k] ? 1 : 0) +
+                   (kk.w < key[k] ? 1 : 0);
+        };
+        int j = s_ps[br];
+        for (; j + 32 <= j1; j += 32) {  // long rows: the reads' latency once per eight
+            uint4 kk[8];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) kk[u] = *reinterpret_cast<const uint4 *>(&s_key[j + 4 * u]);
+#pragma unroll
+            for (int u = 0; u < 8; ++u) rank += below(kk[u]);
+        }
+        for (; j < j1; j += 4) rank += below(*reinterpret_cast<const uint4 *>(&s_key[j]));
         const int to = min(s_I[4 * br] + rank, n - 1);
         s_sorted[to] = key[k];
         // places within the entry's own block row: a wave's stores stay within a
@@ -371,11 +447,7 @@ __global__ __launch_bounds__(THREADS) void k_sort_block(
     const int r0 = 4 * br;
     const int s = entry_at(I, r0, nnz);
     const int n = entry_at(I, min(r0 + 4, nrows), nnz) - s;
-    if (n <= kTileCap) return;  // k_conv_tile's row
-    if (n > CAP) {
-        if (t == 0) atomicOr(err_out, kErrBig);
-        return;
-    }
+    if (n <= kTileCap || n > CAP) return;  // k_conv_tile's row (or refused before)
     int np = 64;
     while (np < n) np <<= 1;
     if (t == 0) s_err = s_descends = 0;
@@ -525,7 +597,7 @@ __global__ __launch_bounds__(kTileThreads) void k_conv_list_sum(
 // One workgroup: the tiles' first blocks, the totals and the list of the tiles
 // over the capacity (in no order); four consecutive tiles per thread and step.
 constexpr int kFinThreads = 1024;
-__global__ __launch_bounds__(kFinThreads) void k_conv_finish(int32_t ntiles,
+__global__ __launch_bounds__(kFinThreads) void k_conv_finish(int32_t ntiles, int32_t nerr,
                                                              const TilePart *__restrict__ parts,
                                                              const int32_t *__restrict__ err_in,
                                                              int32_t *__restrict__ first,
@@ -538,6 +610,7 @@ __global__ __launch_bounds__(kFinThreads) void k_conv_finish(int32_t ntiles,
     int run = 0, mx = 0, err = 0;
     unsigned long long sq = 0ull;
     if (threadIdx.x == 0) s_over = 0;
+    for (int k = threadIdx.x; k < nerr; k += kFinThreads) err |= err_in[k];
     __syncthreads();
     for (int g = 0; g < ntiles; g += 4 * kFinThreads) {
         const int t = g + 4 * int(threadIdx.x);
@@ -582,7 +655,7 @@ __global__ __launch_bounds__(kFinThreads) void k_conv_finish(int32_t ntiles,
     }
     __syncthreads();
     if (threadIdx.x == 0) {
-        ConvTotals r{run, 0, *err_in, s_over, 0ull};
+        ConvTotals r{run, 0, 0, s_over, 0ull};
         for (int q = 0; q < NW; ++q) {
             r.max_blocks = max(r.max_blocks, s_mx[q]);
             r.err |= s_err[q];
@@ -590,10 +663,6 @@ __global__ __launch_bounds__(kFinThreads) void k_conv_finish(int32_t ntiles,
         }
         *tot = r;
     }
-}
-
-__global__ void k_conv_zero(int32_t *p) {
-    if (threadIdx.x == 0) *p = 0;
 }
 
 // row pointers of a matrix without rows
@@ -655,25 +724,42 @@ double stand_from(const RowStats &h, int64_t nblk, int32_t brow) {
 
 namespace {
 
-// Device scratch of one conversion.
+// Device scratch of one conversion: one block (each block of the pool costs a
+// lookup and, when it is given back, an event).
 struct ConvWork {
-    int32_t ntiles = 0;
+    int32_t ntiles = 0, nerr = 0;
     TilePart *parts = nullptr;
     ConvTotals *tot = nullptr;
     int32_t *first = nullptr, *rel = nullptr, *tmp_col = nullptr, *tiles = nullptr;
     int32_t *tile_lo = nullptr, *err = nullptr;
     uint16_t *tmp_map = nullptr;
+    char *block = nullptr;
     hipStream_t s = nullptr;
-    ~ConvWork() {
-        tmp_free(parts, s);
-        tmp_free(tot, s);
-        tmp_free(first, s);
-        tmp_free(rel, s);
-        tmp_free(tmp_col, s);
-        tmp_free(tmp_map, s);
-        tmp_free(tiles, s);
-        tmp_free(tile_lo, s);
-        tmp_free(err, s);
+    ~ConvWork() { tmp_free(block, s); }
+    int alloc(size_t brow, size_t nnz, bool blocks) {
+        size_t bytes = 0;
+        auto place = [&](auto *&p, size_t n) {
+            if (block) p = reinterpret_cast<std::decay_t<decltype(p)>>(block + bytes);
+            bytes += (n * sizeof(*p) + 255) & ~size_t(255);
+        };
+        auto all = [&] {
+            bytes = 0;
+            place(parts, size_t(ntiles));
+            place(tot, 1);
+            place(first, size_t(ntiles));
+            place(tiles, size_t(ntiles));
+            place(tile_lo, size_t(ntiles) + 1);
+            place(err, size_t(nerr));
+            if (blocks) {
+                place(rel, brow);
+                place(tmp_col, nnz);
+                place(tmp_map, nnz);
+            }
+        };
+        all();
+        AMGT_TRY(tmp_alloc_t(&block, bytes, s));
+        all();
+        return AMGT_OK;
     }
 };
 
@@ -690,28 +776,18 @@ int sort_tiles(int32_t nrows, int32_t ncols, int64_t nnz, const int32_t *I, cons
     const int32_t start = std::max(64, std::min(full, nz / 2048));
     const int32_t rows = std::max(4, std::min(kTileRows, brow / 1024));
     w.ntiles = brow > 0 ? nz / start + brow / rows + 1 : 0;
-    AMGT_TRY(tmp_alloc_t(&w.tile_lo, size_t(w.ntiles) + 1, s));
-    AMGT_TRY(tmp_alloc_t(&w.err, 1, s));
-    AMGT_TRY(tmp_alloc_t(&w.parts, size_t(w.ntiles), s));
-    AMGT_TRY(tmp_alloc_t(&w.tot, 1, s));
-    AMGT_TRY(tmp_alloc_t(&w.first, size_t(w.ntiles), s));
-    AMGT_TRY(tmp_alloc_t(&w.tiles, size_t(w.ntiles), s));
-    if (!values_only) {
-        AMGT_TRY(tmp_alloc_t(&w.rel, size_t(brow), s));
-        AMGT_TRY(tmp_alloc_t(&w.tmp_col, size_t(nnz), s));
-        AMGT_TRY(tmp_alloc_t(&w.tmp_map, size_t(nnz), s));
-    }
-    hipLaunchKernelGGL(k_conv_zero, dim3(1), dim3(64), 0, s, w.err);
+    const unsigned cuts = unsigned(brow / kTileThreads + 1);
+    w.nerr = w.ntiles > 0 ? int32_t(cuts) + 1 : 0;
+    AMGT_TRY(w.alloc(size_t(brow), size_t(nnz), !values_only));
     if (w.ntiles > 0) {
-        hipLaunchKernelGGL(k_conv_cut, dim3(unsigned(brow / kTileThreads + 1)), dim3(kTileThreads),
-                           0, s, nrows, brow, nz, start, rows, w.ntiles, I, w.tile_lo, w.err);
+        hipLaunchKernelGGL(k_conv_cut, dim3(cuts), dim3(kTileThreads), 0, s, nrows, brow, nz, start, rows, w.ntiles, I, w.tile_lo, w.err);
         hipLaunchKernelGGL((k_conv_tile<false>), dim3(unsigned(w.ntiles)), dim3(kTileThreads), 0,
                            s, nrows, ncols, nz, I, J, A, w.tile_lo,
                            static_cast<const int32_t *>(nullptr), val, w.tmp_col, w.tmp_map, w.rel,
                            w.parts, values_only);
     }
     auto totals = [&](int32_t *ends) -> int {
-        hipLaunchKernelGGL(k_conv_finish, dim3(1), dim3(kFinThreads), 0, s, w.ntiles, w.parts,
+        hipLaunchKernelGGL(k_conv_finish, dim3(1), dim3(kFinThreads), 0, s, w.ntiles, w.nerr, w.parts,
                            w.err, w.first, w.tiles, w.tot);
         AMGT_HIP(hipGetLastError());
         const Readback rb[3] = {{ht, w.tot, sizeof(ConvTotals)},
@@ -729,25 +805,28 @@ int sort_tiles(int32_t nrows, int32_t ncols, int64_t nnz, const int32_t *I, cons
         set_error("CSR->mBSR: row pointers must ascend");
         return AMGT_ERR_INPUT;
     }
+    if (ht->err & kErrBig) {
+        set_error("CSR->mBSR: a block row has more than 8192 entries (4 rows with > 2048 "
+                  "nonzeros on average); this build does not convert such rows");
+        return AMGT_ERR_UNSUPPORTED;
+    }
     if (ht->over > 0) {  // the tiles over the capacity, their last rows by themselves
         const unsigned nt = unsigned(ht->over);
         hipLaunchKernelGGL((k_conv_tile<true>), dim3(2 * nt), dim3(kTileThreads), 0, s, nrows,
                            ncols, nz, I, J, A, w.tile_lo, w.tiles, val, w.tmp_col, w.tmp_map,
                            w.rel, w.parts, values_only);
-        hipLaunchKernelGGL((k_sort_block<1024, 8192>), dim3(nt), dim3(1024), 0, s, nrows, ncols,
+        hipLaunchKernelGGL((k_sort_block<1024, kRowCap>), dim3(nt), dim3(1024), 0, s, nrows, ncols,
                            nz, I, J, A, w.tile_lo, w.tiles, val, w.tmp_col, w.tmp_map, w.rel,
                            w.err, values_only);
-        if (!values_only)
-            hipLaunchKernelGGL(k_conv_list_sum, dim3((nt + kTileThreads - 1) / kTileThreads),
-                               dim3(kTileThreads), 0, s, ht->over, w.tile_lo, w.tiles, w.rel,
-                               w.parts);
+        if (values_only) {  // (nothing to read back; the caller's arrays are read until here)
+            AMGT_HIP(hipGetLastError());
+            AMGT_HIP(hipStreamSynchronize(s));
+            return AMGT_OK;
+        }
+        hipLaunchKernelGGL(k_conv_list_sum, dim3((nt + kTileThreads - 1) / kTileThreads),
+                           dim3(kTileThreads), 0, s, ht->over, w.tile_lo, w.tiles, w.rel, w.parts);
         AMGT_HIP(hipGetLastError());
         AMGT_TRY(totals(ends));
-        if (ht->err & kErrBig) {
-            set_error("CSR->mBSR: a block row has more than 8192 entries (4 rows with > 2048 "
-                      "nonzeros on average); this build does not convert such rows");
-            return AMGT_ERR_UNSUPPORTED;
-        }
     }
     return AMGT_OK;
 }

@@ -140,6 +140,50 @@ def test_conversion_tiles_of_short_and_long_rows(dev, ascending):
     assert np.array_equal(M.arrays()["val"].cpu().numpy(), -3.0 * ref["val"])
 
 
+@pytest.mark.parametrize("order", ["ascending", "diagonal first", "random", "one pair swapped"])
+def test_conversion_long_rows_in_tiles(dev, order):
+    """Block rows of 189 to 196 entries (padded lengths around the line of the binary search),
+    and of 400 to 1023 with CSR rows around 32, 64 and 2048 / 4 entries, beside short and
+    empty rows in one tile: values, structure and the refreshed values."""
+    print(f"[conversion long rows] {order}", flush=True)
+    rng = np.random.default_rng(len(order))
+    quads = [[47, 47, 47, 48], [48] * 4, [49, 48, 48, 48], [49] * 4, [0, 0, 0, 193], [193, 0, 0, 0],
+             [1, 190, 1, 1], [300, 2, 301, 0], [32, 33, 64, 65], [600, 0, 0, 1], [1, 0, 0, 600],
+             [255] * 4, [256, 256, 256, 255], [0, 512, 511, 0], [1, 1, 1, 1020]]
+    lens = []
+    for q in quads * 24:  # over a million entries: tiles of 128 block rows
+        lens += q + [9, 8, 0, 7] * int(rng.integers(0, 240))
+    m, n = len(lens) - 1, 1500
+    lens = np.array(lens[:m])
+    rows = []
+    for r, k in enumerate(lens):
+        if k < 32:
+            c = np.sort((7 * r + 131 * np.arange(k)) % n)
+        else:
+            c = np.sort(rng.permutation(n)[:k])
+        if order == "random":
+            c = c[::-1] if k < 32 else rng.permutation(c)
+        elif order == "diagonal first" and k:
+            c = np.concatenate([c[k // 2:k // 2 + 1], np.delete(c, k // 2)])
+        elif order == "one pair swapped" and k > 4 and r % 3 == 0:
+            c[[k - 1, k - 2]] = c[[k - 2, k - 1]]
+        rows.append(c)
+    I = np.zeros(m + 1, np.int32)
+    I[1:] = np.cumsum(lens)
+    J = np.concatenate(rows).astype(np.int32)
+    A = rng.standard_normal(len(J))
+    ref = O.csr2mbsr(m, n, I, J, A)
+    M = make(dev, m, n, I, J, A)
+    check_structure(M, ref)
+    M.update_values(T(I, dev), T(J, dev), T(3.0 * A, dev))
+    assert np.array_equal(M.arrays()["val"].cpu().numpy(), 3.0 * ref["val"])
+    dup = int(np.flatnonzero(lens == 600)[0])
+    J[I[dup] + 599] = J[I[dup]]
+    with pytest.raises(L.AmgtError) as e:
+        make(dev, m, n, I, J, A)
+    assert e.value.status == L.AMGT_ERR_INPUT
+
+
 def test_conversion_complete_on_return(dev):
     """On a side stream: when from_csr returns, none of its work is pending; after it or
     update_values the CSR tensors may be overwritten on another stream and the handle
