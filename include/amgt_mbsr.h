@@ -36,7 +36,8 @@ enum {
     AMGT_ERR_DIM = 2,          /* incompatible dimensions (csr_matop_device.c:257-263) */
     AMGT_ERR_ALLOC = 3,        /* device allocation failed */
     AMGT_ERR_HIP = 4,          /* a HIP runtime call failed */
-    AMGT_ERR_INPUT = 5,        /* CSR input invalid: duplicate entry or column out of range */
+    AMGT_ERR_INPUT = 5,        /* CSR input invalid: duplicate entry, column out of range, row
+                                * pointers that descend or whose ends are not 0 and nnz */
     AMGT_ERR_UNSUPPORTED = 6   /* valid input outside the sizes this build handles */
 };
 
@@ -92,7 +93,9 @@ int amgt_mbsr_create_from_csr(int32_t nrows, int32_t ncols, int64_t nnz, const i
 /* frees the handle and every array it owns (csr_matrix.c:94-103) */
 int amgt_mbsr_destroy(amgt_mbsr_t A);
 /* Re-reads values from a CSR with the same pattern (the reference never
- * invalidates its cache; this is the refresh hook). */
+ * invalidates its cache; this is the refresh hook).  Synchronises the stream: the CSR
+ * arrays are no longer read on return.  The row pointers are checked (AMGT_ERR_INPUT);
+ * after an error the handle's values are undefined until the next refresh. */
 int amgt_mbsr_update_values(amgt_mbsr_t A, const int32_t *d_rowptr, const int32_t *d_colidx,
                             const double *d_val, void *stream);
 int amgt_mbsr_get_info(amgt_mbsr_t A, amgt_mbsr_info_t *info);

@@ -184,6 +184,49 @@ def test_conversion_long_rows_in_tiles(dev, order):
     assert e.value.status == L.AMGT_ERR_INPUT
 
 
+def test_conversion_bad_row_pointers(dev):
+    """Row pointers that descend inside (ends kept) and ends that do not fit: errors, by
+    from_csr and update_values, with every access inside the arrays (the kernels clamp the
+    pointers).  A block row over 8192 entries beside short ones is refused."""
+    m, n = 4000, 300
+    I = np.arange(m + 1, dtype=np.int32) * 6
+    J = ((np.arange(6 * m) // 6 * 5 + np.arange(6 * m) % 6 * 41) % n).astype(np.int32)
+    A = np.ones(len(J))
+    M = make(dev, m, n, I, J, A)
+    for at, v in ((1, 13), (2001, 0), (2002, 6 * m), (4 * 500, -5), (4 * 700, 2**31 - 1), (m - 1, 6 * m + 1)):
+        B = I.copy()
+        B[at] = v
+        print(f"[row pointers] {at}: {B[at]}", flush=True)
+        with pytest.raises(L.AmgtError) as e:
+            make(dev, m, n, B, J, A)
+        assert e.value.status == L.AMGT_ERR_INPUT and "ascend" in str(e.value)
+        with pytest.raises(L.AmgtError) as e:
+            M.update_values(T(B, dev), T(J, dev), T(A, dev))
+        assert e.value.status == L.AMGT_ERR_INPUT and "ascend" in str(e.value)
+    for at, v in ((0, 1), (m, 6 * m - 1)):
+        B = I.copy()
+        B[at] = v
+        for call in (lambda: make(dev, m, n, B, J, A),
+                     lambda: M.update_values(T(B, dev), T(J, dev), T(A, dev))):
+            with pytest.raises(L.AmgtError) as e:
+                call()
+            assert e.value.status == L.AMGT_ERR_INPUT and "rowptr" in str(e.value)
+    M.update_values(T(I, dev), T(J, dev), T(5.0 * A, dev))  # the handle is usable again
+    assert torch.equal(M.arrays()["val"].cpu(), torch.full((6 * m,), 5.0, dtype=torch.float64))
+    lens = np.array([3, 1, 0, 2] * 40 + [2048, 2048, 2048, 2049] + [1, 2, 3, 4] * 9)
+    I = np.zeros(len(lens) + 1, np.int32)
+    I[1:] = np.cumsum(lens)
+    J = np.concatenate([np.arange(k) * 4 + 1 for k in lens]).astype(np.int32)
+    with pytest.raises(L.AmgtError) as e:
+        make(dev, len(lens), 9000, I, J, np.ones(len(J)))
+    assert e.value.status == L.AMGT_ERR_UNSUPPORTED
+    lens[163] = 2048
+    I[1:] = np.cumsum(lens)
+    J = np.concatenate([np.arange(k) * 4 + 1 for k in lens]).astype(np.int32)
+    M = make(dev, len(lens), 9000, I, J, np.arange(len(J), dtype=np.float64))
+    check_structure(M, O.csr2mbsr(len(lens), 9000, I, J, np.arange(len(J), dtype=np.float64)))
+
+
 def test_conversion_complete_on_return(dev):
     """On a side stream: when from_csr returns, none of its work is pending; after it or
     update_values the CSR tensors may be overwritten on another stream and the handle
