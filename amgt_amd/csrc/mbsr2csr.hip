@@ -22,6 +22,7 @@ constexpr int kCap = 1024;       // entries (and blocks) of a tile held in LDS
 constexpr int kMaxRows = 128;    // block rows of a tile, at most
 // entries between the starts of two tiles, and for longer block rows
 constexpr int kStart = 768, kStartLong = 512, kLongRow = 128;
+constexpr int kPartBlocks = 768;  // blocks of a row exported in parts, more than
 
 // first block row of every tile: block row br belongs to tile
 // val_ptr[br] / start + br / rows
@@ -47,9 +48,10 @@ __device__ __forceinline__ int field_sum(uint32_t a, uint32_t b) {
     return int((a & 0xFFFFu) + (a >> 16) + (b & 0xFFFFu) + (b >> 16));
 }
 
-// One wave exports block row br: 16 block slots x 4 rows per step, each lane's
-// place from scans over the slots.  For the tiles the LDS form does not hold.
-__device__ void export_row(int br, int32_t nrows, const int32_t *__restrict__ blk_ptr,
+// One wave exports part `part` of `parts` of block row br's blocks: 16 block slots x
+// 4 rows per step, each lane's place from scans over the slots.  For the tiles the
+// LDS form does not hold.
+__device__ void export_row(int br, int part, int parts, int32_t nrows, const int32_t *__restrict__ blk_ptr,
                            const int32_t *__restrict__ blk_col,
                            const uint16_t *__restrict__ blk_map,
                            const int32_t *__restrict__ val_ptr, const double *__restrict__ val,
@@ -58,9 +60,19 @@ __device__ void export_row(int br, int32_t nrows, const int32_t *__restrict__ bl
     const int lane = threadIdx.x & 63;
     const int r = lane & 3, s = lane >> 2;
     const int p0 = blk_ptr[br], p1 = blk_ptr[br + 1];
-    int rowlen = 0;
-    for (int j = p0 + s; j < p1; j += 16) rowlen += __popc((blk_map[j] >> (4 * r)) & 0xFu);
-    for (int d = 4; d < 64; d <<= 1) rowlen += __shfl_xor(rowlen, d);  // lane r: row r
+    const int per = (p1 - p0 + 16 * parts - 1) / (16 * parts) * 16;
+    const int j0 = min(p0 + part * per, p1), j1 = min(j0 + per, p1);
+    int rowlen = 0, before = 0;  // entries of row r, of them before the part
+#pragma unroll 4
+    for (int j = p0 + s; j < p1; j += 16) {
+        const int c = __popc((blk_map[j] >> (4 * r)) & 0xFu);
+        rowlen += c;
+        before += j < j0 ? c : 0;
+    }
+    for (int d = 4; d < 64; d <<= 1) {  // lane r: row r
+        rowlen += __shfl_xor(rowlen, d);
+        before += __shfl_xor(before, d);
+    }
     int voff = val_ptr[br];
     int woff = voff;
 #pragma unroll
@@ -69,13 +81,16 @@ __device__ void export_row(int br, int32_t nrows, const int32_t *__restrict__ bl
         if (q < r) woff += len;
     }
     const int row = 4 * br + r;
-    if (s == 0 && row < nrows) I[row] = woff;
+    if (part == 0 && s == 0 && row < nrows) I[row] = woff;
+    woff += before;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) voff += __shfl(before, q);
     const uint32_t low = (1u << (4 * r)) - 1u;
-    for (int jb = p0; jb < p1; jb += 16) {
+    for (int jb = j0; jb < j1; jb += 16) {
         const int j = jb + s;
         uint32_t m = 0;
         int col = 0;
-        if (j < p1) {
+        if (j < j1) {
             m = blk_map[j];
             col = blk_col[j];
         }
@@ -135,8 +150,15 @@ __global__ __launch_bounds__(kThreads) void k_export_tile(
     const int b0 = blk_ptr[t0], nb = blk_ptr[t0 + rows] - b0;
     const int base = val_ptr[t0], n = val_ptr[t0 + rows] - base;
     if (n > kCap || nb > kCap) {  // uniform
-        for (int r = w; r < rows; r += NW)
-            export_row(t0 + r, nrows, blk_ptr, blk_col, blk_map, val_ptr, val, I, J, A);
+        // the last row, the only one that can be long, in a part per wave if it is (40000
+        // rows of 100 entries, every eighth of 1100: 456 us by one wave, 220; each part
+        // counts all bitmaps, which does not pay for rows of 600)
+        const int parts = blk_ptr[t0 + rows] - blk_ptr[t0 + rows - 1] > kPartBlocks ? NW : 1;
+        for (int k = w; k < rows - 1 + parts; k += NW) {
+            const int r = min(k, rows - 1);
+            export_row(t0 + r, k - r, r < rows - 1 ? 1 : parts, nrows, blk_ptr, blk_col, blk_map,
+                       val_ptr, val, I, J, A);
+        }
         return;
     }
     double v[BPT];  // the tile's values, wanted at the end

@@ -140,6 +140,30 @@ def test_conversion_tiles_of_short_and_long_rows(dev, ascending):
     assert np.array_equal(M.arrays()["val"].cpu().numpy(), -3.0 * ref["val"])
 
 
+@pytest.mark.parametrize("cut", [0, 1, 3])
+def test_export_long_rows(dev, cut):
+    """Block rows of 768 and 769 blocks (the line of the export in parts), 1025 to 2000 blocks
+    spread over one or four rows, alone and behind short ones; the last one ragged."""
+    print(f"[export long rows] cut={cut}", flush=True)
+    rng = np.random.default_rng(9)
+    lens = []
+    for q in ([0, 768, 0, 0], [769, 0, 0, 0], [0, 0, 0, 1025], [1040, 1, 0, 1040], [2000, 3, 2000, 2000],
+              [1, 2, 3, 4], [1100, 0, 0, 0]):
+        lens += [2, 0, 1, 3] * int(rng.integers(0, 3)) + q
+    lens = np.array(lens[:len(lens) - cut])
+    m, n = len(lens), 8400
+    I = np.zeros(m + 1, np.int32)
+    I[1:] = np.cumsum(lens)
+    # every fourth column of most rows: a block per entry
+    J = np.concatenate([4 * rng.permutation(n // 4)[:k] + rng.integers(0, 4, k) for k in lens]).astype(np.int32)
+    A = rng.standard_normal(len(J))
+    S = sp.csr_matrix((A, J, I), shape=(m, n))
+    S.sort_indices()
+    EI, EJ, EV = (t.cpu().numpy() for t in make(dev, m, n, I, J, A).to_csr())
+    assert np.array_equal(EI, S.indptr) and np.array_equal(EJ, S.indices)
+    assert np.array_equal(EV, S.data)
+
+
 @pytest.mark.parametrize("order", ["ascending", "diagonal first", "random", "one pair swapped"])
 def test_conversion_long_rows_in_tiles(dev, order):
     """Block rows of 189 to 196 entries (padded lengths around the line of the binary search),
