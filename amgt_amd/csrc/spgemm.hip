@@ -2027,8 +2027,14 @@ __global__ __launch_bounds__(256) void k_scale_values(int64_t n, double f, doubl
 // 5.7 entries); 5 blocks 339/382, 412/392, 442/394, 533/398, 620/420 (3.3);
 // 7 blocks of 2, 4, 6 entries 391/430, 554/454, 686/488 (2.5); numeric pass of
 // A P on 7-pt 128^3, trilinear P (23 products per scalar row, 4 lanes) 385/566.
+// Two or four rows share a wave, each a longer chain of loads, so the chip must
+// have waves enough besides: whole products of 3 blocks of 2 entries by block rows
+// 5000 129/122, 16000 135/139, 24000 139/146, 32000 146/148, 96000 185/213; 7 of 2
+// 139/128, 149/148, 159/156, 169/176, 252/266.
+constexpr int32_t kRowsMinBrow = 32768;
 int numeric_rows_lanes(const Mbsr &A, const Mbsr &B) {
     if (A.max_row_blocks > kRowsA || A.nblk == 0 || B.nblk == 0) return 0;
+    if (A.brow < kRowsMinBrow) return 0;
     if (A.avg_nnz > 6.0 || B.avg_nnz > 6.0) return 0;
     const int lanes = B.nblk <= 4 * int64_t(B.brow) ? 4 : 8;
     const double pa = double(A.nnz) / (4.0 * A.brow), pb = double(B.nnz) / (4.0 * B.brow);

@@ -135,7 +135,7 @@ def _filled_blocks_csr(nbr, nbc, counts, fill, seed, cut=0):
 
 # (A: longest block row, entries per block, entries per block of row 5; B: longest
 # block row, entries per block, blocks of row 3)
-@pytest.mark.parametrize("ca,fa,fa5,cb,fb,cb3", [
+SHORT_ROWS = [
     (8, 2, 2, 4, 1, 4),     # 4 lanes, at most 32 products
     (16, 1, 1, 4, 2, 4),    # 4 lanes, 16 A blocks, 64 products
     (16, 1, 16, 4, 2, 4),   # one row over the A values staged, C row over 64 values
@@ -147,7 +147,10 @@ def _filled_blocks_csr(nbr, nbc, counts, fill, seed, cut=0):
     (17, 1, 1, 3, 1, 3),    # 17 A blocks: the MFMA kernel
     (3, 5, 5, 3, 5, 3),     # below the line of 3-block rows
     (3, 6, 6, 3, 6, 3),     # above it
-])
+]
+
+
+@pytest.mark.parametrize("ca,fa,fa5,cb,fb,cb3", SHORT_ROWS)
 def test_spgemm_short_sparse_rows(dev, ca, fa, fa5, cb, fb, cb3):
     AI, AJ, AA = _filled_blocks_csr(67, 41, lambda i: ca if i == 5 else i % (ca + 1),
                                     lambda i: fa5 if i == 5 else fa, 21, cut=3)
@@ -155,6 +158,34 @@ def test_spgemm_short_sparse_rows(dev, ca, fa, fa5, cb, fb, cb3):
                                     lambda i: fb, 22)
     check_product(dev, 4 * 67 - 3, 4 * 41, 4 * 53, AI, AJ, AA, BI, BJ, BA,
                   f"short rows {ca}x{fa} {cb}x{fb}")
+
+
+@pytest.mark.parametrize("ca,fa,fa5,cb,fb,cb3", SHORT_ROWS)
+def test_spgemm_short_sparse_rows_many(dev, ca, fa, fa5, cb, fb, cb3):
+    """The same rows 490 times below each other: over the 32768 block rows from which the
+    row kernel runs, the last block row ragged."""
+    copies, cut = 490, 3
+    AI, AJ, AA = _filled_blocks_csr(67, 41, lambda i: ca if i == 5 else i % (ca + 1),
+                                    lambda i: fa5 if i == 5 else fa, 21)
+    BI, BJ, BA = _filled_blocks_csr(41, 53, lambda i: cb3 if i == 3 else cb - i % 2,
+                                    lambda i: fb, 22)
+    m, k, n = 4 * 67, 4 * 41, 4 * 53
+    print(f"[spgemm] {copies} x short rows {ca}x{fa} {cb}x{fb}", flush=True)
+    RI, RJ, RV = O.mbsr2csr(O.mbsr_spgemm(O.csr2mbsr(m, k, AI, AJ, AA), O.csr2mbsr(k, n, BI, BJ, BA)))
+    scale = abs_product_scale(m, k, n, AI, AJ, AA, BI, BJ, BA)
+    scale.sort_indices()
+
+    def stack(I, J, V):
+        lens = np.tile(np.diff(I), copies)[:m * copies - cut]
+        out = np.zeros(len(lens) + 1, np.int32)
+        out[1:] = np.cumsum(lens)
+        return out, np.tile(J, copies)[:out[-1]], np.tile(V, copies)[:out[-1]]
+
+    GC = make(dev, m * copies - cut, k, *stack(AI, AJ, AA)).spgemm(make(dev, k, n, BI, BJ, BA))
+    CI, CJ, CV = (t.cpu().numpy() for t in GC.to_csr())
+    EI, EJ, EV = stack(RI, RJ, RV)
+    assert np.array_equal(CI, EI) and np.array_equal(CJ, EJ)
+    assert np.all(np.abs(CV - EV) <= 1e-12 * np.tile(scale.data, copies)[:len(EV)] + 1e-300)
 
 
 def test_spgemm_stencils(dev):
