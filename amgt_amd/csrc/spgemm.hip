@@ -1449,9 +1449,10 @@ __global__ __launch_bounds__(256) void k_numeric_rows(int count, const int32_t *
         double av[kRowsAv];
         int2 rec[PR];                // B bitmap | C bitmap << 16, B value offset
         uint8_t rc[PR];              // first entry of the C block
-        int4 pad;                    // rows start four banks apart
+        int4 pad;                    // rows start 12 (PR 32) or 20 (PR 64) of the 64 banks apart
         int4 ab[kRowsA];             // bitmap | B blocks << 16, first value, first product, first B block
     };
+    static_assert(sizeof(Row) / 4 % 64 == (PR == 32 ? 12 : 20), "bank stride of the rows");
     __shared__ Row s_row[NR];
     const double *__restrict__ aval = static_cast<const double *>(g.av);
     const double *__restrict__ bval = static_cast<const double *>(g.bv);
@@ -2048,8 +2049,7 @@ int numeric_rows_lanes(const Mbsr &A, const Mbsr &B) {
 // bitmaps from the symbolic temporaries (slots, tcol, tmap) to C; the other
 // kernels read them from C.
 template <typename VT>
-int launch_numeric(const SpgemmArgs &g, const Mbsr &A, const Mbsr &B, const int32_t *boff,
-                   const Mbsr &C, int32_t brow,
+int launch_numeric(const SpgemmArgs &g, const int32_t *boff, const Mbsr &C, int32_t brow,
                    const int32_t *list, int32_t reg_rows, int32_t lds_rows, int32_t big_rows,
                    const CSlots &slots, const int32_t *tcol, const uint32_t *tmap,
                    const int32_t *big, int rows_l, double **nslab, hipStream_t s) {
@@ -2405,17 +2405,17 @@ int spgemm(const Mbsr &A, const Mbsr &B, int precision, hipStream_t s, Mbsr *Cp)
     if (!C.pattern_only && brow > 0) {
         switch (precision) {
             case AMGT_FLOAT:
-                st = launch_numeric<float>(g, A, B, boff, C, brow, list, reg_rows, lds_rows, big_rows, slots, tcol, tmap, ct.big, rows_l, &nslab, s);
+                st = launch_numeric<float>(g, boff, C, brow, list, reg_rows, lds_rows, big_rows, slots, tcol, tmap, ct.big, rows_l, &nslab, s);
                 break;
             case AMGT_HALF:
-                st = launch_numeric<__half>(g, A, B, boff, C, brow, list, reg_rows, lds_rows, big_rows, slots, tcol, tmap, ct.big, rows_l, &nslab, s);
+                st = launch_numeric<__half>(g, boff, C, brow, list, reg_rows, lds_rows, big_rows, slots, tcol, tmap, ct.big, rows_l, &nslab, s);
                 // the FP16 copies hold A and B times half_scale: undo both (powers of two, exact)
                 if (st == AMGT_OK && C.nnz > 0)
                     hipLaunchKernelGGL(k_scale_values, dim3(unsigned((C.nnz + 255) / 256)), dim3(256),
                                        0, s, C.nnz, 1.0 / (A.half_scale * B.half_scale), C.val);
                 break;
             default:
-                st = launch_numeric<double>(g, A, B, boff, C, brow, list, reg_rows, lds_rows, big_rows, slots, tcol, tmap, ct.big, rows_l, &nslab, s);
+                st = launch_numeric<double>(g, boff, C, brow, list, reg_rows, lds_rows, big_rows, slots, tcol, tmap, ct.big, rows_l, &nslab, s);
         }
         if (st != AMGT_OK) {
             cleanup();
