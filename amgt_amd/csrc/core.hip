@@ -408,7 +408,7 @@ int amgt_mbsr_get_info(amgt_mbsr_t A, amgt_mbsr_info_t *info) {
     info->max_row_blocks = m.max_row_blocks;
     info->level = m.level;
     info->precision = effective_precision(m);
-    info->spmv_lanes = m.spmv_lanes ? m.spmv_lanes : spmv_default_lanes(m);
+    info->spmv_lanes = m.spmv_lanes ? m.spmv_lanes : spmv_default_lanes(m, effective_precision(m));
     info->spmv_kernel = m.spmv_kernel;
     return AMGT_OK;
 }
@@ -473,8 +473,9 @@ static int spmv_sweep(Mbsr &m, hipStream_t s, float *t_min) {
     AMGT_HIP(hipEventCreate(&e0));
     AMGT_HIP(hipEventCreate(&e1));
     // bring the clocks up before the first measurement
-    AMGT_TRY(spmv_prepare(&m, spmv_default_lanes(m), s));
-    for (int r = 0; r < 30; ++r) AMGT_TRY(spmv(m, prec, spmv_default_lanes(m), 1.0, x, 0.0, nullptr, y, s));
+    const int lanes = spmv_default_lanes(m, prec);
+    AMGT_TRY(spmv_prepare(&m, lanes, s));
+    for (int r = 0; r < 30; ++r) AMGT_TRY(spmv(m, prec, lanes, 1.0, x, 0.0, nullptr, y, s));
     for (int sweep = 0; sweep < 2; ++sweep) {
         for (int kk = 0; kk < 4; ++kk) {
             m.spmv_kernel = kTuneKinds[kk];
@@ -504,7 +505,7 @@ static int spmv_sweep(Mbsr &m, hipStream_t s, float *t_min) {
     tmp_free(y, s);
     m.spmv_kernel = kind0;
     m.spmv_lanes = lanes0;
-    return spmv_prepare(&m, m.spmv_lanes ? m.spmv_lanes : spmv_default_lanes(m), s);
+    return spmv_prepare(&m, m.spmv_lanes ? m.spmv_lanes : spmv_default_lanes(m, prec), s);
 }
 
 int amgt_mbsr_spmv_sweep(amgt_mbsr_t A, void *stream, float *times_ms) {
@@ -526,7 +527,7 @@ int amgt_mbsr_autotune(amgt_mbsr_t A, void *stream) {
     float t[20];
     AMGT_TRY(spmv_sweep(m, s, t));
     float best = 1e30f;
-    int best_lanes = spmv_default_lanes(m), best_kind = kTuneKinds[0];
+    int best_lanes = spmv_default_lanes(m, effective_precision(m)), best_kind = kTuneKinds[0];
     for (int kk = 0; kk < 4; ++kk)
         for (int c = 0; c < 5; ++c)
             if (t[kk * 5 + c] < best) {
@@ -539,7 +540,9 @@ int amgt_mbsr_autotune(amgt_mbsr_t A, void *stream) {
     return spmv_prepare(&m, best_lanes, s);
 }
 
-static int lanes_of(const Mbsr &m) { return m.spmv_lanes ? m.spmv_lanes : spmv_default_lanes(m); }
+static int lanes_of(const Mbsr &m, int prec) {
+    return m.spmv_lanes ? m.spmv_lanes : spmv_default_lanes(m, prec);
+}
 
 static int get_transpose(Mbsr &m, hipStream_t s, Mbsr **t) {
     if (!m.trans) {
@@ -575,8 +578,8 @@ int amgt_mbsr_spmv(amgt_mbsr_t A, int trans, double alpha, const double *d_x, do
     if (trans) AMGT_TRY(get_transpose(m, s, &op));
     int prec = effective_precision(m);
     AMGT_TRY(mbsr_ensure_lowp(op, &prec, s));
-    AMGT_TRY(spmv_prepare(op, lanes_of(*op), s));
-    return spmv(*op, prec, lanes_of(*op), alpha, d_x, beta, d_b, d_y, s);
+    AMGT_TRY(spmv_prepare(op, lanes_of(*op, prec), s));
+    return spmv(*op, prec, lanes_of(*op, prec), alpha, d_x, beta, d_b, d_y, s);
 }
 
 int amgt_mbsr_spmm(amgt_mbsr_t A, int trans, int k, double alpha, const double *d_x, int64_t ldx,
@@ -596,8 +599,8 @@ int amgt_mbsr_spmm(amgt_mbsr_t A, int trans, int k, double alpha, const double *
     if (trans) AMGT_TRY(get_transpose(m, s, &op));
     int prec = effective_precision(m);
     AMGT_TRY(mbsr_ensure_lowp(op, &prec, s));
-    AMGT_TRY(spmv_prepare(op, lanes_of(*op), s));  // k == 1 runs the SpMV kernels
-    return spmm(*op, prec, lanes_of(*op), k, alpha, d_x, ldx, beta, d_b, ldb, d_y, ldy, s);
+    AMGT_TRY(spmv_prepare(op, lanes_of(*op, prec), s));  // k == 1 runs the SpMV kernels
+    return spmm(*op, prec, lanes_of(*op, prec), k, alpha, d_x, ldx, beta, d_b, ldb, d_y, ldy, s);
 }
 
 int amgt_mbsr_spmm_interleaved(amgt_mbsr_t A, int trans, int k, double alpha, const double *d_x,
@@ -660,8 +663,8 @@ int amgt_mbsr_relax_jacobi(amgt_mbsr_t A, double omega, const double *d_dinv, co
     hipStream_t s = as_stream(stream);
     int prec = effective_precision(m);
     AMGT_TRY(mbsr_ensure_lowp(&m, &prec, s));
-    AMGT_TRY(spmv_prepare(&m, lanes_of(m), s));
-    return relax_jacobi(m, prec, lanes_of(m), omega, d_dinv, d_f, d_u, d_u_new, s);
+    AMGT_TRY(spmv_prepare(&m, lanes_of(m, prec), s));
+    return relax_jacobi(m, prec, lanes_of(m, prec), omega, d_dinv, d_f, d_u, d_u_new, s);
 }
 
 int amgt_mbsr_spgemm(amgt_mbsr_t A, amgt_mbsr_t B, void *stream, amgt_mbsr_t *C) {

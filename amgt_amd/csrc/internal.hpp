@@ -192,7 +192,7 @@ int spmv_balanced_ws(const Mbsr &A, int lanes, double alpha, const double *x, do
 int spmm(const Mbsr &A, int precision, int lanes, int k, double alpha, const double *x,
          int64_t ldx, double beta, const double *b, int64_t ldb, double *y, int64_t ldy,
          hipStream_t s);
-int spmv_default_lanes(const Mbsr &A);
+int spmv_default_lanes(const Mbsr &A, int precision);
 // k right-hand sides interleaved (entry (row i, vector v) at x[i * k + v])
 int spmm_interleaved(const Mbsr &A, int precision, int k, double alpha, const double *x,
                      double beta, const double *b, double *y, hipStream_t s);

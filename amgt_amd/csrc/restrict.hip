@@ -77,7 +77,7 @@ static void plan_release(RestrictPlan *p, hipStream_t s) {
 }
 
 static int plan_build(const Mbsr &A, const Mbsr &R, hipStream_t s, RestrictPlan *p) {
-    const int lanes = A.spmv_lanes ? A.spmv_lanes : spmv_default_lanes(A);
+    const int lanes = A.spmv_lanes ? A.spmv_lanes : spmv_default_lanes(A, AMGT_DOUBLE);
     p->nfine = A.nrows;
     p->nc = R.nrows;
     p->rpb = blk_tile_rows(lanes);

@@ -411,6 +411,30 @@ def test_default_kernel_from_statistics(dev):
         assert M.info()["spmv_kernel"] == want
 
 
+@pytest.mark.parametrize("blocks,fill,lanes", [(14, 9, (32, 32, 32)), (14, 11, (64, 64, 16)),
+                                               (11, 12, (32, 32, 32)), (17, 11, (64, 64, 64))])
+def test_block_tile_by_precision(dev, blocks, fill, lanes):
+    """Tiles whose 16 rows pass the value capacity: eight rows, 16 for a slight excess, 32 in
+    FP16 where their blocks fit; products in all three precisions."""
+    print(f"[block tile] {blocks} blocks of {fill}", flush=True)
+    rng = np.random.default_rng(fill)
+    brow = 170000 // blocks
+    br = np.repeat(np.arange(brow), blocks)
+    bc = (br + 3 * np.tile(np.arange(blocks), brow)) % brow
+    e = np.argsort(rng.random((len(br), 16)), 1)[:, :fill]
+    S = sp.csr_matrix((rng.standard_normal(e.size), ((4 * br[:, None] + e // 4).ravel(),
+                                                     (4 * bc[:, None] + e % 4).ravel())),
+                      shape=(4 * brow, 4 * brow))
+    n, (I, J, A) = 4 * brow, (S.indptr.astype(np.int32), S.indices.astype(np.int32), S.data)
+    M = make(dev, n, n, I, J, A)
+    x = rng.standard_normal(n)
+    for prec, tol, want in zip((L.AMGT_DOUBLE, L.AMGT_FLOAT, L.AMGT_HALF), (1e-12, 2e-6, 2e-3), lanes):
+        M.set_precision(prec)
+        assert M.info()["spmv_kernel"] == L.AMGT_SPMV_BLOCK and M.info()["spmv_lanes"] == want
+        y = M.spmv(T(x, dev)).cpu().numpy()
+        assert np.all(np.abs(y - S @ x) <= tol * row_scale(n, n, I, J, A, x, 0.0, np.zeros(n)))
+
+
 # block rows of 1 to 130 blocks (edges of the 16-block steps and the 64-block
 # loads), rows of more values than eight of a tile hold, ragged columns
 @pytest.mark.parametrize("prec,tol", [(L.AMGT_DOUBLE, 1e-12), (L.AMGT_FLOAT, 2e-6),
