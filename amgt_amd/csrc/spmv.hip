@@ -102,6 +102,14 @@ struct EpResidRestrict {
     __device__ __forceinline__ double operator()(int row, double ax) const { return f[row] - ax; }
 };
 
+// epilogues with work per tile: for the kernels that call tile_post only
+template <typename EP>
+struct HasTilePost : std::false_type {};
+template <>
+struct HasTilePost<EpResidRestrict> : std::true_type {};
+template <typename EP>
+struct HasTilePost<EpScaled<EP>> : HasTilePost<EP> {};
+
 // Work of a whole tile after its rows are stored (every thread of the
 // workgroup calls it): nothing for the plain epilogues.
 template <typename EP>
@@ -1662,6 +1670,9 @@ bool spmv_long_rows(const Mbsr &A, int lanes) {
 template <typename VT, typename AT, typename EP>
 int launch_spmv_t(const Mbsr &A, const VT *val, int lanes, const double *x, EP ep, double *y,
                   hipStream_t s) {
+    // (the direct, balanced and long-row kernels have no tiles to finish; the fused
+    // restriction launches the block kernel itself, also for long rows)
+    static_assert(!HasTilePost<EP>::value, "launch_spmv_t: epilogue with work per tile");
     if (lanes != 4 && lanes != 8 && lanes != 16 && lanes != 32 && lanes != 64) {
         set_error("lanes per block row must be 4, 8, 16, 32 or 64");
         return AMGT_ERR_ARG;
