@@ -30,9 +30,12 @@ namespace amgt {
 namespace {
 
 constexpr int kThreads = 256;
-// extended+i rows of 65 to 512 entries take the wave kernels on levels of at
-// most kWaveMaxRows rows (16 to 70 KB of LDS per wave: worth it only when the
-// thread kernel would leave the chip idle behind a few long serial rows)
+// extended+i rows of 257 to 512 entries take the wave kernel on levels of at most
+// kWaveMaxRows rows: at 74 KB of LDS two waves fit a CU, worth it only when the
+// thread kernel would leave the chip idle behind a few long serial rows (300000
+// rows of 400: 639 ms against 420 by threads).  Shorter ones take it on any level
+// (thread / wave kernel, ms: 300000 rows of 80 23.0 / 11.2, of 120 47 / 18, of 200 119 /
+// 89; 2.2 M of 70 111 / 68).
 constexpr int kWaveMaxRows = 1 << 18;
 
 inline unsigned grid_of(int64_t n) { return unsigned((n + kThreads - 1) / kThreads); }
@@ -604,8 +607,7 @@ __global__ __launch_bounds__(kThreads) void k_extpi_row(
 // capacities: WA entries of row i (A and S), WT distinct P columns kept in
 // LDS, WH table slots: at most WT + 64 candidate columns (the insertions stop
 // once WT is passed) plus WA strong F neighbours ever enter the table, which
-// stays at most about half full.  Two sets: rows of up to 64 entries (about
-// 15 KB of LDS, many rows per CU) and of up to 256.
+// stays at most about half full (8.5 to 74 KB of LDS, below).
 template <int WA, int WT, int WH>
 struct WaveRow {
     static_assert(2 * (WT + 64 + WA) <= WH + 128 && (WH & (WH - 1)) == 0, "table size");
@@ -941,8 +943,8 @@ __global__ __launch_bounds__(64) void k_extpi_wave(
 
 // ---- extended+i, G lanes per row (G = 8, 16, 32: rows of up to G entries in A and S) ----
 // The same results as k_extpi_row.  64 / G rows share a wave, a row's state is
-// 4 G columns and a table of 8 G slots in LDS (0.9 KB for G = 8, 29 KB per
-// workgroup whatever G), a lane holds one entry of A and one of S.  The
+// 4 G columns and a table of 8 G slots in LDS (152 G bytes: 1.2 KB for G = 8, 39 KB
+// per workgroup whatever G, four workgroups per CU), a lane holds one entry of A and one of S.  The
 // thread kernel is bound by its per-row tables in global memory (scattered
 // probes, a few lanes of a cache line used); here only the neighbours' rows
 // are read from memory, all of a row's neighbours at once, and every probe
@@ -971,6 +973,7 @@ struct GroupRow {
     uint64_t tp[G];            // positions of the terms, 16 bits each (0xffff: none)
     int32_t pcol[4 * G];
 };
+static_assert(sizeof(GroupRow<8>) == 152 * 8 && sizeof(GroupRow<32>) == 152 * 32, "LDS per row");
 
 template <int WH>
 __device__ __forceinline__ int kv_find(const int2 *kv, int k) {
@@ -1358,7 +1361,7 @@ constexpr int kListed = 8, kCodes = 11;
 __global__ __launch_bounds__(kThreads) void k_extpi_class(
     int32_t n, const int32_t *__restrict__ I, const int32_t *__restrict__ J,
     const double *__restrict__ A, const int32_t *__restrict__ SI, const int32_t *__restrict__ cf,
-    int allow_big, int32_t *__restrict__ flag, int32_t *__restrict__ use,
+    int longest, int32_t *__restrict__ flag, int32_t *__restrict__ use,
     int8_t *__restrict__ dneg, RowSlots out) {
     const int i = blockIdx.x * kThreads + threadIdx.x;
     if (i >= n) return;
@@ -1375,7 +1378,7 @@ __global__ __launch_bounds__(kThreads) void k_extpi_class(
     } else {
         u = len <= 8 ? kGroup8 : (len <= 16 ? kGroup16 : (len <= 32 ? kGroup32 : kThreadRow));
         if (len > 32 && len <= 64) u = kTier64;
-        if (allow_big && len > 64 && len <= 512)
+        if (len > 64 && len <= longest)  // of the wave kernels
             u = len <= 128 ? kTier128 : (len <= 256 ? kTier256 : kTier512);
     }
     flag[i] = f >= 0 ? 1 : 0;
@@ -1727,7 +1730,7 @@ int amgt_amg_extpi_interp(int32_t n, const int32_t *A_i, const int32_t *A_j,
     };
     if (n > 0) {
         hipLaunchKernelGGL(k_extpi_class, g, b, 0, s, n, A_i, A_j, A_data, S_i, cf_marker,
-                           n <= kWaveMaxRows ? 1 : 0, flag, use, dneg, slots);
+                           n <= kWaveMaxRows ? 512 : 256, flag, use, dneg, slots);
         AMGT_TRY(count_codes());
     }
     AMGT_TRY(exclusive_scan_i32(flag, f2c, n, s));
@@ -1791,13 +1794,13 @@ int amgt_amg_extpi_interp(int32_t n, const int32_t *A_i, const int32_t *A_j,
                        rows, A_i, A_j, A_data, S_i, S_j, cf_marker, dneg, wo, wcol, max_elmts, \
                        slots, use, NEXT_, ovf)
             switch (code) {
-                case kTier64: AMGT_EXTPI_WAVE(64, 128, 512, kTier64Big); break;      // ~8.4 KB
-                case kTier64Big: AMGT_EXTPI_WAVE(64, 384, 1024, kThreadRow); break;  // ~15.6 KB
-                case kTier128: AMGT_EXTPI_WAVE(128, 256, 1024, kTier128Big); break;  // ~16 KB
-                case kTier256: AMGT_EXTPI_WAVE(256, 768, 2048, kTier256Big); break;  // ~35 KB
+                case kTier64: AMGT_EXTPI_WAVE(64, 128, 512, kTier64Big); break;      // 8.5 KB
+                case kTier64Big: AMGT_EXTPI_WAVE(64, 384, 1024, kThreadRow); break;  // 15.5 KB
+                case kTier128: AMGT_EXTPI_WAVE(128, 256, 1024, kTier128Big); break;  // 17 KB
+                case kTier256: AMGT_EXTPI_WAVE(256, 768, 2048, kTier256Big); break;  // 37 KB
                 case kTier128Big: AMGT_EXTPI_WAVE(256, 768, 2048, kThreadRow); break;
-                case kTier256Big: AMGT_EXTPI_WAVE(256, 1536, 4096, kThreadRow); break;  // ~60 KB
-                case kTier512: AMGT_EXTPI_WAVE(512, 1536, 4096, kThreadRow); break;  // ~70 KB
+                case kTier256Big: AMGT_EXTPI_WAVE(256, 1536, 4096, kThreadRow); break;  // 62 KB
+                case kTier512: AMGT_EXTPI_WAVE(512, 1536, 4096, kThreadRow); break;  // 74 KB
                 default:
                     hipLaunchKernelGGL(k_extpi_row, dim3(grid_of(cw)), b, 0, s, cw, rows, A_i, A_j,
                                        A_data, S_i, S_j, cf_marker, max_elmts, wo, wcol, wval,

@@ -225,6 +225,36 @@ def test_extpi_group_edges_match_oracle(dev, per_row, mixed):
         assert np.array_equal(PA.cpu().numpy(), rPA), pmx
 
 
+def test_extpi_long_rows_of_large_level(dev):
+    """A level over 2^18 rows: rows of 65, 128, 129, 256 (wave kernels), 257, 300 and 512
+    entries (thread kernel) among tridiagonal ones; P unlimited and truncated equals the
+    oracle's exactly."""
+    n = (1 << 18) + 77
+    print(f"[extpi large level] n={n}", flush=True)
+    rng = np.random.default_rng(4)
+    rows, cols = [np.repeat(np.arange(n), 3)], [(np.repeat(np.arange(n), 3) + np.tile([-1, 0, 1], n)) % n]
+    for q, k in enumerate([65, 128, 129, 256, 257, 300, 512] * 30):
+        r = 1000 * q + 13
+        rows.append(np.full(k - 3, r))
+        cols.append((r + 2 + rng.permutation(4 * k)[:k - 3]) % n)
+    r, c = np.concatenate(rows), np.concatenate(cols)
+    M = sp.csr_matrix((-rng.uniform(0.5, 1.0, len(r)), (r, c)), shape=(n, n))
+    M.setdiag(np.asarray(abs(M).sum(1)).ravel())
+    M.sort_indices()
+    assert sorted(set(np.diff(M.indptr))) == [3, 65, 128, 129, 256, 257, 300, 512]
+    I, J, A = M.indptr.astype(np.int32), M.indices.astype(np.int32), M.data.copy()
+    dI, dJ, dA = T(I, dev), T(J, dev), T(A, dev)
+    SI, SJ = C.strength(n, dI, dJ, dA, 0.25, 1.0)
+    cf, _ = C.pmis(n, SI, SJ, 0)
+    rSI, rSJ, rcf = SI.cpu().numpy(), SJ.cpu().numpy(), cf.cpu().numpy()
+    for pmx in (0, 4):
+        PI, PJ, PA, _ = C.extpi_interp(n, dI, dJ, dA, SI, SJ, cf, pmx)
+        rPI, rPJ, rPA, _ = O.amg_extpi(n, I, J, A, rSI, rSJ, rcf, pmx)
+        assert np.array_equal(PI.cpu().numpy(), rPI), pmx
+        assert np.array_equal(PJ.cpu().numpy(), rPJ), pmx
+        assert np.array_equal(PA.cpu().numpy(), rPA), pmx
+
+
 @pytest.mark.parametrize("n", [3001, 40003, 270001])
 @pytest.mark.parametrize("diagonal", ["ascending", "first", "none"])
 def test_strength_parts(dev, n, diagonal):
