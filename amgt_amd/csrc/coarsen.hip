@@ -457,20 +457,21 @@ struct RowSlots {
 };
 
 // One thread per listed row: the row's columns (fine indices) and weights in
-// the host's discovery order into work arrays at woff[t], truncated there, then
-// copied to the row's slot.
+// the host's discovery order into work arrays at woff[t] (the weights at woff[t] -
+// wfirst: only this kernel's rows have them), truncated there, then copied to the
+// row's slot.
 __global__ __launch_bounds__(kThreads) void k_extpi_row(
     int32_t count, const int32_t *__restrict__ rows, const int32_t *__restrict__ I,
     const int32_t *__restrict__ J, const double *__restrict__ A, const int32_t *__restrict__ SI,
     const int32_t *__restrict__ SJ, const int32_t *__restrict__ cf, int max_elmts,
-    const int64_t *__restrict__ woff, int32_t *__restrict__ wcol, double *__restrict__ wval,
-    const int64_t *__restrict__ hoff, int2 *__restrict__ hkv, RowSlots out,
+    const int64_t *__restrict__ woff, int64_t wfirst, int32_t *__restrict__ wcol,
+    double *__restrict__ wval, const int64_t *__restrict__ hoff, int2 *__restrict__ hkv, RowSlots out,
     int32_t *__restrict__ use) {
     const int t = blockIdx.x * kThreads + threadIdx.x;
     if (t >= count) return;
     const int i = rows[t];
     int32_t *cols = wcol + woff[t];
-    double *w = wval + woff[t];
+    double *w = wval + (woff[t] - wfirst);
     int2 *kv = hkv + hoff[t];
     const uint32_t mask = uint32_t(hoff[t + 1] - hoff[t]) - 1u;
     // structure (:1501-1560)
@@ -1768,14 +1769,15 @@ int amgt_amg_extpi_interp(int32_t n, const int32_t *A_i, const int32_t *A_j,
                            S_j, cf_marker, ub, hs);
         AMGT_HIP(hipGetLastError());
         AMGT_TRY(exclusive_scan_i64(ub, woff, np, s));
-        int64_t total_w = 0, total_h = 0;
-        if (nthread > 0) {
+        int64_t total_w = 0, total_h = 0, wfirst = 0;
+        if (nthread > 0) {  // (the thread kernel's rows are the last ones)
             AMGT_TRY(tmp.get(&hoff, size_t(np) + 1));
             AMGT_TRY(exclusive_scan_i64(hs, hoff, np, s));
-            const Readback rb[2] = {{&total_w, woff + np, sizeof(int64_t)},
-                                    {&total_h, hoff + np, sizeof(int64_t)}};
-            AMGT_TRY(readback(rb, 2, s));
-            AMGT_TRY(tmp.get(&wval, size_t(total_w)));
+            const Readback rb[3] = {{&total_w, woff + np, sizeof(int64_t)},
+                                    {&total_h, hoff + np, sizeof(int64_t)},
+                                    {&wfirst, woff + (np - nthread), sizeof(int64_t)}};
+            AMGT_TRY(readback(rb, 3, s));
+            AMGT_TRY(tmp.get(&wval, size_t(total_w - wfirst)));
             AMGT_TRY(tmp.get(&hkv, size_t(total_h)));
             AMGT_HIP(hipMemsetAsync(hkv, 0xff, sizeof(int2) * size_t(total_h), s));
         } else {
@@ -1803,7 +1805,7 @@ int amgt_amg_extpi_interp(int32_t n, const int32_t *A_i, const int32_t *A_j,
                 case kTier512: AMGT_EXTPI_WAVE(512, 1536, 4096, kThreadRow); break;  // 74 KB
                 default:
                     hipLaunchKernelGGL(k_extpi_row, dim3(grid_of(cw)), b, 0, s, cw, rows, A_i, A_j,
-                                       A_data, S_i, S_j, cf_marker, max_elmts, wo, wcol, wval,
+                                       A_data, S_i, S_j, cf_marker, max_elmts, wo, wfirst, wcol, wval,
                                        hoff + t0, hkv, slots, use);
             }
 #undef AMGT_EXTPI_WAVE

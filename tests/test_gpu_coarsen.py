@@ -225,6 +225,29 @@ def test_extpi_group_edges_match_oracle(dev, per_row, mixed):
         assert np.array_equal(PA.cpu().numpy(), rPA), pmx
 
 
+@pytest.mark.parametrize("n,per_row", [(1501, 7), (1501, 14), (1501, 30), (3000, 45), (2000, 100)])
+@pytest.mark.parametrize("equal", [False, True])
+def test_extpi_limits_match_oracle(dev, n, per_row, equal):
+    """Limits with padded slots (3, 5), the largest slot (16), truncation into rows sized by
+    their bounds (17) and above the wave kernels' 64 entries (100), by the kernels of 8, 16
+    and 32 lanes and by the wave kernels; equal weights tie, so that the quicksort orders
+    them.  P equals the oracle's exactly."""
+    print(f"[extpi limits] n={n} per_row={per_row} equal={equal}", flush=True)
+    I, J, A = _rand_long(n, per_row, per_row)
+    if equal:
+        A = np.where(A < 0, -1.0, A)
+    dI, dJ, dA = T(I, dev), T(J, dev), T(A, dev)
+    SI, SJ = C.strength(n, dI, dJ, dA, 0.25, 0.9)
+    cf, _ = C.pmis(n, SI, SJ, 0)
+    rSI, rSJ, rcf = SI.cpu().numpy(), SJ.cpu().numpy(), cf.cpu().numpy()
+    for pmx in (1, 3, 5, 16, 17, 100):
+        PI, PJ, PA, _ = C.extpi_interp(n, dI, dJ, dA, SI, SJ, cf, pmx)
+        rPI, rPJ, rPA, _ = O.amg_extpi(n, I, J, A, rSI, rSJ, rcf, pmx)
+        assert np.array_equal(PI.cpu().numpy(), rPI), pmx
+        assert np.array_equal(PJ.cpu().numpy(), rPJ), pmx
+        assert np.array_equal(PA.cpu().numpy(), rPA), pmx
+
+
 def test_extpi_long_rows_of_large_level(dev):
     """A level over 2^18 rows: rows of 65, 128, 129, 256 (wave kernels), 257, 300 and 512
     entries (thread kernel) among tridiagonal ones; P unlimited and truncated equals the
