@@ -1421,9 +1421,9 @@ __global__ __launch_bounds__(256) void k_numeric_outer(int count, const int32_t 
 // The MFMA form (k_numeric_outer) multiplies whole 4x4 blocks: at the fill of
 // stencil and interpolation operators (1/4 and less) 1 of 16 to 1 of 64 of its
 // products exist, and it is bound by the VALU work of gathering padded operands
-// (550 instructions per row of A P on 7-pt 128^3, one row per wave).  Here only
-// existing products are formed and 2 or 4 rows share a wave (235 instructions
-// per row); it waits on the chain row pointers -> A blocks -> B rows -> B blocks
+// (549 vector instructions per row of A P on 7-pt 128^3, one row per wave).  Here only
+// existing products are formed and 2 or 4 rows share a wave (289 per
+// row); it waits on the chain row pointers -> A blocks -> B rows -> B blocks
 // -> values, so LDS per row (waves per CU) and loads in flight count: 566 us
 // (MFMA) -> 544 with one value load at a time, 500 with four A blocks' loads
 // together, 385 with packed C blocks and 12-byte records.
