@@ -135,6 +135,7 @@ def _filled_blocks_csr(nbr, nbc, counts, fill, seed, cut=0):
 
 # (A: longest block row, entries per block, entries per block of row 5; B: longest
 # block row, entries per block, blocks of row 3)
+# (the kernels named run from 32768 block rows on; single copies take the matrix-core one)
 SHORT_ROWS = [
     (8, 2, 2, 4, 1, 4),     # 4 lanes, at most 32 products
     (16, 1, 1, 4, 2, 4),    # 4 lanes, 16 A blocks, 64 products
